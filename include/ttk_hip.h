@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define TTK_ABI_VERSION 9
+#define TTK_ABI_VERSION 10
 
 /* Bytes of the arrival-counter block that leads every attention workspace
  * (and the library's static scratch): the same for every launch shape. */
@@ -233,6 +233,50 @@ ttk_status ttk_gelu_fwd(const void* x, void* y, int dtype, int64_t n, void* stre
 ttk_status ttk_linear_fwd(const void* x, const void* w, const void* bias, void* y, int dtype,
                           int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                           int64_t ldy, int activation, void* stream);
+
+/*
+ * Bytes of the buffer ttk_linear_f32_split_weight fills for W [N, K]:
+ * ceil(N / 32) * 32 * K * 6 (0 for N <= 0 or K <= 0).
+ */
+int64_t ttk_linear_f32_split_bytes(int64_t N, int64_t K);
+
+/*
+ * fp32 W [N, K] (row stride ldw elements) as three bf16 terms whose sum is W
+ * exactly (values below 2^-110 in magnitude may lose their last bits), in the
+ * MFMA fragment order ttk_linear_f32_fwd reads: 16-byte chunk
+ * ((fb * K/16 + q) * 3 + t) * 64 + l holds term t of
+ * W[32 fb + l % 32][16 q + 8 (l / 32) .. + 7], rows past N zero.
+ * Requirements (TTK_EUNSUPPORTED otherwise): K a multiple of 32 below 2^22, w
+ * and w_split 16-byte aligned, ldw a multiple of 4 and >= K; w_split must not
+ * overlap w (TTK_EINVAL).  A weight that does not change is split once.
+ */
+ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, int64_t K, int64_t ldw,
+                                       void* stream);
+
+/*
+ * fp32 linear layer with an optional exact (erf) GELU:
+ *
+ *   Y = act( X W^T + bias )
+ *
+ * X [M, K] (row stride ldx elements), W [N, K] (row stride ldw) and the same
+ * W as split by ttk_linear_f32_split_weight, bias [N] or NULL, Y [M, N] (row
+ * stride ldy), all fp32.  Each operand enters as its three bf16 terms and the
+ * six products of terms above 2^-22 are accumulated in fp32, the leading ones
+ * apart from the rest: the error is below that of an fp32 fma chain over K.
+ * A result that is not finite is recomputed from the fp32 operands.
+ *
+ * Requirements (TTK_EUNSUPPORTED otherwise): K a multiple of 32 below 2^22, N
+ * a multiple of 4; x, w, w_split, bias and y 16-byte aligned; ldx, ldw and
+ * ldy multiples of 4 with ldx, ldw >= K and ldy >= N, ldx and ldy below 2^22;
+ * M and N below 2^31.  y must not overlap an input (TTK_EINVAL).  M == 0 is a
+ * no-op.
+ *
+ * Replaces the fp32 library GEMMs of the encoder's projections and the GELU
+ * pass after the FFN input (reference transformer_opt/submission.py:484-508).
+ */
+ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split, const void* bias, void* y,
+                              int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy,
+                              int activation, void* stream);
 
 /* Bytes of the counter block that leads every ttk_linear_residual_ln_fwd
  * workspace: the same for every M (one counter per 64 rows of the largest M

@@ -1,0 +1,124 @@
+"""The fp32 linear kernels (three-term bf16 splits on the bf16 matrix cores)
+against float64, at the edges of each form's tiles, and the non-finite results
+they recompute from the fp32 operands."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    # 32 x 32 tiles, K split over four wavefronts (some without a k-step).
+    (1, 4, 32), (31, 36, 64), (33, 32, 96), (129, 132, 224),
+    # 64 x 64 tiles, ragged both ways.
+    (2047, 516, 544), (2049, 1540, 512),
+    # 128 x 128 tiles: whole, ragged, several tiles per workgroup, one stage.
+    (4096, 1024, 1024), (3999, 1000, 1024), (16385, 1160, 96), (32768, 1024, 32),
+]
+
+
+def _inputs(rows, out_features, in_features, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(rows, in_features, device="cuda", generator=g)
+    w = torch.randn(out_features, in_features, device="cuda", generator=g) * in_features ** -0.5
+    b = torch.randn(out_features, device="cuda", generator=g)
+    return x, w, b
+
+
+@pytest.mark.parametrize("rows,out_features,in_features", SHAPES)
+@pytest.mark.parametrize("bias", [True, False], ids=["bias", "nobias"])
+def test_linear_f32_against_float64(gpu_ready, rows, out_features, in_features, bias):
+    from transformer_opt.kernels import gelu
+    from transformer_opt.kernels.linear_f32 import linear_f32, split_weight
+
+    x, w, b = _inputs(rows, out_features, in_features, rows + in_features)
+    b = b if bias else None
+    with torch.inference_mode():
+        split = split_weight(w)
+        y = linear_f32(x, w, split, b)
+        exact = torch.matmul(x.double(), w.double().t().contiguous())
+        scale = torch.matmul(x.double().abs(), w.double().abs().t().contiguous())
+        if bias:
+            exact, scale = exact + b.double(), scale + b.double().abs()
+        err = (y.double() - exact).abs()
+        # Products left out: 3 * 2^-22 of |x||w|; two roundings per 16 values
+        # of K and sum, and a few at the end.
+        assert bool((err <= (2.0 * in_features / 16 + 24) * 2.0 ** -24 * scale).all())
+        # No less accurate than the library's fp32 GEMM (2-norm).
+        library = F.linear(x, w, b).double() - exact
+        assert (y.double() - exact).norm() <= max(library.norm(), 1e-7 * exact.norm())
+        z = linear_f32(x, w, split, b, gelu=True)
+        torch.testing.assert_close(z, gelu(y), rtol=1e-6, atol=1e-7)
+        # The same call gives the same bits.
+        assert torch.equal(linear_f32(x, w, split, b), y)
+
+
+@pytest.mark.parametrize("rows,out_features,in_features", [(40, 64, 64), (2048, 512, 512), (4096, 1024, 1024)])
+def test_non_finite_results_are_those_of_the_fp32_operands(gpu_ready, rows, out_features, in_features):
+    from transformer_opt.kernels.linear_f32 import linear_f32, split_weight
+
+    x, w, b = _inputs(rows, out_features, in_features, 3)
+    inf = float("inf")
+    x[3, 5], x[7, 1], x[9, 0], x[11, 2] = inf, float("nan"), 3.4e38, -inf
+    w[4] = 1.0        # +inf, NaN, an overflow past bf16 and -inf meet a plain row
+    w[6, 5] = 0.0     # 0 * inf
+    w[8, 3] = inf
+    x[:, 3] = x[:, 3].abs() + 1.0
+    x[9, 1:] = 0.0
+    with torch.inference_mode():
+        y = linear_f32(x, w, split_weight(w), b)
+        exact = torch.addmm(b.double(), x.double(), w.double().t().contiguous()).float()
+    assert torch.equal(torch.isnan(y), torch.isnan(exact))
+    at_inf = torch.isinf(exact)
+    assert bool(at_inf.any()) and torch.equal(y[at_inf], exact[at_inf])
+    fine = torch.isfinite(exact)
+    torch.testing.assert_close(y[fine], exact[fine], rtol=1e-5, atol=1e-4)
+
+
+def test_split_weight_declines_what_the_kernel_cannot_take(gpu_ready):
+    from transformer_opt.kernels.linear_f32 import linear_f32_supported, split_weight
+
+    ok = torch.zeros(64, 64, device="cuda")
+    assert split_weight(ok).numel() == 64 * 64 * 6
+    for bad in (ok.cpu(), ok.bfloat16(), ok.t()[:, :33], ok[:, :48], ok[:62], ok.view(-1)):
+        assert split_weight(bad) is None
+    x = torch.zeros(5, 64, device="cuda")
+    assert linear_f32_supported(x, ok, None)
+    assert not linear_f32_supported(x[:, :32], ok, None)
+    assert not linear_f32_supported(x.double(), ok, None)
+    with torch.enable_grad():
+        assert not linear_f32_supported(x.clone().requires_grad_(), ok, None)
+        assert not linear_f32_supported(x, ok.clone().requires_grad_(), None)
+    with torch.autocast("cuda"):
+        assert not linear_f32_supported(x, ok, None)
+
+
+def test_split_terms_follow_the_weights_across_streams(gpu_ready):
+    # A weight edited in place is split again, and an eager call on another
+    # stream is ordered after the split.
+    from transformer_opt.submission import TransformerConfig, UserOptimizedTransformer
+
+    torch.manual_seed(5)
+    model = UserOptimizedTransformer(TransformerConfig(2, 96, 128, 4, 256, 2, True), execution_mode="eager")
+    model = model.cuda().eval()
+    x = torch.randn(2, 96, 128, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.inference_mode():
+        first = model(x).clone()
+    with torch.no_grad():
+        model.layers[0].ffn_out.weight.mul_(-1.0)
+        model.layers[1].attention.k_proj.weight.mul_(0.5)
+    fresh = UserOptimizedTransformer(model.config, execution_mode="eager").cuda().eval()
+    fresh.load_state_dict(model.state_dict())
+    with torch.inference_mode():
+        expected = fresh(x)
+        edited = model(x).clone()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            again = model(x)
+        torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(edited, expected) and torch.equal(again, expected)
+    assert not torch.allclose(first, expected)

@@ -1,0 +1,62 @@
+"""The fp32 linear entry points on the CPU: rejected arguments, and the M0
+invariant of their inline LDS-DMA copies in the compiled kernels."""
+
+from __future__ import annotations
+
+import pytest
+
+from test_isa_invariants import CSRC, _assembly
+from transformer_opt import _native
+
+
+def _linear(lib, **over):
+    args = dict(x=1 << 20, w=2 << 20, wp=3 << 20, b=None, y=4 << 20, M=64, N=64, K=64, ldx=64, ldw=64, ldy=64,
+                act=_native.TTK_ACT_NONE, stream=None)
+    args.update(over)
+    return lib.ttk_linear_f32_fwd(args["x"], args["w"], args["wp"], args["b"], args["y"], args["M"], args["N"],
+                                  args["K"], args["ldx"], args["ldw"], args["ldy"], args["act"], args["stream"])
+
+
+@pytest.mark.parametrize("over,status,message", [
+    (dict(act=7), _native.TTK_EINVAL, "activation"),
+    (dict(M=-1), _native.TTK_EINVAL, "M must be"),
+    (dict(N=0), _native.TTK_EINVAL, "positive"),
+    (dict(x=None), _native.TTK_EINVAL, "NULL"),
+    (dict(wp=None), _native.TTK_EINVAL, "NULL"),
+    (dict(K=48, ldx=48, ldw=48), _native.TTK_EUNSUPPORTED, "multiple of 32"),
+    (dict(N=62), _native.TTK_EUNSUPPORTED, "multiple of 4"),
+    (dict(x=(1 << 20) + 4), _native.TTK_EUNSUPPORTED, "16-byte aligned"),
+    (dict(b=(5 << 20) + 8), _native.TTK_EUNSUPPORTED, "16-byte aligned"),
+    (dict(ldx=62), _native.TTK_EUNSUPPORTED, "multiples of 4"),
+    (dict(ldw=60), _native.TTK_EUNSUPPORTED, "ldw"),
+    (dict(ldy=1 << 22), _native.TTK_EUNSUPPORTED, "below 2^22"),
+    (dict(y=(3 << 20) + 64 * 64 * 6 - 16), _native.TTK_EINVAL, "overlaps"),
+    (dict(y=1 << 20), _native.TTK_EINVAL, "overlaps"),
+    (dict(M=0), _native.TTK_OK, ""),
+])
+def test_fp32_linear_argument_errors_are_reported_without_launching(over, status, message):
+    lib = _native.load()
+    assert _linear(lib, **over) == status
+    assert message in _native.last_error()
+
+
+def test_split_weight_arguments_and_sizes():
+    lib = _native.load()
+    size, split = lib.ttk_linear_f32_split_bytes, lib.ttk_linear_f32_split_weight
+    assert size(64, 64) == 64 * 64 * 6 and size(33, 32) == 64 * 32 * 6
+    assert size(0, 64) == size(64, 0) == size(-1, 64) == size(64, 1 << 22) == 0
+    assert split(None, 1 << 20, 64, 64, 64, None) == _native.TTK_EINVAL
+    assert split(1 << 20, 2 << 20, 64, 40, 40, None) == _native.TTK_EUNSUPPORTED
+    assert split(1 << 20, (1 << 20) + 16, 64, 64, 64, None) == _native.TTK_EINVAL
+    assert split(1 << 20, 2 << 20, 64, 64, 32, None) == _native.TTK_EUNSUPPORTED
+
+
+def test_m0_is_only_written_by_the_inline_copies(tmp_path):
+    in_asm, inside, outside = False, 0, 0
+    for line in _assembly(CSRC / "linear_f32_fwd.hip", tmp_path).splitlines():
+        text = line.strip()
+        if text.startswith(";;#ASM"):
+            in_asm = text.startswith(";;#ASMSTART")
+        elif not text.startswith(";") and "m0" in text.replace(",", " ").split():
+            inside, outside = inside + in_asm, outside + (not in_asm)
+    assert inside > 0 and outside == 0

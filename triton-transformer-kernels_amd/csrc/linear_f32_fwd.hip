@@ -1,0 +1,620 @@
+// fp32 Linear (+ exact GELU) forward for gfx950 (MI355X):
+//
+//   Y[m, n] = act( sum_k X[m, k] * W[n, k] + bias[n] ),   all fp32
+//
+// - the projections of the fp32 encoder (reference transformer_opt/
+// submission.py:484-508: packed QKV, output projection, FFN input with its
+// GELU, FFN output) - on the bf16 matrix cores without giving up fp32
+// accuracy.
+//
+// The fp32 MFMA runs at 1/16 of the bf16 rate (157 against 2517 TFLOP/s), so
+// each operand is written as the sum of three bf16 numbers, which is exact
+// (8 + 8 + 8 significant bits), and the product is formed from the six
+// products of terms that matter: x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0 (the
+// three left out are below 2^-22 of |x w|, and of random sign: W's terms are
+// rounded to nearest).  Products of bf16 pairs are exact in fp32, and the
+// leading products and the five small ones have an fp32 accumulator each, so
+// the leading sum is rounded K / 16 times instead of K / 2 times by the fp32
+// MFMA.  Relative error against float64 (2-norm): 1.8e-7 at K = 1024 and
+// 3.9e-7 at K = 4096, where the library's fp32 GEMM has 5.7e-7 and 1.15e-6.
+// The ceiling is 2517 / 6 = 419 TFLOP/s; with N(0, 1) data the chip's power
+// limit holds bf16 MFMAs to about 1.85 PFLOP/s, i.e. 308.
+//
+// What a bf16 split cannot carry - infinities, values that round to infinity,
+// NaN - makes the sum NaN or infinite, so every non-finite result is
+// recomputed from the fp32 operands (fp32 MFMA or fma): those results are
+// what a plain fp32 product gives.
+//
+// W is split once (launch_split_weight), in MFMA fragment order: 6 bytes a
+// weight, one contiguous 1 KB copy per fragment, no work on it in the main
+// loop.  X is split in registers: truncation, 5.5 VALU operations per value
+// in the shadow of the MFMAs (v_dot2_f32_bf16, which would subtract a term in
+// one instruction, holds up the matrix pipe: a probe measured 14.6 ns per
+// MFMA with four other VALU operations beside it and 28 ns with four dot2).
+//
+// Tiled kernel (one workgroup = 4 wavefronts, two workgroups per CU; a 128 x
+// 128 tile): a wavefront owns 32 tokens x 128 features, as C^T = W . X^T with
+// v_mfma_f32_32x32x16_bf16, so no X value is split twice in a workgroup and a
+// lane ends holding one token and 4 consecutive features per register group.
+// K advances in stages of 32 through a 2-deep LDS ring (X as fp32 rows of 128
+// bytes, 16-byte chunks XOR-swizzled by row; W as packed), filled by LDS-DMA;
+// operands are read half a k-step ahead and the barrier of a stage sits where
+// its last fragments have been read.  The grid is persistent and copies the
+// next tile's first stages during the current tile's last.
+// Measured, against the library's fp32 GEMM: 8192 x 4096 x 1024 479 -> 321 us
+// (214 TFLOP/s; matrix pipe busy 70 % at the 1.7 GHz the power limit leaves),
+// 8192 x 1024 x 4096 460 -> 313 us, 32768 x 1536 x 512 367 -> 275 us, and the
+// GELU, a pass of its own of 39 us on the first, costs 6 us in the epilogue.
+// 256-token tiles with one workgroup per CU ran 3-6 % slower (no second
+// workgroup to cover the epilogue), 128 x 64 and 128 x 32 tiles 15-50 %.
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <type_traits>
+
+#include "ttk_common.h"
+
+namespace ttk {
+namespace {
+
+constexpr int kFlThreads = 256;  // 4 wavefronts, one per SIMD
+constexpr int kFlBK = 32;        // k per stage: 128-byte rows of X
+constexpr int kFlTile = 128;     // tokens and features per tile
+constexpr int kFlFrag = 1024;    // bytes of one fragment (32 rows x 16 k of one term)
+
+#define TTK_FL_LDS(ptr) ((__attribute__((address_space(3))) void*)(ptr))
+
+typedef __bf16 flbf16x2 __attribute__((ext_vector_type(2)));
+
+// The three bf16 terms of eight fp32 values.
+struct Split8 {
+  u32x4 t[3];
+};
+
+__device__ __forceinline__ f32x16 flmfma(const u32x4& a, const u32x4& b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                 0, 0);
+}
+__device__ __forceinline__ float high_half(float a) {
+  return __uint_as_float(__float_as_uint(a) & 0xffff0000u);
+}
+// The upper 16 bits of (a, b) as a packed pair.
+__device__ __forceinline__ unsigned pack_high(float a, float b) {
+  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+// Splits the pair (a, b) by truncation into dword d of the three terms: exact,
+// 8 + 8 + 8 significant bits.
+__device__ __forceinline__ void split_pair(Split8& s, int d, float a, float b) {
+  const float a1 = a - high_half(a), b1 = b - high_half(b);
+  const float a2 = a1 - high_half(a1), b2 = b1 - high_half(b1);
+  s.t[0][d] = pack_high(a, b);
+  s.t[1][d] = pack_high(a1, b1);
+  unsigned p2 = pack_high(a2, b2);
+  // Opaque here, so that the split stays where it is written: between the
+  // MFMAs of the step before the one that uses it.
+  asm volatile("" : "+v"(p2));
+  s.t[2][d] = p2;
+}
+
+__device__ __forceinline__ void fl_dma16(const void* gbase, unsigned voff, unsigned lds) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(voff), "s"(gbase), "s"(lds)
+               : "memory", "m0");
+#pragma clang diagnostic pop
+}
+
+// The six products kept, as (term of W, term of X): consecutive ones share an
+// operand.  Number 2 is the product of the leading terms.
+constexpr int kTermW[6] = {2, 1, 0, 0, 1, 0};
+constexpr int kTermX[6] = {0, 0, 0, 1, 1, 2};
+
+template <int N>
+__device__ __forceinline__ void fl_vm_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// Output tile of slot `slot`; false for a slot past the last tile of its XCD.
+// Workgroups are dealt round-robin to the 8 XCDs, so the slots of one
+// workgroup stay on one XCD, which gets a contiguous band of the tile grid
+// (group_m token tiles x all feature tiles) and keeps its operands in its L2.
+__device__ __forceinline__ bool fl_tile(const LinearF32Params& p, int slot, int& m0, int& n0) {
+  const int q = slot >> 3;
+  const int o = (slot & 7) * p.per_xcd + q;
+  if (q >= p.per_xcd || o >= p.tiles) return false;
+  const int span = p.group_m * p.tiles_n;
+  const int band = o / span;
+  const int first = band * p.group_m;
+  const int gs = min(p.group_m, p.tiles_m - first);
+  const int rem = o - band * span;
+  m0 = (first + rem % gs) * kFlTile;
+  n0 = (rem / gs) * kFlTile;
+  return true;
+}
+
+template <bool GELU, bool BIAS>
+__global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Params p) {
+  constexpr int R = 2;                         // LDS ring depth
+  constexpr int TN = kFlTile / 32;             // feature blocks of a wavefront
+  constexpr int kXBytes = kFlTile * kFlBK * 4;
+  constexpr int kWFrags = 6 * TN;              // W fragments of a stage
+  constexpr int kStage = kXBytes + kWFrags * kFlFrag;
+  constexpr int XC = 4;                        // X copies per wavefront per stage
+  constexpr int WC = (kWFrags + 3) / 4;        // W copies per wavefront per stage
+  constexpr int DMA = XC + WC;
+  constexpr int STORES = 4 * TN;               // stores per wavefront per tile
+  static_assert((R - 2) * DMA + STORES <= 63, "wait counts fit vmcnt");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[R * kStage];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r32 = lane & 31;
+  const int h = lane >> 5;
+
+  const int grid = static_cast<int>(gridDim.x);
+  const int slot_end = 8 * p.per_xcd;
+  const int last_fb = (p.N - 1) >> 5;          // last feature block of 32
+
+  // The copy stream runs R stages ahead of the compute stream.  Past the last
+  // tile it repeats its last stage (into ring slots that nobody reads any
+  // more), so every stage issues the same number of copies.
+  int slot = static_cast<int>(blockIdx.x), m0 = 0, n0 = 0;
+  while (slot < slot_end && !fl_tile(p, slot, m0, n0)) slot += grid;
+  if (slot >= slot_end) return;
+  const int NS = p.K / kFlBK;
+  int c_slot = slot, c_m0 = m0, c_n0 = n0, c_ks = 0;
+  auto c_advance = [&]() __attribute__((always_inline)) {
+    if (c_ks + 1 < NS) {
+      ++c_ks;
+      return;
+    }
+    int s = c_slot + grid, sm = 0, sn = 0;
+    while (s < slot_end && !fl_tile(p, s, sm, sn)) s += grid;
+    if (s < slot_end) {
+      c_slot = s;
+      c_m0 = sm;
+      c_n0 = sn;
+      c_ks = 0;
+    }
+  };
+
+  // X copies: lane L of copy c fills row 32 c + 8 wave + L / 8 at physical
+  // 16-byte chunk L % 8, which holds logical chunk (L % 8) ^ ((row >> 1) & 7).
+  // W copies: one fragment each, as packed.
+  const unsigned dchunk = static_cast<unsigned>((lane & 7) ^ (((wave & 1) << 2) | ((lane >> 4) & 3))) * 16u;
+  const int drow = 8 * wave + (lane >> 3);
+  const unsigned xpitch = static_cast<unsigned>(p.ldx) * 4u;
+  const unsigned lane16 = lane * 16;
+  const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<size_t>(TTK_FL_LDS(smem)));
+  struct Copy {
+    const float* x;
+    const char* w;
+    int xr;           // last row of X, counted from the tile's first
+    int wb;           // last feature block of W, counted from the tile's first
+    unsigned lds;     // LDS address of the ring slot
+  };
+  const int64_t wblock = static_cast<int64_t>(NS) * (6 * kFlFrag);  // bytes of a packed feature block
+  auto c_stage = [&](unsigned ring) __attribute__((always_inline)) -> Copy {
+    return Copy{p.x + static_cast<int64_t>(c_m0) * p.ldx + c_ks * kFlBK,
+                static_cast<const char*>(p.wp) + (c_n0 >> 5) * wblock + static_cast<int64_t>(c_ks) * (6 * kFlFrag),
+                p.M - 1 - c_m0, last_fb - (c_n0 >> 5), lds0 + ring};
+  };
+  auto issue_one = [&](const Copy& s, int c) __attribute__((always_inline)) {
+    if (c < XC) {
+      const int row = min(32 * c + drow, s.xr);
+      fl_dma16(s.x, static_cast<unsigned>(__umul24(row, xpitch)) + dchunk, s.lds + wave * 1024 + c * 4096);
+    } else {
+      const int f = min(wave + 4 * (c - XC), kWFrags - 1);  // fragment of the stage
+      const int fb = f / 6;
+      const char* src = s.w + min(fb, s.wb) * wblock + (f - 6 * fb) * kFlFrag;
+      fl_dma16(src, lane16, s.lds + kXBytes + f * kFlFrag);
+    }
+  };
+
+  // Fragment addresses: X chunk 4 kk + 2 h + j of row r is stored at
+  // chunk ^ ((r >> 1) & 7); W fragments are lane-ordered.
+  const int swz = (r32 >> 1) & 7;
+  unsigned xfrag[2][2];  // [k-step of the stage][16-byte half]
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      xfrag[kk][j] = (32 * wave + r32) * 128 + 16 * ((4 * kk + 2 * h + j) ^ swz);
+
+  f32x4 rx[2];            // next k-step's X, fp32
+  Split8 px[2];           // split X of this and the next k-step
+  Split8 pw[TN];          // W
+  f32x16 hi[TN], lo[TN];  // sums of the leading and of the other products
+
+  auto load_x = [&](unsigned ring, int kk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) rx[j] = *reinterpret_cast<const f32x4*>(smem + (ring + xfrag[kk][j]));
+  };
+  auto load_w = [&](Split8& d, unsigned ring, int kk, int i, int t) __attribute__((always_inline)) {
+    d.t[t] = *reinterpret_cast<const u32x4*>(smem + (ring + lane16) + kXBytes + (6 * i + 3 * kk + t) * kFlFrag);
+  };
+
+  // One k-step (P: which of its stage) in two groups of two feature blocks,
+  // six products each, the blocks interleaved.  Group 0 reads the W fragments
+  // of group 1; group 1 reads those of the next k-step's group 0 and the next
+  // k-step's X, and splits it.  So after group 0 of a stage's second k-step
+  // nobody reads that stage any more, and what follows is read from stage S +
+  // 1: `between` waits for it there, and group 1 then issues the copies of
+  // stage S + R into the freed ring slot.
+  auto kstep = [&](auto zero, auto step, unsigned ring, auto&& between) __attribute__((always_inline)) {
+    constexpr int P = decltype(step)::value;
+    unsigned nring = ring;
+    Copy copy{};
+#pragma unroll
+    for (int g = 0; g < 24; ++g) {
+      const int grp = g / 12, t = g % 12, pr = t / 2, i = 2 * grp + t % 2;
+      if (g == 12) {
+        if constexpr (P == 1) {
+          between(nring, copy);
+        }
+        load_x(nring, P ^ 1);
+      }
+      const u32x4& a = pw[i].t[kTermW[pr]];
+      const u32x4& b = px[P].t[kTermX[pr]];
+      if (pr == 2) {
+        hi[i] = flmfma(a, b, decltype(zero)::value ? f32x16{} : hi[i]);
+      } else {
+        lo[i] = flmfma(a, b, decltype(zero)::value && pr == 0 ? f32x16{} : lo[i]);
+      }
+      if (t < 6) {
+        if (grp == 0) load_w(pw[2 + t / 3], ring, P, 2 + t / 3, t % 3);
+        else load_w(pw[t / 3], nring, P ^ 1, t / 3, t % 3);
+      }
+      // The pair splits start once their operands have arrived.
+      if (grp == 1 && t >= 4 && t % 2 == 1) {
+        const int u = (t - 5) / 2;
+        split_pair(px[P ^ 1], u, rx[u >> 1][2 * (u & 1)], rx[u >> 1][2 * (u & 1) + 1]);
+      }
+      if (P == 1 && grp == 1) {
+        static_assert(DMA <= 12, "at most one copy per MFMA");
+        if (t * DMA / 12 < (t + 1) * DMA / 12) issue_one(copy, t * DMA / 12);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // Bias, activation and store of the wavefront's rows.
+  auto epilogue = [&](int tm0, int tn0) __attribute__((always_inline)) {
+    int el = lane;
+    asm volatile("" : "+v"(el));
+    const int eh = el >> 5, er = el & 31;
+    const int rows = min(p.M - tm0, kFlTile);
+    const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(
+        p.y + static_cast<int64_t>(tm0) * p.ldy, static_cast<short>(0),
+        static_cast<int>(static_cast<unsigned>((rows - 1) * p.ldy + p.N) * 4u), 0x00020000);
+    auto put = [&](int i, int g, f32x4 v) __attribute__((always_inline)) {
+      const int f = tn0 + 32 * i + 8 * g + 4 * eh;
+      if constexpr (GELU) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = gelu_exact(v[e]);
+      }
+      const int m = 32 * wave + er;
+      const unsigned off = (m < rows && f < p.N)
+          ? (static_cast<unsigned>(m) * static_cast<unsigned>(p.ldy) + static_cast<unsigned>(f)) * 4u
+          : 0x80000000u;
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), yrsrc, static_cast<int>(off), 0, 0);
+    };
+    // The bias is one more product per feature block: its three terms in k
+    // slots 0..2 of lane half 0, times ones.
+    if constexpr (BIAS) {
+      float bias[TN];
+#pragma unroll
+      for (int i = 0; i < TN; ++i) bias[i] = p.bias[min(tn0 + 32 * i + er, p.N - 1)];
+      const u32x4 ones = {eh ? 0u : 0x3f803f80u, eh ? 0u : 0x00003f80u, 0u, 0u};
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const float b1 = bias[i] - high_half(bias[i]);
+        const float b2 = b1 - high_half(b1);
+        const u32x4 terms = {pack_high(bias[i], b1), __float_as_uint(b2) >> 16, 0u, 0u};
+        lo[i] = flmfma(terms, ones, lo[i]);
+      }
+    }
+    float bad = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] = hi[i][4 * g + e] + lo[i][4 * g + e];
+          bad = __builtin_fmaf(v[e], 0.0f, bad);
+        }
+        put(i, g, v);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) != 0, 0)) {
+      fl_vm_wait<0>();
+#pragma unroll 1
+      for (int i = 0; i < TN; ++i) {
+        const float* wrow = p.w + static_cast<int64_t>(min(tn0 + 32 * i + er, p.N - 1)) * p.ldw + eh;
+        const float* xrow = p.x + static_cast<int64_t>(min(tm0 + 32 * wave + er, p.M - 1)) * p.ldx + eh;
+        f32x16 acc{};
+#pragma unroll 1
+        for (int k = 0; k < p.K; k += 2) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wrow[k], xrow[k], acc, 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          f32x4 v = {acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+          if constexpr (BIAS) v += *reinterpret_cast<const f32x4*>(p.bias + min(tn0 + 32 * i + 8 * g + 4 * eh, p.N - 4));
+          put(i, g, v);
+        }
+      }
+    }
+  };
+
+  // Prologue: copies of the first R stages; the operands of k-step 0.
+#pragma unroll 1
+  for (int s = 0; s < R; ++s) {
+    const Copy copy = c_stage(s * kStage);
+#pragma unroll
+    for (int c = 0; c < DMA; ++c) issue_one(copy, c);
+    c_advance();
+  }
+  fl_vm_wait<(R - 1) * DMA>();
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int t = 0; t < 3; ++t) load_w(pw[i], 0, 0, i, t);
+  load_x(0, 0);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) split_pair(px[0], u, rx[u >> 1][2 * (u & 1)], rx[u >> 1][2 * (u & 1) + 1]);
+
+  constexpr std::integral_constant<int, 0> kStep0{};
+  constexpr std::integral_constant<int, 1> kStep1{};
+  unsigned ring = 0;    // slot of the current stage
+  int since = R;        // stages since the last epilogue
+  for (;;) {
+    auto stage = [&](auto zero) __attribute__((always_inline)) {
+      kstep(zero, kStep0, ring, [](unsigned&, Copy&) {});
+      kstep(std::false_type{}, kStep1, ring, [&](unsigned& nring, Copy& copy) __attribute__((always_inline)) {
+        // Stage S + 1 has to be in LDS, and every wavefront done reading
+        // stage S.  Younger than stage S + 1's copies: those of S + 2 .. S +
+        // R - 1, and the stores of an epilogue less than R - 1 stages ago.
+        if (since < R - 1) {
+          fl_vm_wait<(R - 2) * DMA + STORES>();
+        } else {
+          fl_vm_wait<(R - 2) * DMA>();
+        }
+        ++since;
+        __syncthreads();
+        copy = c_stage(ring);
+        nring = ring == static_cast<unsigned>((R - 1) * kStage) ? 0u : ring + kStage;
+      });
+      ring = ring == static_cast<unsigned>((R - 1) * kStage) ? 0u : ring + kStage;
+      c_advance();
+    };
+    stage(std::true_type{});
+    for (int s = 1; s < NS; ++s) stage(std::false_type{});
+    epilogue(m0, n0);
+    since = 0;
+    slot += grid;
+    while (slot < slot_end && !fl_tile(p, slot, m0, n0)) slot += grid;
+    if (slot >= slot_end) break;
+  }
+  fl_vm_wait<0>();
+}
+
+// Small products: one workgroup of four wavefronts per TB*32 x TB*32 tile, the
+// wavefronts splitting K.  Fragments come straight from global memory (W as
+// packed, X as two 16-byte halves of a row's 8 values); the wavefronts' sums
+// are added in order through LDS.
+template <int TB, bool GELU, bool BIAS>
+__global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_kernel(LinearF32Params p) {
+  constexpr int NW = kFlThreads / 64;
+  __shared__ f32x4 part[NW][TB * TB * 4][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r32 = lane & 31;
+  const int h = lane >> 5;
+  const int m0 = static_cast<int>(blockIdx.x) / p.tiles_n * (32 * TB);
+  const int n0 = static_cast<int>(blockIdx.x) % p.tiles_n * (32 * TB);
+  const int KQ = p.K / 16;
+  const int q0 = KQ * wave / NW, q1 = KQ * (wave + 1) / NW;
+  const float* xrow[TB];
+  const u32x4* wf[TB];
+#pragma unroll
+  for (int b = 0; b < TB; ++b) {
+    xrow[b] = p.x + static_cast<int64_t>(min(m0 + 32 * b + r32, p.M - 1)) * p.ldx + 8 * h;
+    wf[b] = static_cast<const u32x4*>(p.wp) +
+            static_cast<int64_t>(min((n0 >> 5) + b, (p.N - 1) >> 5)) * KQ * 192 + lane;
+  }
+  f32x16 hi[TB][TB], lo[TB][TB];
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) hi[i][j] = lo[i][j] = f32x16{};
+  constexpr int UN = TB == 1 ? 4 : 2;  // k-steps whose loads are in flight together
+  for (int q = q0; q < q1; q += UN) {
+    f32x4 rx[UN][TB][2];
+    Split8 w[UN][TB];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      const int qq = min(q + u, q1 - 1);
+#pragma unroll
+      for (int b = 0; b < TB; ++b) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) rx[u][b][j] = *reinterpret_cast<const f32x4*>(xrow[b] + 16 * qq + 4 * j);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) w[u][b].t[t] = wf[b][(qq * 3 + t) * 64];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < UN; ++u) {
+      if (q + u < q1) {
+        Split8 x[TB];
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+          for (int d = 0; d < 4; ++d)
+            split_pair(x[b], d, rx[u][b][d >> 1][2 * (d & 1)], rx[u][b][d >> 1][2 * (d & 1) + 1]);
+#pragma unroll
+        for (int pr = 0; pr < 6; ++pr)
+#pragma unroll
+          for (int j = 0; j < TB; ++j)
+#pragma unroll
+            for (int i = 0; i < TB; ++i) {
+              f32x16& c = pr == 2 ? hi[i][j] : lo[i][j];
+              c = flmfma(w[u][i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
+            }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = hi[i][j][4 * g + e] + lo[i][j][4 * g + e];
+        part[wave][(i * TB + j) * 4 + g][lane] = v;
+      }
+  __syncthreads();
+#pragma unroll
+  for (int c = wave; c < TB * TB * 4; c += NW) {
+    const int i = c / (4 * TB), j = (c >> 2) % TB, g = c & 3;
+    const int m = m0 + 32 * j + r32, f = n0 + 32 * i + 8 * g + 4 * h;
+    f32x4 v = part[0][c][lane];
+#pragma unroll
+    for (int s = 1; s < NW; ++s) v += part[s][c][lane];
+    const float bad = __builtin_fmaf(v[0], 0.0f, v[1] * 0.0f) + __builtin_fmaf(v[2], 0.0f, v[3] * 0.0f);
+    if (m >= p.M || f >= p.N) continue;
+    if (__builtin_expect(!(bad == 0.0f), 0)) {
+      const float* xr = p.x + static_cast<int64_t>(m) * p.ldx;
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e) {
+        const float* wr = p.w + static_cast<int64_t>(f + e) * p.ldw;
+        float a = 0.0f;
+#pragma unroll 1
+        for (int k = 0; k < p.K; ++k) a = __builtin_fmaf(wr[k], xr[k], a);
+        v[e] = a;
+      }
+    }
+    if constexpr (BIAS) v += *reinterpret_cast<const f32x4*>(p.bias + f);
+    if constexpr (GELU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = gelu_exact(v[e]);
+    }
+    *reinterpret_cast<f32x4*>(p.y + static_cast<int64_t>(m) * p.ldy + f) = v;
+  }
+}
+
+template <int TB>
+hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
+  p.tiles_n = (p.N + 32 * TB - 1) / (32 * TB);
+  p.tiles_m = (p.M + 32 * TB - 1) / (32 * TB);
+  const dim3 grid(static_cast<unsigned>(p.tiles_n) * static_cast<unsigned>(p.tiles_m)), blk(kFlThreads);
+  if (gelu) {
+    if (p.bias) linear_f32_small_kernel<TB, true, true><<<grid, blk, 0, stream>>>(p);
+    else linear_f32_small_kernel<TB, true, false><<<grid, blk, 0, stream>>>(p);
+  } else {
+    if (p.bias) linear_f32_small_kernel<TB, false, true><<<grid, blk, 0, stream>>>(p);
+    else linear_f32_small_kernel<TB, false, false><<<grid, blk, 0, stream>>>(p);
+  }
+  return hipGetLastError();
+}
+
+int fl_cu_count() {
+  static std::atomic<int> cache[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+hipError_t launch_tiled(LinearF32Params& p, bool gelu, hipStream_t stream) {
+  p.tiles_m = (p.M + kFlTile - 1) / kFlTile;
+  p.tiles_n = (p.N + kFlTile - 1) / kFlTile;
+  p.tiles = p.tiles_m * p.tiles_n;
+  p.per_xcd = (p.tiles + 7) / 8;
+  p.group_m = std::max(1, std::min(p.tiles_m, p.per_xcd / p.tiles_n));
+  const int slots = fl_cu_count() / 8 * 8 * 2;  // two workgroups per CU
+  const dim3 grid(static_cast<unsigned>(std::max(8, std::min(slots, 8 * p.per_xcd)))), blk(kFlThreads);
+  if (gelu) {
+    if (p.bias) linear_f32_kernel<true, true><<<grid, blk, 0, stream>>>(p);
+    else linear_f32_kernel<true, false><<<grid, blk, 0, stream>>>(p);
+  } else {
+    if (p.bias) linear_f32_kernel<false, true><<<grid, blk, 0, stream>>>(p);
+    else linear_f32_kernel<false, false><<<grid, blk, 0, stream>>>(p);
+  }
+  return hipGetLastError();
+}
+
+// W [N, K] fp32 into its three bf16 terms (round to nearest even at every
+// step, so the terms' signs are independent), in MFMA fragment order: 16-byte
+// chunk ((fb * K/16 + q) * 3 + t) * 64 + l holds term t of
+// W[32 fb + l % 32][16 q + 8 (l / 32) .. + 7]; rows past N are zero.
+__global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4* wp, int N, int K, int64_t ldw) {
+  const int kq = K / 16;
+  const int64_t items = static_cast<int64_t>((N + 31) / 32) * kq * 64;
+  for (int64_t c = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; c < items;
+       c += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int l = static_cast<int>(c & 63);
+    const int64_t frag = c >> 6;
+    const int q = static_cast<int>(frag % kq);
+    const int64_t n = 32 * (frag / kq) + (l & 31);
+    const int64_t k = 16 * static_cast<int64_t>(q) + 8 * (l >> 5);
+    f32x4 v[2] = {};
+    if (n < N) {
+      v[0] = *reinterpret_cast<const f32x4*>(w + n * ldw + k);
+      v[1] = *reinterpret_cast<const f32x4*>(w + n * ldw + k + 4);
+    }
+    u32x4 t[3];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      float a = v[d >> 1][2 * (d & 1)], b = v[d >> 1][2 * (d & 1) + 1];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const flbf16x2 r = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+        t[i][d] = __builtin_bit_cast(unsigned, r);
+        a -= static_cast<float>(r.x);
+        b -= static_cast<float>(r.y);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) wp[(frag * 3 + i) * 64 + l] = t[i];
+  }
+}
+
+}  // namespace
+
+hipError_t launch_linear_f32(LinearF32Params& p, bool gelu, hipStream_t stream) {
+  // The form with the least expected time (us) on 256 CUs, from the measured
+  // times of the three over products from 100 x 132 x 64 to 32768 x 2048 x
+  // 512: a launch's fixed cost, then the longest chain of k-steps or the rate
+  // at which the full chip runs, whichever lasts longer.  E.g. 256 x 256 x
+  // 256: 3.7 us for 32 x 32 tiles, 6.6 for 64 x 64, 13.4 for 128 x 128; 2048
+  // x 512 x 512: 14.5, 11.6, 22.2; 4096 x 1024 x 1024: 93, 56, 49.
+  const double flops = 2.0 * p.M * p.N * p.K;
+  const double rounds = std::ceil(std::ceil(p.M / 128.0) * std::ceil(p.N / 128.0) / 256.0);
+  const double t32 = 3.2 + std::max(flops / 105e6, p.K / 256.0);
+  const double t64 = 4.0 + std::max(flops / 150e6, p.K / 102.0);
+  const double t128 = 5.0 + p.K / kFlBK * 1.37 * rounds;
+  if (t32 <= t64 && t32 <= t128) return launch_small<1>(p, gelu, stream);
+  if (t64 <= t128) return launch_small<2>(p, gelu, stream);
+  return launch_tiled(p, gelu, stream);
+}
+
+hipError_t launch_split_weight(const float* w, void* wp, int N, int K, int64_t ldw, hipStream_t stream) {
+  const int64_t items = static_cast<int64_t>((N + 31) / 32) * (K / 16) * 64;
+  const int64_t blocks = std::min<int64_t>((items + 255) / 256, 8192);
+  split_weight_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(w, static_cast<u32x4*>(wp), N, K,
+                                                                                  ldw);
+  return hipGetLastError();
+}
+
+}  // namespace ttk

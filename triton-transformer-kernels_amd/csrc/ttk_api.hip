@@ -432,6 +432,101 @@ extern "C" ttk_status ttk_linear_fwd(const void* x, const void* w, const void* b
   return TTK_OK;
 }
 
+extern "C" int64_t ttk_linear_f32_split_bytes(int64_t N, int64_t K) {
+  if (N <= 0 || K <= 0 || N >= (int64_t{1} << 31) || K >= (int64_t{1} << 22)) return 0;
+  return (N + 31) / 32 * 32 * K * 6;
+}
+
+namespace {
+
+// What both fp32 linear entry points ask of W.
+ttk_status check_linear_f32_weight(const char* what, const void* w, const void* w_split, int64_t N, int64_t K,
+                                   int64_t ldw) {
+  if (N <= 0 || K <= 0) {
+    return fail(TTK_EINVAL, "%s: N and K must be positive (N=%lld K=%lld)", what, (long long)N, (long long)K);
+  }
+  if (!w || !w_split) return fail(TTK_EINVAL, "%s: w and w_split must not be NULL", what);
+  if (K % 32 != 0 || K >= (int64_t{1} << 22) || N >= (int64_t{1} << 31)) {
+    return fail(TTK_EUNSUPPORTED, "%s: K=%lld must be a multiple of 32 below 2^22 and N=%lld below 2^31", what,
+                (long long)K, (long long)N);
+  }
+  if (!aligned16(w) || !aligned16(w_split) || ldw % 4 != 0 || ldw < K || ldw >= (int64_t{1} << 31)) {
+    return fail(TTK_EUNSUPPORTED,
+                "%s: w and w_split must be 16-byte aligned, ldw a multiple of 4 and >= K (ldw=%lld)", what,
+                (long long)ldw);
+  }
+  return TTK_OK;
+}
+
+}  // namespace
+
+extern "C" ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, int64_t K,
+                                                  int64_t ldw, void* stream) {
+  g_error[0] = '\0';
+  const ttk_status st = check_linear_f32_weight("split weight", w, w_split, N, K, ldw);
+  if (st != TTK_OK) return st;
+  const uint64_t wbytes = (static_cast<uint64_t>(N - 1) * ldw + K) * 4;
+  if (overlaps(w_split, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K)), w, wbytes)) {
+    return fail(TTK_EINVAL, "split weight: w_split overlaps w");
+  }
+  const hipError_t err = ttk::launch_split_weight(static_cast<const float*>(w), w_split, static_cast<int>(N),
+                                                  static_cast<int>(K), ldw, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(TTK_ELAUNCH, "split weight: launch failed: %s", hipGetErrorString(err));
+  return TTK_OK;
+}
+
+extern "C" ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split, const void* bias,
+                                         void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                         int64_t ldy, int activation, void* stream) {
+  g_error[0] = '\0';
+  if (activation != TTK_ACT_NONE && activation != TTK_ACT_GELU) {
+    return fail(TTK_EINVAL, "fp32 linear: unknown activation code %d", activation);
+  }
+  if (M < 0) return fail(TTK_EINVAL, "fp32 linear: M must be >= 0 (M=%lld)", (long long)M);
+  if (M == 0) return TTK_OK;
+  const ttk_status st = check_linear_f32_weight("fp32 linear", w, w_split, N, K, ldw);
+  if (st != TTK_OK) return st;
+  if (!x || !y) return fail(TTK_EINVAL, "fp32 linear: x and y must not be NULL");
+  if (N % 4 != 0 || M >= (int64_t{1} << 31)) {
+    return fail(TTK_EUNSUPPORTED, "fp32 linear: N=%lld must be a multiple of 4 and M=%lld below 2^31", (long long)N,
+                (long long)M);
+  }
+  if (!aligned16(x) || !aligned16(y) || (bias != nullptr && !aligned16(bias))) {
+    return fail(TTK_EUNSUPPORTED, "fp32 linear: x, bias and y must be 16-byte aligned");
+  }
+  if (ldx % 4 != 0 || ldy % 4 != 0 || ldx < K || ldy < N || ldx >= (int64_t{1} << 22) ||
+      ldy >= (int64_t{1} << 22)) {
+    return fail(TTK_EUNSUPPORTED,
+                "fp32 linear: ldx and ldy must be multiples of 4 below 2^22 with ldx >= K and ldy >= N "
+                "(ldx=%lld ldy=%lld)",
+                (long long)ldx, (long long)ldy);
+  }
+  const uint64_t xbytes = (static_cast<uint64_t>(M - 1) * ldx + K) * 4;
+  const uint64_t wbytes = (static_cast<uint64_t>(N - 1) * ldw + K) * 4;
+  const uint64_t ybytes = (static_cast<uint64_t>(M - 1) * ldy + N) * 4;
+  if (overlaps(y, ybytes, x, xbytes) || overlaps(y, ybytes, w, wbytes) ||
+      overlaps(y, ybytes, w_split, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K))) ||
+      (bias != nullptr && overlaps(y, ybytes, bias, static_cast<uint64_t>(N) * 4))) {
+    return fail(TTK_EINVAL, "fp32 linear: y overlaps an input");
+  }
+  ttk::LinearF32Params p{};
+  p.x = static_cast<const float*>(x);
+  p.w = static_cast<const float*>(w);
+  p.wp = w_split;
+  p.bias = static_cast<const float*>(bias);
+  p.y = static_cast<float*>(y);
+  p.ldx = ldx;
+  p.ldw = ldw;
+  p.ldy = ldy;
+  p.M = static_cast<int>(M);
+  p.N = static_cast<int>(N);
+  p.K = static_cast<int>(K);
+  const hipError_t err =
+      ttk::launch_linear_f32(p, activation == TTK_ACT_GELU, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(TTK_ELAUNCH, "fp32 linear: launch failed: %s", hipGetErrorString(err));
+  return TTK_OK;
+}
+
 namespace {
 constexpr int64_t kLnRowsPerBlock = 64;
 constexpr int64_t kLnWidth = 1024;

@@ -171,6 +171,21 @@ struct LinearLnParams {
   unsigned x_bytes, r_bytes, y_bytes;  // extents of the buffer resources
 };
 
+// Launch parameters of the fp32 Linear kernels: Y = act(X W^T + b), X [M, K],
+// W [N, K], Y [M, N] row-major fp32 with element leading dimensions.
+struct LinearF32Params {
+  const float* x;
+  const float* w;
+  const void* wp;     // W's three bf16 terms as packed by launch_split_weight
+  const float* bias;  // [N] or null
+  float* y;
+  int64_t ldx, ldw, ldy;
+  int M, N, K;
+  int tiles_m, tiles_n, tiles;
+  int per_xcd;        // tiles dealt to each XCD (the last may get fewer)
+  int group_m;        // token tiles per band of the tile order
+};
+
 // Host-side launchers (defined next to their kernels).  Return a HIP error.
 // launch_attention fills p.pair / p.units / the split plan and sizes the
 // grid itself.  `workspace` (workspace_bytes, 256-byte aligned) may be null;
@@ -192,6 +207,13 @@ hipError_t launch_gelu(int dtype, const void* x, void* y, int64_t n, hipStream_t
 // Linear + activation (0 none, 1 exact GELU) for dtype 1 (bf16) or 2 (fp16);
 // fills the tile fields of p and sizes the grid.
 hipError_t launch_linear(int dtype, int activation, LinearParams& p, hipStream_t stream);
+
+// fp32 Linear, optionally with the exact GELU; fills the tile fields of p and
+// sizes the grid.  K a multiple of 32, N of 4.
+hipError_t launch_linear_f32(LinearF32Params& p, bool gelu, hipStream_t stream);
+// W [N, K] fp32 (row stride ldw, K a multiple of 16) as three bf16 terms in
+// MFMA fragment order: ceil(N / 32) * 32 * K * 6 bytes.
+hipError_t launch_split_weight(const float* w, void* wp, int N, int K, int64_t ldw, hipStream_t stream);
 
 // Linear + residual + LayerNorm, dtype 1 (bf16) or 2 (fp16).
 hipError_t launch_linear_ln(int dtype, LinearLnParams& p, hipStream_t stream);

@@ -1,0 +1,75 @@
+"""fp32 linear layer (optionally with the exact GELU) on the gfx950 HIP kernel.
+
+``linear_f32(x, weight, split, bias, gelu=...)`` returns ``F.linear(x, weight,
+bias)``, or its exact GELU, of fp32 tensors: the projections of the fp32
+encoder (reference transformer_opt/submission.py:484-508).  The products run on
+the bf16 matrix cores, each operand as three bf16 terms that sum to it exactly,
+with an error below that of a plain fp32 GEMM (``ttk_linear_f32_fwd``).
+``split`` is the weight's terms in the order the kernel reads, made once per
+weight by ``split_weight``.
+
+The encoder model uses it (``submission.UserOptimizedTransformer``); where
+``split_weight`` or ``linear_f32_supported`` declines, the model's library
+route runs.
+"""
+
+from __future__ import annotations
+
+from typing import Optional
+
+import torch
+
+from .. import _native
+
+
+def _float_rows(t: torch.Tensor) -> bool:
+    return t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+
+
+def split_weight(weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """The three bf16 terms of ``weight`` [N, K] (N * K * 6 bytes, N rounded up
+    to 32), or None when the kernel cannot take the weight: not a contiguous
+    fp32 ROCm matrix with K a multiple of 32 and N of 4."""
+    if weight.ndim != 2 or not _float_rows(weight):
+        return None
+    n, k = weight.shape
+    if n == 0 or k == 0 or n % 4 != 0 or k % 32 != 0 or max(n, k) >= 1 << 22:
+        return None
+    lib = _native.load()
+    split = torch.empty(lib.ttk_linear_f32_split_bytes(n, k), dtype=torch.uint8, device=weight.device)
+    with torch.cuda.device(weight.device):
+        status = lib.ttk_linear_f32_split_weight(weight.data_ptr(), split.data_ptr(), n, k, k,
+                                                 torch.cuda.current_stream(weight.device).cuda_stream)
+    _native.check(status, "split weight")
+    return split
+
+
+def linear_f32_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    """Whether ``linear_f32`` takes this call (``weight`` one that
+    ``split_weight`` took).  Calls that autograd or autocast would see stay
+    with the library route."""
+    if not _float_rows(x) or x.shape[-1] != weight.shape[1] or x.device != weight.device:
+        return False
+    if bias is not None and not (_float_rows(bias) and bias.device == x.device):
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad
+                                    or (bias is not None and bias.requires_grad)):
+        return False
+    return not torch.is_autocast_enabled("cuda") and not torch.compiler.is_compiling()
+
+
+def linear_f32(x: torch.Tensor, weight: torch.Tensor, split: torch.Tensor, bias: Optional[torch.Tensor],
+               gelu: bool = False) -> torch.Tensor:
+    """``F.linear(x, weight, bias)``, with ``gelu`` its exact GELU, in one kernel."""
+    if not linear_f32_supported(x, weight, bias):
+        raise ValueError("unsupported HIP fp32 linear input")
+    lib = _native.load()
+    n, k = weight.shape
+    y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        status = lib.ttk_linear_f32_fwd(
+            x.data_ptr(), weight.data_ptr(), split.data_ptr(), None if bias is None else bias.data_ptr(),
+            y.data_ptr(), x.numel() // k, n, k, k, k, n, _native.TTK_ACT_GELU if gelu else _native.TTK_ACT_NONE,
+            torch.cuda.current_stream(x.device).cuda_stream)
+    _native.check(status, "fp32 linear")
+    return y
