@@ -1,0 +1,99 @@
+"""The fp32 attention kernel that runs on the bf16 matrix cores (head dims 32,
+64, 128): accuracy against float64 at the edges of its tiles, overlapping and
+strided rows, and operands its three-term splits cannot carry."""
+
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _exact(q, k, v, mask, causal, scale):
+    """float64 attention (rows without an allowed key: zeros) and, per output,
+    sum_t P |v|."""
+    qh, kt, vh = (t.double().permute(p).contiguous() for t, p in ((q, (0, 2, 1, 3)), (k, (0, 2, 3, 1)), (v, (0, 2, 1, 3))))
+    s = torch.matmul(qh, kt) * scale
+    seq = q.shape[1]
+    if causal:
+        s = s.masked_fill(torch.ones(seq, seq, dtype=torch.bool, device=q.device).triu(1), -math.inf)
+    if mask is not None:
+        s = s.masked_fill(~mask[:, None, None, :], -math.inf)
+    weights = torch.softmax(s, -1)
+    weights = torch.where(torch.isneginf(s.amax(-1, keepdim=True)), torch.zeros_like(weights), weights)
+    back = (0, 2, 1, 3)
+    return torch.matmul(weights, vh).permute(back), torch.matmul(weights, vh.abs()).permute(back)
+
+
+@pytest.mark.parametrize("seq_len", [1, 31, 32, 33, 64, 95, 96, 97, 129, 255, 257, 700])
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True], ids=["noncausal", "causal"])
+@pytest.mark.parametrize("masked", [False, True], ids=["nomask", "masked"])
+def test_error_against_float64(gpu_ready, seq_len, head_dim, causal, masked):
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(seq_len * head_dim)
+    packed = torch.randn(2, seq_len, 3, 3, head_dim, device="cuda", generator=g)
+    q, k, v = packed.unbind(2)
+    mask = torch.rand(2, seq_len, device="cuda", generator=g) < 0.7 if masked else None
+    with torch.inference_mode():
+        out = hip_attention(q, k, v, mask, causal=causal)
+        exact, spread = _exact(q, k, v, mask, causal, head_dim ** -0.5)
+    # fp32 scores up to ~6 in magnitude (8 in exp2 units): their rounding and
+    # the exponential's move a weight by about 8 * 2^-23; sums over the keys
+    # and the division add a few 2^-24 each.
+    bound = (8 + 4 + seq_len / 32) * 2.0 ** -23 * spread + 1e-30
+    assert bool(((out.double() - exact).abs() <= bound).all())
+
+
+def test_rows_that_overlap_and_broadcast(gpu_ready):
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(9)
+    q = torch.randn(2, 77, 4, 64, device="cuda", generator=g)
+    row = torch.randn(2, 1, 4, 64, device="cuda", generator=g)
+    line = torch.randn(2, 80 * 16, device="cuda", generator=g)
+    window = line.as_strided((2, 77, 4, 64), (80 * 16, 16, 0, 1))  # rows 16 values apart
+    with torch.inference_mode():
+        for k, v in ((row.expand(2, 77, 4, 64), window), (window, row.expand(2, 77, 4, 64)), (window, window)):
+            got = hip_attention(q, k, v, causal=True)
+            want = hip_attention(q, k.contiguous(), v.contiguous(), causal=True)
+            assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+def test_non_finite_operands_give_the_fp32_results(gpu_ready, head_dim):
+    # Infinities and NaN in q, k or v, and values that round to infinity in
+    # bf16: the same finite rows, infinities and NaN as plain fp32 arithmetic.
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (torch.randn(1, 130, 5, head_dim, device="cuda", generator=g) for _ in range(3))
+    inf, nan = math.inf, math.nan
+    k[0, 40, 0, 3] = inf     # scores of +-inf: a row of NaN, or the key drops out
+    q[0, 7, 1, 0] = nan      # one NaN row
+    v[0, 0, 2, 5] = -inf     # one output column (key 0: every row weighs it)
+    v[0, 0, 3, 2] = 3.4e38   # finite, infinite as bf16
+    k[0, 20, 4, :] = 0.0
+    k[0, 20, 4, 1] = 3.4e38  # one row's score overflows, the others' do not
+    q[0, :, 4, 1] = q[0, :, 4, 1].clamp(-2.0, 2.0)
+    q[0, 50, 4, 1] = 1000.0
+    scale = head_dim ** -0.5
+    with torch.inference_mode():
+        out = hip_attention(q, k, v, causal=True, scale=scale)
+        s = torch.matmul((q * scale).permute(0, 2, 1, 3).contiguous(), k.permute(0, 2, 3, 1).contiguous()).cpu()
+        s = s.masked_fill(torch.ones(130, 130, dtype=torch.bool).triu(1), -inf)
+        top = s.masked_fill(s.isnan(), -inf).amax(-1, keepdim=True)
+        weights = torch.exp(s - top)
+        weights = weights / weights.sum(-1, keepdim=True)
+        terms = weights[..., None] * v.permute(0, 2, 1, 3).cpu()[:, :, None]
+        want = terms.sum(-2).permute(0, 2, 1, 3)
+    out = out.cpu()
+    for head in range(5):
+        a, b = out[:, :, head], want[:, :, head]
+        both = torch.isfinite(a) & torch.isfinite(b)
+        torch.testing.assert_close(a[both], b[both], rtol=2e-4, atol=2e-4)
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b)), head

@@ -23,11 +23,13 @@
 //   rows are padded by 16 bytes, so the 16-byte MFMA operand reads of 16
 //   consecutive key rows start on distinct banks and cover all 64 banks, and
 //   every per-step operand address is the lane's base plus an immediate.
-//     - fp32: the next tile's global loads are issued into registers before
-//       the current tile's MFMAs and written to the other buffer after them.
-//       The fp32 MFMA is 16 passes long, so the matrix core is the bound and
-//       the softmax VALU of one wavefront runs under the MFMAs of the other
-//       wavefront on the SIMD.
+//     - fp32, head_dim 32 and up: products of three-term bf16 splits on the
+//       bf16 matrix cores, see attn_fwd_x3_kernel.
+//     - fp32, head_dim 8 and 16: the next tile's global loads are issued into
+//       registers before the current tile's MFMAs and written to the other
+//       buffer after them; the fp32 MFMA is 16 passes long, and the softmax
+//       VALU of one wavefront runs under the MFMAs of the other wavefront on
+//       the SIMD.
 //     - bf16/fp16: the 8-pass MFMA leaves the softmax as the bound (per
 //       64-key tile of the unmasked steady body a wavefront issues 16
 //       (head_dim 64) or 32 (128) MFMAs against 134 other VALU instructions
@@ -50,7 +52,7 @@
 //   mask) take the masked path; interior tiles run unmasked.  Causal
 //   workgroups stop at their diagonal (future tiles are never loaded) and a
 //   wavefront skips the 32-key sub-blocks entirely after its last query.
-//   fp32 with 64-key tiles: in the last tile of a query tile, wavefront 0
+//   fp32 MFMA kernel: in the last tile of a query tile, wavefront 0
 //   (whose rows are complete) takes wavefront 3's diagonal sub-block and
 //   hands its partial softmax state over through LDS, so the diagonal costs
 //   3 sub-block times instead of 4.
@@ -63,19 +65,19 @@
 //   nq+1 blocks of work and the launch has no tail.  Otherwise the flat grid
 //   is ordered heaviest query tile first, or, for an fp32 grid resident in
 //   one round, folded so that the two workgroups of a CU hold a heavy and a
-//   light tile.  fp32 non-causal with S <= 64 runs two (batch, head) pairs
-//   per workgroup (the twin grid).  When B*H is a multiple of 8 all
+//   light tile.  The fp32 MFMA kernel, non-causal with S <= 64, runs two
+//   (batch, head) pairs per workgroup (the twin grid).  When B*H is a multiple of 8 all
 //   workgroups of one head run on the same XCD (workgroups are dealt
 //   round-robin to the 8 XCDs), so a head's K/V is fetched from HBM into one
-//   XCD's L2 instead of eight.  The fp32 kernel alternates wave priority per
+//   XCD's L2 instead of eight.  The fp32 MFMA kernel alternates wave priority per
 //   tile between the two workgroups of a CU (the age order otherwise favours
 //   the older one throughout).
 // * Output: the 16-bit kernel stages each wavefront's 32 x D tile in LDS so
 //   that each store covers whole rows; fp32 stores straight from registers.
 //
-// fp32 path: v_mfma_f32_32x32x2_f32 (IEEE fp32 products, fp32 accumulate).
-// Q is pre-multiplied by scale*log2(e) so scores are already in the exp2
-// domain.  bf16/fp16 path: v_mfma_f32_32x32x16_{bf16,f16}; scores stay fp32,
+// fp32 path: fp32 products, exact to 2^-22 of each where they are formed from
+// bf16 terms, fp32 accumulate.  Q is pre-multiplied by scale*log2(e) so scores
+// are already in the exp2 domain.  bf16/fp16 path: v_mfma_f32_32x32x16_{bf16,f16}; scores stay fp32,
 // the row max is taken on raw scores and the scale is folded into one fma per
 // element before exp2; P is rounded to the input type (v_cvt_pk_bf16_f32 /
 // v_cvt_f16_f32) for the P.V product; the 16-bit A operand (8 keys of one d)
@@ -83,6 +85,7 @@
 #include <algorithm>
 #include <atomic>
 
+#include "bf16x3.h"
 #include "ttk_common.h"
 
 namespace ttk {
@@ -302,10 +305,8 @@ __device__ __forceinline__ void apply_mask(f32x16 (&s)[NSB], int k0, uint64_t kv
 }
 
 // Waves per SIMD the register budget is sized for: two workgroups per CU,
-// except fp32 head_dim 128, whose live state (64 accumulator + 64 Q registers
-// + score tiles + staging) does not fit 256 registers; it runs one workgroup
-// per CU with the accumulators in AGPRs; and 16-bit head_dim <= 64, sized for
-// three (at most 168 VGPRs; the LDS of three workgroups fits).  The 16-bit
+// except fp32 head_dim 128, whose live state does not fit 256 registers and
+// runs one workgroup per CU; and 16-bit head_dim <= 64, sized for three (at most 168 VGPRs; the LDS of three workgroups fits).  The 16-bit
 // loop is VALU-issue and latency bound, so the third workgroup pays: left to
 // itself the compiler gave the causal head_dim-64 kernel 176 VGPRs (two
 // workgroups per CU), and capping it at 168 - five registers spilled, reloaded
@@ -315,58 +316,34 @@ template <bool F32, int D>
 constexpr int kMinWaves = (D >= 128 && F32) ? 1 : ((!F32 && D <= 64) ? 3 : 2);
 
 // ----------------------------------------------------------------------------
-// fp32
+// fp32, head_dim 8 and 16 (fp32 MFMA)
 // ----------------------------------------------------------------------------
-template <int D, bool CAUSAL>
+template <int D>
 struct F32Cfg {
-  // Keys per tile.  Head dim 128 runs one workgroup per CU; 64-key tiles fit
-  // its LDS and halve the barriers (non-causal +5-7 %), but the causal
-  // variants then spill 14-51 registers (with or without the diagonal
-  // hand-off), so causal keeps 32-key tiles.
-  static constexpr int BN = (D >= 128 && CAUSAL) ? 32 : 64;
+  static constexpr int BN = 64;                     // keys per tile
   static constexpr int NSB = BN / 32;               // 32-key sub-blocks per tile
   static constexpr int CPR = D / 4;                 // 16-byte chunks per key row
   static constexpr int KS = D + 4;                  // LDS K row stride (floats, 16-byte pad)
-  static constexpr int DB = D >= 32 ? D / 32 : 1;   // output blocks of 32 d-rows
   static constexpr int G = D / 8;                   // Q.K groups of 4 k-steps
   static constexpr int CHUNKS = BN * CPR;
   static constexpr int CPT = (CHUNKS + kThreads - 1) / kThreads;  // chunks per thread
 };
 
-template <int D>
-struct VFrag32 {
-  using type = float;
-};
-template <>
-struct VFrag32<64> {
-  using type = float2;
-};
-template <>
-struct VFrag32<128> {
-  using type = f32x4;
-};
-
 template <int D, bool CAUSAL, bool HAS_MASK>
 __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_kernel(AttnParams p) {
-  using C = F32Cfg<D, CAUSAL>;
-  constexpr int BN = C::BN, NSB = C::NSB, CPR = C::CPR, KS = C::KS, DB = C::DB, CPT = C::CPT,
-                G = C::G;
-  using VF = typename VFrag32<D>::type;
+  static_assert(D <= 16, "wider heads run attn_fwd_x3_kernel");
+  using C = F32Cfg<D>;
+  constexpr int BN = C::BN, NSB = C::NSB, CPR = C::CPR, KS = C::KS, CPT = C::CPT, G = C::G;
   __shared__ __attribute__((aligned(16))) float smK[2][BN * KS];
   __shared__ __attribute__((aligned(16))) float smV[2][BN * D];
   // Causal hand-off (two-sub-block tiles): in the last key tile of a query
   // tile only wavefronts 2 (one sub-block) and 3 (two) have keys left, so
   // wavefront 0 - whose rows are complete by then - takes wavefront 3's
   // diagonal sub-block and passes its partial state through smX: per lane
-  // 16*DB accumulator values, the row max and the lane half's row sum, as
+  // 8 accumulator values, the row max and the lane half's row sum, as
   // 16-byte chunks at smX[(chunk * 64 + lane) * 4].
-  constexpr bool kHandoff = CAUSAL && NSB == 2;
-  // head_dim 8 and 16: P.V on 16x16x4 MFMAs (a 32x32 block would leave 3/4 or
-  // half of its rows empty); the accumulator keeps the f32x16 storage,
-  // elements 0-7 used.
-  constexpr bool kNarrowD = D <= 16;
-  constexpr int NX4 = 4 * DB + 1;
-  __shared__ __attribute__((aligned(16))) float smX[kHandoff ? NX4 * 256 : 4];
+  constexpr bool kHandoff = CAUSAL;
+  __shared__ __attribute__((aligned(16))) float smX[kHandoff ? 3 * 256 : 4];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -381,7 +358,7 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
   // pair of the last workgroup may not exist (odd B*H): its wavefronts hold
   // no rows and read nothing.  Built into the non-causal kernels only (the
   // causal ones keep their register budget for the pairing and hand-off).
-  constexpr bool kTwin = !CAUSAL && BN == 64;
+  constexpr bool kTwin = !CAUSAL;
   const bool twin = kTwin && p.twin != 0;
   const int slot = twin ? (wave >> 1) : 0;
   const int bh = twin ? 2 * static_cast<int>(blockIdx.x) + slot : w.bh;
@@ -488,21 +465,11 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
       const int row = sb * 32 + m;
       return *reinterpret_cast<const f32x4*>(&smK[buf][row * KS + 8 * g + 4 * h]);
     };
-    auto vread = [&](int buf, int sb, int r) -> VF {
-      const int krow = sb * 32 + acc_row(r, h);
-      const float* vrow = &smV[buf][krow * D];
-      if constexpr (DB == 1) {
-        return (D >= 32 || m < D) ? vrow[m] : 0.0f;
-      } else {
-        return *reinterpret_cast<const VF*>(vrow + DB * m);
-      }
-    };
-
     float m_run = -INFINITY;
     float l_run = 0.0f;  // partial sum over this lane half's keys
-    f32x16 acc[DB];
-#pragma unroll
-    for (int i = 0; i < DB; ++i) acc[i] = f32x16{};
+    // O^T in two blocks of 16 queries (16x16x4 MFMAs: a 32x32 block would
+    // leave 3/4 or half of its d-rows empty).
+    f32x4 acc_lo{}, acc_hi{};
 
     // One tile: S^T = K.Q^T, (mask), online softmax, O^T += V^T.P^T.
     // MASKED: apply the key / causal mask; PARTIAL: only the first of the two
@@ -517,17 +484,12 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
       constexpr bool PARTIAL = decltype(partial_tag)::value;
       constexpr int SB0 = decltype(sb0_tag)::value;
       // Live sub-blocks (nlive, 1 on partial tiles, which have two) as a
-      // compile-time count: a run-time one puts every MFMA of sub-block 1
-      // under its own branch, and the compiler copies its operands through
-      // each (head_dim 64 causal: 337 -> 271 moves, config 2 -0.6 %).
-      // Kernels that never run a partial tile at the measured shapes keep
-      // the run-time form: non-causal (partial only at a ragged end) and
-      // head dim 128 causal (one-sub-block tiles).  Their register
-      // allocation moved with the shape of that dead path, and they ran
-      // 0.8 % (non-causal head_dim 64) and 2-3 % (causal head_dim 128)
-      // slower.
-      constexpr bool kStaticLive = CAUSAL && D < 128;
-      constexpr int NL = (PARTIAL && NSB == 2) ? 1 : NSB;
+      // compile-time count in the causal kernels: a run-time one puts every
+      // MFMA of sub-block 1 under its own branch, and the compiler copies its
+      // operands through each.  Non-causal kernels see partial tiles only at a
+      // ragged end and keep the run-time form.
+      constexpr bool kStaticLive = CAUSAL;
+      constexpr int NL = PARTIAL ? 1 : NSB;
       auto live = [&](int sb) __attribute__((always_inline)) {
         return kStaticLive ? sb < NL : (!PARTIAL || sb < nlive);
       };
@@ -583,129 +545,53 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
           ls += pr;
         }
       l_run = __builtin_fmaf(l_run, alpha, ls);
-      if constexpr (kNarrowD) {
-        float a_lo, a_hi;
-        by_query16(alpha, a_lo, a_hi);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          acc[0][e] *= a_lo;
-          acc[0][4 + e] *= a_hi;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < DB; ++i) acc[i] *= alpha;
-      }
+      float a_lo, a_hi;
+      by_query16(alpha, a_lo, a_hi);
+      acc_lo *= a_lo;
+      acc_hi *= a_hi;
       m_run = m_new;
       fence();
-      if constexpr (kNarrowD) {
-        // ---- head_dim <= 16: O^T += V^T . P^T on 16x16x4 MFMAs ------------
-        // v_permlane16_swap of score registers r, r + 1 (keys k, k + 1 in lane
-        // half 0, k + 4, k + 5 in half 1, k = 8(r/4) + r%4) leaves queries
-        // 0-15 in the first and 16-31 in the second, with key k + {0,1,4,5}[g]
-        // in 16-lane row g: the B operands of the two 16-query output blocks,
-        // sharing one A operand V[key][d = l % 16].  Accumulator elements
-        // 0-3 hold block 0 (d = 4(l/16) + e, query l % 16), 4-7 block 1;
-        // for head_dim 8 the rows d >= 8 multiply zeros.
-        const int g16 = lane >> 4;
-        const int vkey = (g16 & 1) + 4 * (g16 >> 1);
-        const bool d_ok = (lane & 15) < D;
+      // ---- O^T += V^T . P^T on 16x16x4 MFMAs -----------------------------
+      // v_permlane16_swap of score registers r, r + 1 (keys k, k + 1 in lane
+      // half 0, k + 4, k + 5 in half 1, k = 8(r/4) + r%4) leaves queries
+      // 0-15 in the first and 16-31 in the second, with key k + {0,1,4,5}[g]
+      // in 16-lane row g: the B operands of the two 16-query output blocks,
+      // sharing one A operand V[key][d = l % 16].  acc_lo holds queries 0-15
+      // (d = 4(l/16) + e, query l % 16), acc_hi 16-31; for head_dim 8 the
+      // rows d >= 8 multiply zeros.
+      const int g16 = lane >> 4;
+      const int vkey = (g16 & 1) + 4 * (g16 >> 1);
+      const bool d_ok = (lane & 15) < D;
 #pragma unroll
-        for (int sb = 0; sb < NSB; ++sb) {
-          if (!live(sb)) continue;
-          const float* vb = &smV[buf][((SB0 + sb) * 32 + vkey) * D + (lane & 15 & (D - 1))];
+      for (int sb = 0; sb < NSB; ++sb) {
+        if (!live(sb)) continue;
+        const float* vb = &smV[buf][((SB0 + sb) * 32 + vkey) * D + (lane & 15 & (D - 1))];
 #pragma unroll
-          for (int r = 0; r < 16; r += 2) {
-            const float va = d_ok ? vb[(8 * (r >> 2) + (r & 3)) * D] : 0.0f;
-            const auto pq = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[sb][r]),
-                                                             __float_as_uint(s[sb][r + 1]), false, false);
-            f32x4 lo = {acc[0][0], acc[0][1], acc[0][2], acc[0][3]};
-            f32x4 hi = {acc[0][4], acc[0][5], acc[0][6], acc[0][7]};
-            lo = mfma_f32_16(va, __uint_as_float(pq[0]), lo);
-            hi = mfma_f32_16(va, __uint_as_float(pq[1]), hi);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              acc[0][e] = lo[e];
-              acc[0][4 + e] = hi[e];
-            }
-          }
+        for (int r = 0; r < 16; r += 2) {
+          const float va = d_ok ? vb[(8 * (r >> 2) + (r & 3)) * D] : 0.0f;
+          const auto pq = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[sb][r]), __float_as_uint(s[sb][r + 1]),
+                                                           false, false);
+          acc_lo = mfma_f32_16(va, __uint_as_float(pq[0]), acc_lo);
+          acc_hi = mfma_f32_16(va, __uint_as_float(pq[1]), acc_hi);
         }
-        fence();
-        return;
       }
-      // ---- O^T += V^T . P^T (V fragments read one k-step ahead) -----------
-      const int nsteps = kStaticLive ? NL * 16 : (PARTIAL ? nlive : NSB) * 16;
-      VF vf = vread(buf, SB0, 0);
-#pragma unroll
-      for (int idx = 0; idx < NSB * 16; ++idx) {
-        // Fixed trip count (fully unrolled, so s[][] stays in registers); the
-        // dead sub-blocks' k-steps are skipped (at compile time below head
-        // dim 128).
-        if (idx < nsteps) {
-          const int sb = idx >> 4;
-          const int r = idx & 15;
-          VF vn{};
-          if (idx + 1 < NSB * 16 && idx + 1 < nsteps) {
-            vn = vread(buf, SB0 + ((idx + 1) >> 4), (idx + 1) & 15);
-          }
-          const float pr = s[sb][r];
-          if constexpr (DB == 1) {
-            acc[0] = mfma_f32(vf, pr, acc[0]);
-          } else if constexpr (DB == 2) {
-            acc[0] = mfma_f32(vf.x, pr, acc[0]);
-            acc[1] = mfma_f32(vf.y, pr, acc[1]);
-          } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = mfma_f32(vf[i], pr, acc[i]);
-          }
-          vf = vn;
-        }
-        fence();
-      }
+      fence();
     };
 
-    // O = acc / l for this lane's row.
+    // O = acc / l: queries base + l % 16 and base + 16 + l % 16, d = 4(l/16) + e.
     auto epilogue = [&]() __attribute__((always_inline)) {
       const float lt = sum_with_other_half(l_run);
-      if constexpr (kNarrowD) {
-        // Block 0: query base + l % 16, block 1: base + 16 + l % 16; d = 4(l/16) + e.
-        float lt_lo, lt_hi;
-        by_query16(lt, lt_lo, lt_hi);
-        const float inv_lo = lt_lo > 0.0f ? 1.0f / lt_lo : 0.0f;
-        const float inv_hi = lt_hi > 0.0f ? 1.0f / lt_hi : 0.0f;
-        const int base = qrow - m;  // first query of the rows held (uniform)
-        const int d0 = 4 * (lane >> 4);
-        float* __restrict__ O = static_cast<float*>(p.out) + b * p.ob + hh * p.oh + d0;
-        const int r_lo = base + (lane & 15), r_hi = r_lo + 16;
-        if (d0 >= D) return;  // head_dim 8: d-rows 8-15 are empty
-        if (r_lo < S)
-          *reinterpret_cast<f32x4*>(O + r_lo * p.os) =
-              f32x4{acc[0][0] * inv_lo, acc[0][1] * inv_lo, acc[0][2] * inv_lo, acc[0][3] * inv_lo};
-        if (r_hi < S)
-          *reinterpret_cast<f32x4*>(O + r_hi * p.os) =
-              f32x4{acc[0][4] * inv_hi, acc[0][5] * inv_hi, acc[0][6] * inv_hi, acc[0][7] * inv_hi};
-        return;
-      }
-      const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-      if (qrow < S) {
-        float* __restrict__ O = static_cast<float*>(p.out) + b * p.ob + hh * p.oh + qrow * p.os;
-#pragma unroll
-        for (int j4 = 0; j4 < 4; ++j4) {
-          // Block i of the accumulator holds d = DB*row + i; register 4*j4+e
-          // holds row 8*j4 + 4h + e, so a lane's d-values form one run of 4*DB.
-          const int d0 = DB * (8 * j4 + 4 * h);
-          if (D < 32 && d0 >= D) continue;
-          float vals[4 * DB];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int i = 0; i < DB; ++i) vals[DB * e + i] = acc[i][4 * j4 + e] * inv;
-#pragma unroll
-          for (int c = 0; c < DB; ++c) {
-            *reinterpret_cast<f32x4*>(O + d0 + 4 * c) =
-                f32x4{vals[4 * c], vals[4 * c + 1], vals[4 * c + 2], vals[4 * c + 3]};
-          }
-        }
-      }
+      float lt_lo, lt_hi;
+      by_query16(lt, lt_lo, lt_hi);
+      const float inv_lo = lt_lo > 0.0f ? 1.0f / lt_lo : 0.0f;
+      const float inv_hi = lt_hi > 0.0f ? 1.0f / lt_hi : 0.0f;
+      const int base = qrow - m;  // first query of the rows held (uniform)
+      const int d0 = 4 * (lane >> 4);
+      float* __restrict__ O = static_cast<float*>(p.out) + b * p.ob + hh * p.oh + d0;
+      const int r_lo = base + (lane & 15), r_hi = r_lo + 16;
+      if (d0 >= D) return;  // head_dim 8: d-rows 8-15 are empty
+      if (r_lo < S) *reinterpret_cast<f32x4*>(O + r_lo * p.os) = acc_lo * inv_lo;
+      if (r_hi < S) *reinterpret_cast<f32x4*>(O + r_hi * p.os) = acc_hi * inv_hi;
     };
 
     // Twin grid: both pairs' only key tile, pair 2i into buffer 0 and 2i + 1
@@ -798,17 +684,12 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
           for (int g = 0; g < G; ++g) qf[g] = fq[g];
           m_run = -INFINITY;
           l_run = 0.0f;
-#pragma unroll
-          for (int i = 0; i < DB; ++i) acc[i] = f32x16{};
+          acc_lo = acc_hi = f32x4{};
           tile(std::true_type{}, std::true_type{}, std::integral_constant<int, 1>{}, buf, k0 + 32, 1,
                kvalid >> 32);
-#pragma unroll
-          for (int j = 0; j < 4 * DB; ++j) {
-            const int i = j >> 2, r0 = 4 * (j & 3);
-            *reinterpret_cast<f32x4*>(&smX[(j * 64 + lane) * 4]) =
-                f32x4{acc[i][r0], acc[i][r0 + 1], acc[i][r0 + 2], acc[i][r0 + 3]};
-          }
-          *reinterpret_cast<f32x4*>(&smX[(4 * DB * 64 + lane) * 4]) = f32x4{m_run, l_run, 0.f, 0.f};
+          *reinterpret_cast<f32x4*>(&smX[lane * 4]) = acc_lo;
+          *reinterpret_cast<f32x4*>(&smX[(64 + lane) * 4]) = acc_hi;
+          *reinterpret_cast<f32x4*>(&smX[(128 + lane) * 4]) = f32x4{m_run, l_run, 0.f, 0.f};
         }
       }
       if (q0 < S && (!CAUSAL || k0 <= q0 + 31) && !own_done) {
@@ -846,32 +727,22 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
       if (handoff && wave == 3) {
         // Merge wavefront 0's state for the second sub-block of the last
         // tile (written before the loop's final barrier).
-        const f32x4 ml = *reinterpret_cast<const f32x4*>(&smX[(4 * DB * 64 + lane) * 4]);
+        const f32x4 ml = *reinterpret_cast<const f32x4*>(&smX[(128 + lane) * 4]);
         const float mx = fmaxf(m_run, ml[0]);
         const float mu = mx == -INFINITY ? 0.0f : mx;
         const float a = fast_exp2(m_run - mu);
         const float bb = fast_exp2(ml[0] - mu);
         l_run = __builtin_fmaf(l_run, a, ml[1] * bb);
-        if constexpr (kNarrowD) {
-          // Factors per output block (queries l % 16 and 16 + l % 16).
-          float a_lo, a_hi, b_lo, b_hi;
-          by_query16(a, a_lo, a_hi);
-          by_query16(bb, b_lo, b_hi);
+        // Factors per output block (queries l % 16 and 16 + l % 16).
+        float a_lo, a_hi, b_lo, b_hi;
+        by_query16(a, a_lo, a_hi);
+        by_query16(bb, b_lo, b_hi);
+        const f32x4 x_lo = *reinterpret_cast<const f32x4*>(&smX[lane * 4]);
+        const f32x4 x_hi = *reinterpret_cast<const f32x4*>(&smX[(64 + lane) * 4]);
 #pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const float fa = j == 0 ? a_lo : a_hi, fb = j == 0 ? b_lo : b_hi;
-            const f32x4 x = *reinterpret_cast<const f32x4*>(&smX[(j * 64 + lane) * 4]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[0][4 * j + e] = __builtin_fmaf(acc[0][4 * j + e], fa, x[e] * fb);
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4 * DB; ++j) {
-            const int i = j >> 2, r0 = 4 * (j & 3);
-            const f32x4 x = *reinterpret_cast<const f32x4*>(&smX[(j * 64 + lane) * 4]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[i][r0 + e] = __builtin_fmaf(acc[i][r0 + e], a, x[e] * bb);
-          }
+        for (int e = 0; e < 4; ++e) {
+          acc_lo[e] = __builtin_fmaf(acc_lo[e], a_lo, x_lo[e] * b_lo);
+          acc_hi[e] = __builtin_fmaf(acc_hi[e], a_hi, x_hi[e] * b_hi);
         }
         m_run = mx;
       }
@@ -903,10 +774,17 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
 // fragments read with a lane stride of a whole row (32 rows x 32 bytes per
 // instruction) cost ~8 % more time at config 5b than whole rows.  V is read
 // straight into its operand layout, 256 contiguous bytes per half-wavefront.
-// Fragment layouts, accumulation order and softmax are those of
-// attn_fwd_f32_kernel's single-tile pass, so the two kernels give identical
-// results.
+// (fp32 MFMA: the launch is bound by HBM, 4.6 TB/s at [512, 64, 8, 64], so the
+// bf16 matrix cores would not shorten it.)
 // MASKED: scores need the key mask (HAS_MASK, or S < 64 leaves padded keys).
+template <int D>
+struct VFrag32 {
+  using type = float;
+};
+template <>
+struct VFrag32<64> {
+  using type = float2;
+};
 template <int D, bool HAS_MASK, bool MASKED>
 __global__ __launch_bounds__(kThreads, 2) void attn_fwd_f32_short_kernel(AttnParams p) {
   static_assert(D == 32 || D == 64, "short-sequence kernel: head_dim 32 or 64");
@@ -1948,6 +1826,441 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
   }
 }
 
+// ----------------------------------------------------------------------------
+// fp32 on the bf16 matrix cores (head_dim 32, 64, 128)
+// ----------------------------------------------------------------------------
+// The fp32 MFMA has 1/16 of the bf16 rate, and the fp32 MFMA form of this
+// kernel ran at up to 0.79 of its peak.  Here every operand - scaled Q, K, V
+// and the probabilities - is the sum of three bf16 terms (bf16x3.h) and each
+// product the six products of terms that matter, 16/6 of the fp32 MFMA's rate
+// at best.  Q's terms are rounded to nearest and K's, V's and P's truncated;
+// small products are accumulated before the leading ones of a Q.K, so its sum
+// is rounded D / 16 times.
+//
+// One workgroup = 4 wavefronts x 32 queries; 32-key tiles.  A tile's K and V
+// rows are loaded into registers a tile ahead (16 bytes a lane, through a
+// buffer resource that ends with the tile's last row, so no bounds branches),
+// split once for the workgroup and written to LDS as three row-major bf16
+// planes: K rows padded by 16 bytes, V rows unpadded with permuted column
+// blocks and read with the transposing load, as in the 16-bit kernel.  All of
+// that sits in the shadow of the Q.K MFMAs (one staged 4-value chunk per six
+// MFMAs), the softmax and the split of P in the shadow of the previous tile's
+// P.V MFMAs, and the tile's one barrier between the two halves, so fragments
+// for the start of either half are read before it.  P's reference max lags
+// (see the 16-bit kernel), so the accumulators are rescaled rarely.
+//
+// It is bound by VALU issue and the power limit together: per wavefront and
+// 32-key tile at head_dim 64, 48 MFMAs against ~330 VALU instructions (144 of
+// softmax and 88 of P's split for 16 scores a lane, 88 of staging); measured
+// at [8, 1024, 16, 64] non-causal, the matrix pipe is busy 54 % of the cycles
+// at 2.0 GHz.  Against the fp32 MFMA kernel: causal [8, 1024, 16, 64] 157 ->
+// 113 us (152 TFLOP/s), [8, 4096, 16, 64] 2181 -> 1440 us (191), [8, 1024,
+// 16, 128] 376 -> 243 us, [8, 1024, 16, 32] 94 -> 69 us; non-causal key-masked
+// [3, 777, 12, 128] 132 -> 82 us.  Error against float64 at those shapes:
+// 0.65-0.8 of the fp32 MFMA kernel's.
+//
+// A row with a non-finite operand in reach (or one that rounds to infinity)
+// comes out non-finite; its wavefront then computes its 32 rows again on the
+// fp32 MFMA straight from global memory, which gives what plain fp32
+// arithmetic gives.
+template <int D>
+struct X3Cfg {
+  static constexpr int BN = 32;              // keys per tile
+  static constexpr int G = D / 16;           // Q.K k-steps of 16
+  static constexpr int NDB = D / 32;         // output blocks of 32 d-rows
+  static constexpr int CPR = D / 4;          // 4-value chunks per row
+  static constexpr int CPT = D / 32;         // chunks of K (and of V) per thread
+  static constexpr int KS = D + 8;           // LDS K row stride (bf16, 16-byte pad)
+  static constexpr int KPL = BN * KS;        // one term of a K tile
+  static constexpr int VPL = BN * D;         // one term of a V tile
+  static constexpr bool VSWZ = D >= 64;      // V column blocks permuted per row (see H16Cfg)
+};
+// Workgroups per CU: head_dim 128 keeps its Q terms, accumulators and operand
+// rings in up to 512 registers.
+template <int D>
+constexpr int kX3Groups = D >= 128 ? 1 : 2;
+
+template <int D, bool CAUSAL, bool HAS_MASK>
+__global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(AttnParams p) {
+  using C = X3Cfg<D>;
+  constexpr int BN = C::BN, G = C::G, NDB = C::NDB, CPR = C::CPR, CPT = C::CPT, KS = C::KS, KPL = C::KPL,
+                VPL = C::VPL;
+  using St = unsigned short;
+  __shared__ __attribute__((aligned(16))) St smK[2][3 * KPL];
+  __shared__ __attribute__((aligned(16))) St smV[3][3 * VPL];
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int m = lane & 31;
+  const int h = lane >> 5;
+
+  const Work w = work_item(p, CAUSAL);
+  const int b = w.bh / p.H;
+  const int hh = w.bh - b * p.H;
+  const int S = p.S;
+  const float* __restrict__ Q = static_cast<const float*>(p.q) + b * p.qb + hh * p.qh;
+  const float* __restrict__ K = static_cast<const float*>(p.k) + b * p.kb + hh * p.kh;
+  const float* __restrict__ V = static_cast<const float*>(p.v) + b * p.vb + hh * p.vh;
+  const uint8_t* __restrict__ M = HAS_MASK ? p.mask + b * p.mb : nullptr;
+
+  // Staging: chunk i of a thread is 4 values of row `srow + i * 256 / CPR`.
+  constexpr int RPI = kThreads / CPR;  // rows per staging pass
+  const int srow = tid / CPR;
+  const int sc = tid - srow * CPR;
+  // A tile's rows are read through a buffer resource that ends with row S - 1:
+  // rows past it read as zeros (or, where rows overlap, as other rows: the
+  // mask neutralises them), without a branch.
+  f32x4 rk[CPT], rv[CPT];
+  unsigned koff[CPT], voff[CPT];
+#pragma unroll
+  for (int i = 0; i < CPT; ++i) {
+    koff[i] = (static_cast<unsigned>(srow + RPI * i) * static_cast<unsigned>(p.ks) + 4u * sc) * 4u;
+    voff[i] = (static_cast<unsigned>(srow + RPI * i) * static_cast<unsigned>(p.vs) + 4u * sc) * 4u;
+  }
+  auto tile_rsrc = [&](const float* base, int64_t rs, int t) __attribute__((always_inline)) {
+    const int rows = min(S - t * BN, BN);
+    const unsigned bytes = rows > 0 ? (static_cast<unsigned>(rows - 1) * static_cast<unsigned>(rs) + D) * 4u : 0u;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (rows > 0 ? static_cast<int64_t>(t) * BN * rs : 0)),
+                                             static_cast<short>(0), static_cast<int>(bytes), 0x00020000);
+  };
+  auto load4 = [](const __amdgpu_buffer_rsrc_t& r, unsigned off) __attribute__((always_inline)) -> f32x4 {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
+  };
+  auto put = [&](St* dst, int plane, const unsigned (&lo)[3], const unsigned (&hi)[3]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 3; ++t) *reinterpret_cast<u32x2*>(dst + t * plane) = u32x2{lo[t], hi[t]};
+  };
+  unsigned s_lo[3], s_hi[3];  // terms of the chunk being staged
+  St* const kdst = &smK[0][srow * KS + 4 * sc];
+  // 16-byte chunk c of V row r sits at c ^ 4 ((r >> 1) & 1) (head_dim 64) or
+  // c ^ 4 (r & 3) (128); 32 rows per pass of head_dim 32, else a pass adds a
+  // multiple of 4 rows for 64 and of 8 for 128.
+  const int vswz = C::VSWZ ? (D == 128 ? 4 * (srow & 3) : 4 * ((srow >> 1) & 1)) : 0;
+  St* const vdst = &smV[0][srow * D + 8 * ((sc >> 1) ^ vswz) + 4 * (sc & 1)];
+
+  const int vbase = (4 * h + ((lane & 15) >> 2)) * D + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  const int vflip = C::VSWZ ? (D == 128 ? 32 * ((lane >> 2) & 3) : 32 * ((lane >> 3) & 1)) : 0;
+  auto kread = [&](int buf, int term, int g) __attribute__((always_inline)) -> u32x4 {
+    return *reinterpret_cast<const u32x4*>(&smK[buf][term * KPL + m * KS + 16 * g + 8 * h]);
+  };
+  // A operand of P.V: d-row 32 db + m, keys 16 j + 4 h + {0..3} and + 8.
+  auto vread = [&](int buf, int term, int j, int db) __attribute__((always_inline)) -> u32x4 {
+    const int col = C::VSWZ ? vbase + ((32 * db) ^ vflip) : vbase + 32 * db;
+    const St* base = &smV[buf][term * VPL + col + 16 * j * D];
+    const u32x2 lo = __builtin_bit_cast(u32x2, lds_read_tr16(base));
+    const u32x2 hi = __builtin_bit_cast(u32x2, lds_read_tr16(base + 8 * D));
+    return u32x4{lo[0], lo[1], hi[0], hi[1]};
+  };
+
+  // The first tile's pending P is zero; what it multiplies must be finite.
+  for (int i = tid; i < 3 * VPL / 8; i += kThreads) reinterpret_cast<u32x4*>(smV[2])[i] = u32x4{0u, 0u, 0u, 0u};
+
+  for (int pass = 0; pass < w.npass; ++pass) {
+    const int qb = pass == 0 ? w.q_first : w.q_second;
+    const int q0 = qb * kBM + wave * 32;
+    const int qrow = q0 + m;
+    const int kv_end = CAUSAL ? min(S, (qb + 1) * kBM) : S;
+    const int ntiles = (kv_end + BN - 1) / BN;
+    // Tiles with keys for this wavefront.
+    const int nlive = q0 >= S ? 0 : (CAUSAL ? min(ntiles, (q0 + 31) / BN + 1) : ntiles);
+
+    bool rm = false;
+    auto load_mask = [&](int t) __attribute__((always_inline)) {
+      if constexpr (HAS_MASK) {
+        const int key = t * BN + m;
+        rm = h == 0 && key < S && M[key * p.ms] != 0;
+      }
+    };
+    auto key_bits = [&](int t) __attribute__((always_inline)) -> uint64_t {
+      if constexpr (HAS_MASK) return __builtin_amdgcn_ballot_w64(rm);
+      return range_bits(t * BN, S);
+    };
+
+    // Prologue: K(0) into its buffer, K(1) and V(0) into registers.
+    load_mask(0);
+    {
+      const auto r0 = tile_rsrc(K, p.ks, 0);
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) rk[i] = load4(r0, koff[i]);
+    }
+    // B operand of S^T = K.Q^T: k-step g, lane half h: d = 16 g + 8 h .. + 7,
+    // pre-scaled into exp2 units.
+    Split8 qf[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      f32x4 a = {0.f, 0.f, 0.f, 0.f}, c = a;
+      if (qrow < S) {
+        a = *reinterpret_cast<const f32x4*>(Q + qrow * p.qs + 16 * g + 8 * h) * p.scale_log2;
+        c = *reinterpret_cast<const f32x4*>(Q + qrow * p.qs + 16 * g + 8 * h + 4) * p.scale_log2;
+      }
+      split_pair_rn(qf[g], 0, a[0], a[1]);
+      split_pair_rn(qf[g], 1, a[2], a[3]);
+      split_pair_rn(qf[g], 2, c[0], c[1]);
+      split_pair_rn(qf[g], 3, c[2], c[3]);
+    }
+    {
+      const auto k1 = tile_rsrc(K, p.ks, 1), v0 = tile_rsrc(V, p.vs, 0);
+#pragma unroll
+      for (int i = 0; i < CPT; ++i) {
+        split_pair(rk[i][0], rk[i][1], s_lo[0], s_lo[1], s_lo[2]);
+        split_pair(rk[i][2], rk[i][3], s_hi[0], s_hi[1], s_hi[2]);
+        put(kdst + RPI * i * KS, KPL, s_lo, s_hi);
+        rk[i] = load4(k1, koff[i]);
+        rv[i] = load4(v0, voff[i]);
+      }
+    }
+    uint64_t kvalid = key_bits(0);
+    __syncthreads();
+
+    float m_run = -INFINITY;  // reference max (exp2 units) that P is taken against
+    float l_run = 0.0f;       // partial sum over this lane half's keys
+    f32x16 acc[NDB];
+#pragma unroll
+    for (int i = 0; i < NDB; ++i) acc[i] = f32x16{};
+    Split8 pk[2];  // pending P: k-step j holds registers 8 j .. 8 j + 7 of S^T
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int t = 0; t < 3; ++t) pk[j].t[t] = u32x4{0u, 0u, 0u, 0u};
+
+    // Chunk c of the staging work of iteration t (K(t + 1), V(t), interleaved):
+    // steps 0 and 1 split its pairs, step 2 writes it to LDS and loads the
+    // chunk of the tile after.
+    St* kput = kdst + 3 * KPL;  // where K(t + 1) goes
+    St* vput = vdst;            // where V(t) goes: V(t) lives in buffer t % 3
+    int vb = 2;                 // buffer of V(t - 1)
+    __amdgpu_buffer_rsrc_t knext = tile_rsrc(K, p.ks, 2), vnext = tile_rsrc(V, p.vs, 1);
+    auto stage = [&](int c, int step) __attribute__((always_inline)) {
+      const int i = c >> 1;
+      f32x4& r = (c & 1) ? rv[i] : rk[i];
+      if (step == 0) {
+        split_pair(r[0], r[1], s_lo[0], s_lo[1], s_lo[2]);
+      } else if (step == 1) {
+        split_pair(r[2], r[3], s_hi[0], s_hi[1], s_hi[2]);
+      } else if (c & 1) {
+        put(vput + RPI * i * D, VPL, s_lo, s_hi);
+        rv[i] = load4(vnext, voff[i]);
+      } else {
+        put(kput + RPI * i * KS, KPL, s_lo, s_hi);
+        rk[i] = load4(knext, koff[i]);
+      }
+    };
+    // P.V products of one k-step, in order of V's term; fragments are read two
+    // terms ahead.
+    constexpr int kVT[6] = {2, 1, 1, 0, 0, 0};
+    constexpr int kPT[6] = {0, 1, 0, 2, 1, 0};
+    constexpr int NPV = 12 * NDB;
+    u32x4 vr[3][NDB];
+    auto v_frag = [&](int vbuf, int s) __attribute__((always_inline)) {  // s: k-step * 3 + (2 - term)
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) vr[s % 3][db] = vread(vbuf, 2 - s % 3, s / 3, db);
+    };
+    // MFMA n of P.V: k-step n / (6 NDB), product (n / NDB) % 6, block n % NDB.
+    auto pv_mfma = [&](int vbuf, int n) __attribute__((always_inline)) {
+      const int j = n / (6 * NDB), pr = (n / NDB) % 6, db = n % NDB;
+      const int s = 3 * j + 2 - kVT[pr];
+      acc[db] = mfma_x3(vr[s % 3][db], pk[j].t[kPT[pr]], acc[db]);
+      if (db == 0 && (pr == 0 || pr == 1 || pr == 3) && s + 2 < 6) v_frag(vbuf, s + 2);
+    };
+    // K fragments: the two small terms of this and the next k-step, the leading
+    // term of every k-step.
+    u32x4 kr[2][2], k0f[G];
+    auto k_frag = [&](int buf, int g) __attribute__((always_inline)) {
+      kr[g & 1][0] = kread(buf, 2, g);
+      kr[g & 1][1] = kread(buf, 1, g);
+      k0f[g] = kread(buf, 0, g);
+    };
+    k_frag(0, 0);
+
+    // Iteration t: S(t) = K(t).Q^T with the staging of K(t + 1) and V(t) in its
+    // shadow; the barrier that publishes them; then P(t - 1).V(t - 1) with the
+    // softmax of S(t) in its shadow.  K(t + 1) replaces K(t - 1), read before
+    // the previous barrier, and V(t) replaces V(t - 3), read before that
+    // barrier too.
+    for (int t = 0; t < ntiles; ++t) {
+      const int kb = t & 1;
+      const int k0 = t * BN;
+      const uint64_t kv = kvalid;
+      if (HAS_MASK && t + 1 < ntiles) load_mask(t + 1);
+      const bool live = t < nlive;
+      f32x16 s[1];
+      if (live) {
+        // The small products of every k-step first, then the leading ones.
+        s[0] = f32x16{};
+        constexpr int NQK = 6 * G;
+        constexpr int kQT[5] = {0, 1, 0, 2, 1};
+#pragma unroll
+        for (int n = 0; n < NQK; ++n) {
+          if (n < 5 * G) {
+            const int g = n / 5, pr = n % 5;
+            s[0] = mfma_x3(pr == 0 ? kr[g & 1][0] : (pr < 3 ? kr[g & 1][1] : k0f[g]), qf[g].t[kQT[pr]], s[0]);
+            if (pr == 0 && g + 1 < G) k_frag(kb, g + 1);
+          } else {
+            s[0] = mfma_x3(k0f[n - 5 * G], qf[n - 5 * G].t[0], s[0]);
+          }
+          // 2 CPT chunks over 6 G = 12 CPT MFMAs: one per six.
+          if (n % 6 == 1) stage(n / 6, 0);
+          if (n % 6 == 3) stage(n / 6, 1);
+          if (n % 6 == 4) stage(n / 6, 2);
+          if (n == NQK - 3) v_frag(vb, 0);
+          if (n == NQK - 2) v_frag(vb, 1);
+          fence();
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < 2 * CPT; ++c) {
+          stage(c, 0);
+          stage(c, 1);
+          stage(c, 2);
+        }
+        if (t == nlive) {
+          v_frag(vb, 0);
+          v_frag(vb, 1);
+        }
+      }
+      knext = tile_rsrc(K, p.ks, t + 3);
+      vnext = tile_rsrc(V, p.vs, t + 2);
+      if (t + 1 < ntiles) kvalid = key_bits(t + 1);
+      __syncthreads();
+      if (live) {
+        const bool need_mask = HAS_MASK || k0 + BN > S || (CAUSAL && k0 + BN - 1 > q0);
+        constexpr int N0 = NDB >= 2 ? 4 : 2;  // MFMAs before the exponentials
+#pragma unroll
+        for (int n = 0; n < N0; ++n) pv_mfma(vb, n);
+        fence();
+        if (need_mask) apply_mask<1, CAUSAL>(s, k0, kv, qrow, h);
+        float mt = s[0][0];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[0][r]);
+        mt = max_with_other_half(mt);
+        // The reference moves once a row's max passes it by more than 8 (P <=
+        // 2^8); the accumulators are rescaled after P.V, in that case only.
+        const bool need = mt - m_run > 8.0f;
+        const bool rebase = __builtin_amdgcn_ballot_w64(need) != 0;
+        const float m_use = need ? mt : m_run;
+        const float e_use = m_use == -INFINITY ? 0.0f : m_use;
+        Split8 pn[2];
+        float ls = 0.0f;
+#pragma unroll
+        for (int n = N0; n < NPV; ++n) {
+          pv_mfma(vb, n);
+#pragma unroll
+          for (int d = 0; d < 2; ++d) {
+            constexpr int R = NPV - N0;
+            const int u = (n - N0) * 8 / R + d;
+            if (u < (n + 1 - N0) * 8 / R) {
+              const float a = fast_exp2(s[0][2 * u] - e_use), c = fast_exp2(s[0][2 * u + 1] - e_use);
+              ls += a;
+              ls += c;
+              split_pair(pn[u >> 2], u & 3, a, c);
+            }
+          }
+          if (n == NPV - 4) k_frag(kb ^ 1, 0);
+          fence();
+        }
+        if (rebase) {
+          const float alpha = m_use == m_run ? 1.0f : fast_exp2(m_run - e_use);
+          l_run *= alpha;
+#pragma unroll
+          for (int i = 0; i < NDB; ++i) acc[i] *= alpha;
+          m_run = m_use;
+        }
+        l_run += ls;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) pk[j] = pn[j];
+      } else if (t == nlive && nlive > 0) {
+#pragma unroll
+        for (int n = 0; n < NPV; ++n) pv_mfma(vb, n);
+      }
+      kput = kb ? kdst + 3 * KPL : kdst;
+      vb = vb == 2 ? 0 : vb + 1;
+      vput = vb == 2 ? vdst : vput + 3 * VPL;
+    }
+    if (nlive == ntiles) {
+      // V(ntiles - 1) became visible with the last iteration's barrier.
+      v_frag(vb, 0);
+      v_frag(vb, 1);
+#pragma unroll
+      for (int n = 0; n < NPV; ++n) pv_mfma(vb, n);
+    }
+
+    // ---- O = acc / l ---------------------------------------------------------
+    float* __restrict__ O = static_cast<float*>(p.out) + b * p.ob + hh * p.oh;
+    auto store = [&](float lt) __attribute__((always_inline)) {
+      const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+      if (qrow < S) {
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            f32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = acc[db][4 * g + e] * inv;
+            *reinterpret_cast<f32x4*>(O + qrow * p.os + 32 * db + 8 * g + 4 * h) = o;
+          }
+      }
+    };
+    const float lt = sum_with_other_half(l_run);
+    float bad = lt * 0.0f;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bad = __builtin_fmaf(acc[db][r], 0.0f, bad);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) == 0, 1)) {
+      store(lt);
+      continue;
+    }
+    // Non-finite operands (or results): these rows again on the fp32 MFMA,
+    // straight from global memory.
+    if (q0 >= S) continue;
+    m_run = -INFINITY;
+    l_run = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NDB; ++i) acc[i] = f32x16{};
+#pragma unroll 1
+    for (int t = 0; t < nlive; ++t) {
+      const int k0 = t * BN;
+      const float* kp = K + static_cast<int64_t>(min(k0 + m, S - 1)) * p.ks + h;
+      const float* qp = Q + static_cast<int64_t>(min(qrow, S - 1)) * p.qs + h;
+      f32x16 s[1];
+      s[0] = f32x16{};
+#pragma unroll 1
+      for (int d = 0; d < D; d += 2) s[0] = mfma_f32(kp[d], qp[d] * p.scale_log2, s[0]);
+      uint64_t valid = range_bits(k0, S);
+      if constexpr (HAS_MASK) {
+        valid = __builtin_amdgcn_ballot_w64(h == 0 && k0 + m < S && M[(k0 + m) * p.ms] != 0);
+      }
+      apply_mask<1, CAUSAL>(s, k0, valid, qrow, h);
+      float mt = s[0][0];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[0][r]);
+      mt = max_with_other_half(mt);
+      const float m_new = fmaxf(m_run, mt);
+      const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+      const float alpha = fast_exp2(m_run - m_use);
+      float ls = 0.0f;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        s[0][r] = fast_exp2(s[0][r] - m_use);
+        ls += s[0][r];
+      }
+      l_run = __builtin_fmaf(l_run, alpha, ls);
+      m_run = m_new;
+#pragma unroll
+      for (int i = 0; i < NDB; ++i) acc[i] *= alpha;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int key = k0 + acc_row(r, h);
+        const float* vp = V + static_cast<int64_t>(min(key, S - 1)) * p.vs + m;
+#pragma unroll
+        for (int i = 0; i < NDB; ++i) acc[i] = mfma_f32(key < S ? vp[32 * i] : 0.0f, s[0][r], acc[i]);
+      }
+    }
+    store(sum_with_other_half(l_run));
+  }
+}
+
 // Compute units of the current device (queried once per device).
 int device_cu_count() {
   static std::atomic<int> cache[64];
@@ -2053,7 +2366,7 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
             static_cast<int64_t>(p.nq) * p.BH > static_cast<int64_t>(p.cu_count)) ? 1 : 0;
   // One 64-key tile per head and rows for wavefronts 0-1 only: two heads per
   // workgroup (fp32 non-causal kernels, whose second K/V buffer is free).
-  p.twin = (dtype == 0 && !CAUSAL && F32Cfg<D, CAUSAL>::BN == 64 && p.S <= 64) ? 1 : 0;
+  p.twin = (dtype == 0 && D < 32 && !CAUSAL && p.S <= 64) ? 1 : 0;
   p.split = 0;
   if (dtype != 0 && CAUSAL && ws != nullptr) {
     const SplitPlan sp = plan_key_split(dtype, D, true, p.BH, p.S);
@@ -2137,7 +2450,13 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
                                  : static_cast<unsigned>(p.units) * static_cast<unsigned>(p.BH);
   const dim3 g(groups), blk(kThreads);
   switch (dtype) {
-    case 0: attn_fwd_f32_kernel<D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p); break;
+    case 0:
+      if constexpr (D >= 32) {
+        attn_fwd_x3_kernel<D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p);
+      } else {
+        attn_fwd_f32_kernel<D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p);
+      }
+      break;
     case 1: attn_fwd_h16_kernel<BF16, D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p); break;
     case 2: attn_fwd_h16_kernel<F16, D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p); break;
     default: return hipErrorInvalidValue;

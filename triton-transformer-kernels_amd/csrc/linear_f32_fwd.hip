@@ -52,6 +52,7 @@
 #include <cmath>
 #include <type_traits>
 
+#include "bf16x3.h"
 #include "ttk_common.h"
 
 namespace ttk {
@@ -63,38 +64,6 @@ constexpr int kFlTile = 128;     // tokens and features per tile
 constexpr int kFlFrag = 1024;    // bytes of one fragment (32 rows x 16 k of one term)
 
 #define TTK_FL_LDS(ptr) ((__attribute__((address_space(3))) void*)(ptr))
-
-typedef __bf16 flbf16x2 __attribute__((ext_vector_type(2)));
-
-// The three bf16 terms of eight fp32 values.
-struct Split8 {
-  u32x4 t[3];
-};
-
-__device__ __forceinline__ f32x16 flmfma(const u32x4& a, const u32x4& b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                 0, 0);
-}
-__device__ __forceinline__ float high_half(float a) {
-  return __uint_as_float(__float_as_uint(a) & 0xffff0000u);
-}
-// The upper 16 bits of (a, b) as a packed pair.
-__device__ __forceinline__ unsigned pack_high(float a, float b) {
-  return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-}
-// Splits the pair (a, b) by truncation into dword d of the three terms: exact,
-// 8 + 8 + 8 significant bits.
-__device__ __forceinline__ void split_pair(Split8& s, int d, float a, float b) {
-  const float a1 = a - high_half(a), b1 = b - high_half(b);
-  const float a2 = a1 - high_half(a1), b2 = b1 - high_half(b1);
-  s.t[0][d] = pack_high(a, b);
-  s.t[1][d] = pack_high(a1, b1);
-  unsigned p2 = pack_high(a2, b2);
-  // Opaque here, so that the split stays where it is written: between the
-  // MFMAs of the step before the one that uses it.
-  asm volatile("" : "+v"(p2));
-  s.t[2][d] = p2;
-}
 
 __device__ __forceinline__ void fl_dma16(const void* gbase, unsigned voff, unsigned lds) {
 #pragma clang diagnostic push
@@ -260,9 +229,9 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
       const u32x4& a = pw[i].t[kTermW[pr]];
       const u32x4& b = px[P].t[kTermX[pr]];
       if (pr == 2) {
-        hi[i] = flmfma(a, b, decltype(zero)::value ? f32x16{} : hi[i]);
+        hi[i] = mfma_x3(a, b, decltype(zero)::value ? f32x16{} : hi[i]);
       } else {
-        lo[i] = flmfma(a, b, decltype(zero)::value && pr == 0 ? f32x16{} : lo[i]);
+        lo[i] = mfma_x3(a, b, decltype(zero)::value && pr == 0 ? f32x16{} : lo[i]);
       }
       if (t < 6) {
         if (grp == 0) load_w(pw[2 + t / 3], ring, P, 2 + t / 3, t % 3);
@@ -314,7 +283,7 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
         const float b1 = bias[i] - high_half(bias[i]);
         const float b2 = b1 - high_half(b1);
         const u32x4 terms = {pack_high(bias[i], b1), __float_as_uint(b2) >> 16, 0u, 0u};
-        lo[i] = flmfma(terms, ones, lo[i]);
+        lo[i] = mfma_x3(terms, ones, lo[i]);
       }
     }
     float bad = 0.0f;
@@ -463,7 +432,7 @@ __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_
 #pragma unroll
             for (int i = 0; i < TB; ++i) {
               f32x16& c = pr == 2 ? hi[i][j] : lo[i][j];
-              c = flmfma(w[u][i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
+              c = mfma_x3(w[u][i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
             }
       }
     }
@@ -573,20 +542,11 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4
       v[0] = *reinterpret_cast<const f32x4*>(w + n * ldw + k);
       v[1] = *reinterpret_cast<const f32x4*>(w + n * ldw + k + 4);
     }
-    u32x4 t[3];
+    Split8 t;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      float a = v[d >> 1][2 * (d & 1)], b = v[d >> 1][2 * (d & 1) + 1];
+    for (int d = 0; d < 4; ++d) split_pair_rn(t, d, v[d >> 1][2 * (d & 1)], v[d >> 1][2 * (d & 1) + 1]);
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const flbf16x2 r = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-        t[i][d] = __builtin_bit_cast(unsigned, r);
-        a -= static_cast<float>(r.x);
-        b -= static_cast<float>(r.y);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) wp[(frag * 3 + i) * 64 + l] = t[i];
+    for (int i = 0; i < 3; ++i) wp[(frag * 3 + i) * 64 + l] = t.t[i];
   }
 }
 
