@@ -171,10 +171,10 @@ ttk_status ttk_attention_fwd_noalloc(const void* q, const void* k, const void* v
  * w: N elements; b: N elements or NULL; row_valid: `rows` bytes or NULL
  * (required when either zeroing flag is set).
  * Limits (TTK_EUNSUPPORTED beyond them): N <= 65536; the launch grid at most
- * 16777215 workgroups - rows <= 16777215 for widths that take the
- * one-workgroup-per-row path (N not a multiple of 16 bytes, unaligned
- * buffers, or more than 16 vectors per lane), and 4 * 64 / lanes_per_row
- * times that for the others (at least 4 * 16777215 rows).
+ * 16777215 workgroups - rows <= 16777215 for widths that do not divide into
+ * equal lane groups (N not a multiple of 16 bytes, unaligned buffers, or more
+ * than 16 vectors per lane), and 4 * 64 / lanes_per_row times that for the
+ * others (at least 4 * 16777215 rows).
  *
  * Replaces the launch of `_residual_layer_norm_fwd` inside
  * `fused_residual_layer_norm` (reference

@@ -21,8 +21,12 @@
 //    equal counts, so the update is mean = (ma + mb) / 2,
 //    M2 = M2a + M2b + (mb - ma)^2 * n / 2, and every lane of the group ends
 //    with bitwise-identical statistics.
-// Rows whose width does not fit the register-resident form, or unaligned
-// tensors, take a block-per-row fallback kernel with the same arithmetic.
+// Widths that do not divide into equal power-of-two lane groups, unaligned
+// tensors and rows too wide for one wavefront's registers take the ragged
+// kernel: the same passes with the lanes past the row's end masked, a row per
+// lane group or per workgroup, in 16-byte vectors or single elements.  Only
+// rows beyond 4096 vectors (8192 elements, unaligned) re-read the row: a
+// block-per-row kernel of three passes.
 #include "ttk_common.h"
 
 namespace ttk {
@@ -220,6 +224,140 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// Register-resident rows of any width: a row belongs to `lanes_per_row` lanes
+// (8 .. 64, of one wavefront) or, BLOCK, to the whole workgroup, and lane li
+// holds units li, li + L, ... of it, a unit being a 16-byte vector (VEC) or
+// one element.  Units past the row's end load its last unit and are masked
+// out of the sums and stores, so the loads stay straight-line code.  The mean
+// and the centred sum of squares are two sums over the group.
+// HBM-bound like the kernel above; the three-pass kernel that these widths
+// took reads every element as a scalar of its own, twice more from the caches.
+// Residual + LayerNorm, inputs beyond the caches, before -> here: bf16 7147 x
+// 1000 42.5 -> 14.6 us (3.9 TB/s), fp32 8192 x 8192 373 -> 188 us (5.7), bf16
+// 4096 x 3001 (single elements) 74 -> 28 us (3.5); fp32 65536 x 52 (13 vectors:
+// one lane a row before) 75 -> 17 us.
+template <typename T, bool VEC, int VPL, bool BLOCK, bool HAS_U>
+__device__ __forceinline__ void ln_ragged(const LnParams& p) {
+  using St = typename T::storage;
+  constexpr int VN = VEC ? Vec<T>::N : 1;
+  __shared__ float red[BLOCK ? 4 : 1];
+  const int lane = threadIdx.x & 63;
+  const int L = BLOCK ? kLnThreads : p.lanes_per_row;
+  const int li = BLOCK ? static_cast<int>(threadIdx.x) : lane & (L - 1);
+  int64_t row = blockIdx.x;
+  if constexpr (!BLOCK) {
+    const int64_t wave = static_cast<int64_t>(blockIdx.x) * (kLnThreads / 64) + (threadIdx.x >> 6);
+    row = wave * (64 / L) + lane / L;
+    if (wave * (64 / L) >= p.rows) return;  // whole wavefront
+  }
+  const bool active = row < p.rows;
+  const int64_t lrow = active ? row : p.rows - 1;
+  const int units = p.N / VN;
+
+  float r[VPL][VN];
+  {
+    u32x4 rawx[VEC ? VPL : 1], rawu[VEC ? VPL : 1];
+    St ex[VEC ? 1 : VPL], eu[VEC ? 1 : VPL];
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      const int64_t at = lrow * units + min(j * L + li, units - 1);
+      if constexpr (VEC) {
+        rawx[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.x) + at);
+        if constexpr (HAS_U) rawu[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p.u) + at);
+      } else {
+        ex[j] = static_cast<const St*>(p.x)[at];
+        if constexpr (HAS_U) eu[j] = static_cast<const St*>(p.u)[at];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      float xf[VN], uf[VN];
+      if constexpr (VEC) {
+        unpack(T{}, rawx[j], xf);
+        if constexpr (HAS_U) unpack(T{}, rawu[j], uf);
+      } else {
+        xf[0] = to_f32(T{}, ex[j]);
+        if constexpr (HAS_U) uf[0] = to_f32(T{}, eu[j]);
+      }
+#pragma unroll
+      for (int i = 0; i < VN; ++i) r[j][i] = HAS_U ? round_trip<T>(xf[i] + uf[i]) : xf[i];
+    }
+  }
+  const bool row_ok = p.valid == nullptr || p.valid[lrow] != 0;
+  if (p.zero_res && !row_ok) {
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+#pragma unroll
+      for (int i = 0; i < VN; ++i) r[j][i] = 0.0f;
+  }
+  auto store = [&](void* base, int j, const float (&v)[VN]) __attribute__((always_inline)) {
+    const int64_t at = row * units + j * L + li;
+    if constexpr (VEC) {
+      __builtin_nontemporal_store(pack(T{}, v), reinterpret_cast<u32x4*>(base) + at);
+    } else {
+      static_cast<St*>(base)[at] = static_cast<St>(from_f32(T{}, v[0]));
+    }
+  };
+  if (p.r_out != nullptr && active) {
+#pragma unroll
+    for (int j = 0; j < VPL; ++j)
+      if (j * L + li < units) store(p.r_out, j, r[j]);
+  }
+
+  auto group_sum = [&](float v) __attribute__((always_inline)) -> float {
+    if constexpr (BLOCK) return block_sum(v, red);
+    for (int off = 1; off < L; off <<= 1) v += __shfl_xor(v, off);
+    return v;
+  };
+  float sum = 0.0f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const bool in = j * L + li < units;
+#pragma unroll
+    for (int i = 0; i < VN; ++i) sum += in ? r[j][i] : 0.0f;
+  }
+  const float mean = group_sum(sum) / static_cast<float>(p.N);
+  float m2 = 0.0f;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const bool in = j * L + li < units;
+#pragma unroll
+    for (int i = 0; i < VN; ++i) {
+      const float d = in ? r[j][i] - mean : 0.0f;
+      m2 = __builtin_fmaf(d, d, m2);
+    }
+  }
+  const float rstd = rsqrtf(group_sum(m2) / static_cast<float>(p.N) + p.eps);
+  const bool zero_y = p.zero_norm && !row_ok;
+  if (!active) return;
+#pragma unroll
+  for (int j = 0; j < VPL; ++j) {
+    const int at = j * L + li;
+    if (at < units) {
+      float wf[VN], bf[VN], y[VN];
+      if constexpr (VEC) {
+        unpack(T{}, reinterpret_cast<const u32x4*>(p.w)[at], wf);
+        unpack(T{}, p.b != nullptr ? reinterpret_cast<const u32x4*>(p.b)[at] : u32x4{0u, 0u, 0u, 0u}, bf);
+      } else {
+        wf[0] = to_f32(T{}, static_cast<const St*>(p.w)[at]);
+        bf[0] = p.b != nullptr ? to_f32(T{}, static_cast<const St*>(p.b)[at]) : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < VN; ++i) y[i] = zero_y ? 0.0f : __builtin_fmaf((r[j][i] - mean) * rstd, wf[i], bf[i]);
+      store(p.y_out, j, y);
+    }
+  }
+}
+
+template <typename T, bool VEC, int VPL, bool BLOCK>
+__global__ __launch_bounds__(kLnThreads) void residual_ln_ragged_kernel(LnParams p) {
+  if (p.u != nullptr) {
+    ln_ragged<T, VEC, VPL, BLOCK, true>(p);
+  } else {
+    ln_ragged<T, VEC, VPL, BLOCK, false>(p);
+  }
+}
+
 // Fallback: one 256-thread block per row, scalar accesses, three passes over
 // the row (the row stays in L2 between passes).  Same arithmetic as above
 // except that the mean and M2 are two block-wide sums.
@@ -275,11 +413,39 @@ hipError_t launch_vec(const LnParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <typename T, bool VEC, int VPL>
+hipError_t launch_ragged(const LnParams& p, hipStream_t stream) {
+  const dim3 block(kLnThreads);
+  if (p.lanes_per_row == kLnThreads) {
+    residual_ln_ragged_kernel<T, VEC, VPL, true><<<dim3(static_cast<unsigned>(p.rows)), block, 0, stream>>>(p);
+  } else {
+    const int64_t rows_per_block = (64 / p.lanes_per_row) * (kLnThreads / 64);
+    residual_ln_ragged_kernel<T, VEC, VPL, false>
+        <<<dim3(static_cast<unsigned>((p.rows + rows_per_block - 1) / rows_per_block)), block, 0, stream>>>(p);
+  }
+  return hipGetLastError();
+}
+
+template <typename T, bool VEC>
+hipError_t launch_ragged_vpl(const LnParams& p, int vpl, hipStream_t stream) {
+  if (vpl <= 2) return launch_ragged<T, VEC, 2>(p, stream);
+  if (vpl <= 4) return launch_ragged<T, VEC, 4>(p, stream);
+  if (vpl <= 8) return launch_ragged<T, VEC, 8>(p, stream);
+  if constexpr (!VEC) {
+    if (vpl > 16) return launch_ragged<T, VEC, 32>(p, stream);
+  }
+  return launch_ragged<T, VEC, 16>(p, stream);
+}
+
 template <typename T>
-hipError_t launch_typed(const LnParams& p, bool vector_path, int vpl, hipStream_t stream) {
-  if (!vector_path) {
-    residual_ln_generic_kernel<T><<<dim3(static_cast<unsigned>(p.rows)), dim3(kLnThreads), 0, stream>>>(p);
-    return hipGetLastError();
+hipError_t launch_typed(const LnParams& p, LnPath path, int vpl, hipStream_t stream) {
+  switch (path) {
+    case LnPath::kVector: break;
+    case LnPath::kRaggedVector: return launch_ragged_vpl<T, true>(p, vpl, stream);
+    case LnPath::kRaggedElement: return launch_ragged_vpl<T, false>(p, vpl, stream);
+    case LnPath::kThreePass:
+      residual_ln_generic_kernel<T><<<dim3(static_cast<unsigned>(p.rows)), dim3(kLnThreads), 0, stream>>>(p);
+      return hipGetLastError();
   }
   switch (vpl) {
     case 1: return launch_vec<T, 1>(p, stream);
@@ -304,12 +470,12 @@ hipError_t launch_typed(const LnParams& p, bool vector_path, int vpl, hipStream_
 
 }  // namespace
 
-hipError_t launch_residual_layernorm(int dtype, const LnParams& p, bool vector_path,
-                                     int vectors_per_lane, hipStream_t stream) {
+hipError_t launch_residual_layernorm(int dtype, const LnParams& p, LnPath path, int units_per_lane,
+                                     hipStream_t stream) {
   switch (dtype) {
-    case 0: return launch_typed<F32>(p, vector_path, vectors_per_lane, stream);
-    case 1: return launch_typed<BF16>(p, vector_path, vectors_per_lane, stream);
-    case 2: return launch_typed<F16>(p, vector_path, vectors_per_lane, stream);
+    case 0: return launch_typed<F32>(p, path, units_per_lane, stream);
+    case 1: return launch_typed<BF16>(p, path, units_per_lane, stream);
+    case 2: return launch_typed<F16>(p, path, units_per_lane, stream);
     default: return hipErrorInvalidValue;
   }
 }

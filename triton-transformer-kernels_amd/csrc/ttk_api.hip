@@ -293,44 +293,60 @@ extern "C" ttk_status ttk_residual_layernorm_fwd(const void* x, const void* u, c
   p.zero_res = zero_invalid_residual ? 1 : 0;
   p.zero_norm = zero_invalid_normalized ? 1 : 0;
 
-  // Register-resident vector path: whole 16-byte vectors, aligned tensors,
-  // at most 16 vectors per lane.
+  // Whole 16-byte vectors in aligned tensors, or single elements.
   const int vn = 16 / es;
-  bool vector_path = (N % vn) == 0;
+  bool vectors = (N % vn) == 0;
   for (const void* ptr : {x, u, w, b, static_cast<const void*>(residual_out),
                           static_cast<const void*>(normalized_out)}) {
-    if (ptr != nullptr && !aligned16(ptr)) vector_path = false;
+    if (ptr != nullptr && !aligned16(ptr)) vectors = false;
   }
-  int vpl = 0;
-  if (vector_path) {
-    const int64_t nv = N / vn;
+  const int64_t units = vectors ? N / vn : N;
+  ttk::LnPath path = ttk::LnPath::kThreePass;
+  int64_t per_lane = 0;
+  p.lanes_per_row = 0;
+  if (vectors) {
+    // Equal power-of-two groups of 8 .. 64 lanes, at most 16 vectors each.
     int lpr = 1;
-    while (lpr < 64 && nv % (2 * lpr) == 0) lpr *= 2;
-    int64_t per_lane = nv / lpr;
+    while (lpr < 64 && units % (2 * lpr) == 0) lpr *= 2;
+    per_lane = units / lpr;
     // Narrow rows: several rows per wavefront, >= 4 vectors per lane.
     while (per_lane < 4 && lpr > 8) {
       lpr /= 2;
       per_lane *= 2;
     }
-    if (per_lane > 16) {
-      vector_path = false;
-    } else {
+    // Groups below 8 lanes walk rows of a few hundred bytes lane by lane; the
+    // ragged kernel's wider, partly masked groups read them coalesced (in
+    // grids it can launch: at least 16 rows per workgroup).
+    if (per_lane <= 16 && (lpr >= 8 || per_lane <= 4 || rows > 16 * kMaxGroups)) {
+      path = ttk::LnPath::kVector;
       p.lanes_per_row = lpr;
-      vpl = static_cast<int>(per_lane);
     }
   }
-  // Grid of the chosen path: one workgroup per row (fallback) or per four
-  // wavefronts of 64 / lanes_per_row rows each (vector path).
-  const int64_t groups = vector_path
-      ? ((rows + 64 / p.lanes_per_row - 1) / (64 / p.lanes_per_row) + 3) / 4
-      : rows;
+  // Widths that no equal group divides: at most one workgroup per row's worth
+  // of rows, whichever kernel runs.
+  const bool row_limited = path == ttk::LnPath::kThreePass && !(vectors && per_lane <= 16);
+  if (path == ttk::LnPath::kThreePass && units <= 256 * (vectors ? 16 : 32)) {
+    // About four units per lane on up to 64 lanes, then up to 16, then the
+    // workgroup (up to 16 vectors or 32 elements per lane).
+    int lpr = 8;
+    while (lpr < 64 && 4 * lpr < units) lpr *= 2;
+    if (units > 64 * 16) lpr = 256;
+    path = vectors ? ttk::LnPath::kRaggedVector : ttk::LnPath::kRaggedElement;
+    p.lanes_per_row = lpr;
+    per_lane = (units + lpr - 1) / lpr;
+  }
+  // Grid of the chosen path: one workgroup per row, or per four wavefronts of
+  // 64 / lanes_per_row rows each.
+  const bool by_block = path == ttk::LnPath::kThreePass || p.lanes_per_row == 256;
+  const int64_t groups =
+      by_block || row_limited ? rows : ((rows + 64 / p.lanes_per_row - 1) / (64 / p.lanes_per_row) + 3) / 4;
   if (groups > kMaxGroups) {
     return fail(TTK_EUNSUPPORTED,
                 "layernorm: %lld rows of width %lld need %lld workgroups, above the launch "
                 "limit %lld",
                 (long long)rows, (long long)N, (long long)groups, (long long)kMaxGroups);
   }
-  const hipError_t err = ttk::launch_residual_layernorm(dtype, p, vector_path, vpl,
+  const hipError_t err = ttk::launch_residual_layernorm(dtype, p, path, static_cast<int>(per_lane),
                                                         static_cast<hipStream_t>(stream));
   if (err != hipSuccess) {
     return fail(TTK_ELAUNCH, "layernorm: launch failed: %s", hipGetErrorString(err));

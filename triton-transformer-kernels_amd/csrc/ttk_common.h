@@ -128,7 +128,7 @@ struct LnParams {
   void* y_out;
   int64_t rows;
   int N;
-  int lanes_per_row;  // vector kernel: lanes that share one row (power of 2)
+  int lanes_per_row;  // lanes that share one row (power of 2; 256: the workgroup)
   float eps;
   int zero_res;
   int zero_norm;
@@ -198,8 +198,10 @@ int attention_block_m(int dtype, int D);
 // device (0 when it runs unsplit).
 int64_t attention_workspace_bytes(int dtype, int D, bool causal, int64_t BH, int64_t S);
 
-hipError_t launch_residual_layernorm(int dtype, const LnParams& p, bool vector_path,
-                                     int vectors_per_lane, hipStream_t stream);
+// Kernel of a residual + LayerNorm launch (see residual_layernorm_fwd.hip).
+enum class LnPath { kVector, kRaggedVector, kRaggedElement, kThreePass };
+hipError_t launch_residual_layernorm(int dtype, const LnParams& p, LnPath path, int units_per_lane,
+                                     hipStream_t stream);
 
 // Exact GELU over n contiguous elements of dtype (0 fp32, 1 bf16, 2 fp16).
 hipError_t launch_gelu(int dtype, const void* x, void* y, int64_t n, hipStream_t stream);
