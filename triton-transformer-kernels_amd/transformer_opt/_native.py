@@ -54,6 +54,10 @@ ATTENTION_WS_COUNTER_BYTES = 16384
 # linear + residual + LayerNorm workspace, the same for every M.
 LINEAR_LN_WS_COUNTER_BYTES = 65536
 
+# ttk_attention_fwd_ws with its five stride arrays as plain addresses (of one
+# array that holds all of them), set by load().
+attention_ws = None
+
 _lock = threading.Lock()
 _lib: Optional[ctypes.CDLL] = None
 _load_error: Optional[BaseException] = None
@@ -121,7 +125,7 @@ def _configure(lib: ctypes.CDLL) -> None:
 
 def load() -> ctypes.CDLL:
     """Load (once) and return the library; raise RuntimeError if it is absent."""
-    global _lib, _load_error
+    global _lib, _load_error, attention_ws
     if _lib is not None:
         return _lib
     with _lock:
@@ -143,11 +147,16 @@ def load() -> ctypes.CDLL:
         version = lib.ttk_abi_version()
         if version != ABI_VERSION:
             raise RuntimeError(f"{path} has ABI version {version}, expected {ABI_VERSION}")
+        attention_ws = ctypes.CFUNCTYPE(
+            ctypes.c_int, _vp, _vp, _vp, _vp, _vp, ctypes.c_int, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp,
+            ctypes.c_float, ctypes.c_int, _vp, ctypes.c_size_t, _vp)(("ttk_attention_fwd_ws", lib))
         _lib = lib
         return lib
 
 
 def available() -> bool:
+    if _lib is not None:
+        return True
     try:
         load()
         return True

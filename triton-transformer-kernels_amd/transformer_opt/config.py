@@ -53,12 +53,10 @@ class AttentionLaunchConfig:
 
 
 def attention_launch_config(head_dim: int, dtype: torch.dtype = torch.float32) -> AttentionLaunchConfig:
-    """Return the tile the HIP kernel uses for ``head_dim`` and ``dtype``.
-
-    fp32 stages K/V tiles of 64 keys (32 for head_dim 128, to stay inside the
-    64 KB of LDS that lets two workgroups share a CU); 16-bit types always use
-    64-key tiles.  Both are double-buffered.
-    """
+    """Return the nominal tile of ``head_dim`` and ``dtype``: queries per
+    workgroup and the widest block of keys between two visits of a query tile's
+    softmax state on any of its kernels (which choose narrower ones - 32 keys -
+    by head dim and length)."""
     if head_dim not in SUPPORTED_HEAD_DIMS:
         raise ValueError(f"head_dim={head_dim} is outside {sorted(SUPPORTED_HEAD_DIMS)}")
     if dtype == torch.float32:
@@ -77,24 +75,28 @@ def _validate_qkv_contract(
     """Shape/dtype/device/stride contract; same messages as the reference."""
     if q.ndim != 4:
         return "q, k, and v must have shape [batch, sequence, heads, head_dim]"
-    if k.shape != q.shape or v.shape != q.shape:
+    shape, dtype, device = q.shape, q.dtype, q.device
+    if k.shape != shape or v.shape != shape:
         return "q, k, and v must have identical shapes"
-    if k.dtype != q.dtype or v.dtype != q.dtype:
+    if k.dtype != dtype or v.dtype != dtype:
         return "q, k, and v must have identical dtypes"
-    if k.device != q.device or v.device != q.device:
+    if k.device != device or v.device != device:
         return "q, k, and v must be on the same device"
-    if q.shape[1] <= 0 or q.shape[2] <= 0 or q.shape[3] <= 0:
+    if shape[1] <= 0 or shape[2] <= 0 or shape[3] <= 0:
         return "sequence length, head count, and head dimension must be positive"
     if q.stride(-1) != 1 or k.stride(-1) != 1 or v.stride(-1) != 1:
         return "the head-dimension stride must be 1"
     if valid_token_mask is not None:
-        if valid_token_mask.shape != q.shape[:2]:
+        if valid_token_mask.shape != shape[:2]:
             return "valid_token_mask must have shape [batch, sequence]"
         if valid_token_mask.dtype is not torch.bool:
             return "valid_token_mask must have dtype torch.bool"
-        if valid_token_mask.device != q.device:
+        if valid_token_mask.device != device:
             return "valid_token_mask must be on the q/k/v device"
     return None
+
+
+_INSIDE = SupportResult(True, f"inside the {GFX_ARCH} HIP forward envelope")
 
 
 def hip_attention_support(
@@ -107,11 +109,11 @@ def hip_attention_support(
     contract_error = _validate_qkv_contract(q, k, v, valid_token_mask)
     if contract_error is not None:
         return SupportResult(False, contract_error)
-    if q.device.type != "cuda":
+    if not q.is_cuda:
         return SupportResult(False, "HIP attention requires ROCm device tensors (device type 'cuda')")
     if q.dtype not in SUPPORTED_DTYPES:
         return SupportResult(False, "HIP attention supports float32, bfloat16 and float16")
-    if q.shape[-1] not in SUPPORTED_HEAD_DIMS:
+    if q.shape[3] not in SUPPORTED_HEAD_DIMS:
         return SupportResult(
             False,
             f"head_dim={q.shape[-1]} is outside {sorted(SUPPORTED_HEAD_DIMS)}",
@@ -126,7 +128,7 @@ def hip_attention_support(
     arch = device_arch(q.device)
     if arch != GFX_ARCH:
         return SupportResult(False, f"device architecture {arch} is not {GFX_ARCH}")
-    return SupportResult(True, f"inside the {GFX_ARCH} HIP forward envelope")
+    return _INSIDE
 
 
 _ARCH_CACHE: dict = {}

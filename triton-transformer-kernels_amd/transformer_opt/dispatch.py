@@ -32,7 +32,7 @@ from typing import Optional, Tuple
 import torch
 
 from .config import ATTENTION_BACKENDS, hip_attention_support
-from .kernels.attention import hip_attention, hip_available
+from .kernels.attention import hip_available, run_attention
 
 
 @dataclass(frozen=True)
@@ -107,11 +107,10 @@ def attention_forward(
     if backend == "reference":
         output = explicit_attention(q, k, v, valid_token_mask, causal, scale)
         return output, AttentionDispatch(backend, "reference", "explicit reference backend")
-    route = _route_phrase(backend)
     if not hip_available():
-        raise RuntimeError(f"{route} but ROCm/the HIP kernel library is unavailable")
+        raise RuntimeError(f"{_route_phrase(backend)} but ROCm/the HIP kernel library is unavailable")
     support = hip_attention_support(q, k, v, valid_token_mask)
     if not support.supported:
-        raise ValueError(f"{route} but unsupported: {support.reason}")
-    output = hip_attention(q, k, v, valid_token_mask, causal=causal, scale=scale)
+        raise ValueError(f"{_route_phrase(backend)} but unsupported: {support.reason}")
+    output = run_attention(q, k, v, valid_token_mask, causal, scale)
     return output, AttentionDispatch(backend, "hip", support.reason)

@@ -8,6 +8,7 @@ current stream.  Unsupported inputs raise; nothing falls back.
 
 from __future__ import annotations
 
+import ctypes
 import threading
 from collections import OrderedDict
 from typing import Optional
@@ -15,6 +16,7 @@ from typing import Optional
 import torch
 
 from .. import _native
+from .._launch import launch, raw_stream, vector_ready
 from ..config import hip_attention_support
 
 _DTYPE_CODE = {
@@ -50,6 +52,9 @@ def _workspace_bytes(lib, dtype_code: int, batch: int, seq_len: int, heads: int,
     return nbytes
 
 
+_Strides = ctypes.c_int64 * 14  # q, k, v and out (3 each), mask (2)
+
+
 def _workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
     """Workspace of the key-split attention schedule for the current stream.
 
@@ -69,7 +74,7 @@ def _workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         ws[:_native.ATTENTION_WS_COUNTER_BYTES].zero_()
         return ws
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, raw_stream(device.index))
     with _WS_LOCK:
         ws = _WORKSPACES.pop(key, None)
         if ws is None or ws.numel() < nbytes:
@@ -78,12 +83,6 @@ def _workspace(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
         while len(_WORKSPACES) > _MAX_WORKSPACES:
             _WORKSPACES.popitem(last=False)
     return ws
-
-
-def _vector_ready(t: torch.Tensor) -> bool:
-    """Rows start on 16-byte boundaries (the kernel's 128-bit accesses)."""
-    es = t.element_size()
-    return t.data_ptr() % 16 == 0 and all((s * es) % 16 == 0 for s in t.stride()[:3])
 
 
 def hip_attention(
@@ -102,56 +101,58 @@ def hip_attention(
     missing library raises ``RuntimeError``.  Use
     ``transformer_opt.dispatch.attention_forward`` for the audited entry point.
     """
-    lib = _native.load()
+    _native.load()
     support = hip_attention_support(q, k, v, valid_token_mask)
     if not support.supported:
         raise ValueError(f"unsupported HIP attention input: {support.reason}")
 
+    return run_attention(q, k, v, valid_token_mask, causal, scale, out)
+
+
+def run_attention(q, k, v, valid_token_mask, causal: bool, scale: Optional[float],
+                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``hip_attention`` on inputs that ``hip_attention_support`` accepted, with
+    the library loaded."""
     # Arbitrary B/S/H strides are part of the contract; rows that are not
     # 16-byte aligned are copied into fresh (aligned) storage so the kernel
     # keeps its vector loads - also for a contiguous view at an odd storage
     # offset, which ``contiguous()`` would return unchanged.
-    if not _vector_ready(q):
+    if not vector_ready(q):
         q = q.clone(memory_format=torch.contiguous_format)
-    if not _vector_ready(k):
+    if not vector_ready(k):
         k = k.clone(memory_format=torch.contiguous_format)
-    if not _vector_ready(v):
+    if not vector_ready(v):
         v = v.clone(memory_format=torch.contiguous_format)
 
-    batch, seq_len, num_heads, head_dim = q.shape
+    shape = q.shape
+    batch, seq_len, num_heads, head_dim = shape
     if out is None:
-        out = torch.empty((batch, seq_len, num_heads, head_dim), dtype=q.dtype, device=q.device)
-    elif out.shape != q.shape or out.dtype != q.dtype or out.device != q.device or out.stride(-1) != 1 \
-            or not _vector_ready(out):
+        out = torch.empty(shape, dtype=q.dtype, device=q.device)
+    elif out.shape != shape or out.dtype != q.dtype or out.device != q.device or out.stride(-1) != 1 \
+            or not vector_ready(out):
         raise ValueError("out must be a [B, S, H, D] tensor like q with 16-byte aligned rows")
     if batch == 0:
         return out
 
     softmax_scale = head_dim ** -0.5 if scale is None else float(scale)
-    mask_ptr = None
-    mask_strides = None
+    mask_ptr, mask_strides = None, (0, 0)
     if valid_token_mask is not None:
-        mask_ptr = valid_token_mask.data_ptr()
-        mask_strides = _native.strides2(valid_token_mask.stride())
+        mask_ptr, mask_strides = valid_token_mask.data_ptr(), valid_token_mask.stride()
+    strides = _Strides(*q.stride()[:3], *k.stride()[:3], *v.stride()[:3], *out.stride()[:3], *mask_strides)
+    at = ctypes.addressof(strides)
 
+    index = q.get_device()
     dtype_code = _DTYPE_CODE[q.dtype]
-    with torch.cuda.device(q.device):
-        nbytes = _workspace_bytes(lib, dtype_code, batch, seq_len, num_heads, head_dim, causal,
-                                  q.device.index)
-        ws = _workspace(q.device, nbytes)
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        status = lib.ttk_attention_fwd_ws(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), mask_ptr, out.data_ptr(),
-            dtype_code,
-            batch, seq_len, num_heads, head_dim,
-            _native.strides3(q.stride()[:3]),
-            _native.strides3(k.stride()[:3]),
-            _native.strides3(v.stride()[:3]),
-            mask_strides,
-            _native.strides3(out.stride()[:3]),
-            softmax_scale, 1 if causal else 0,
-            None if ws is None else ws.data_ptr(), nbytes, stream,
-        )
+    # Only 16-bit causal launches have a key-split schedule.
+    nbytes, ws = 0, None
+    if causal and dtype_code != _native.TTK_F32:
+        with torch.cuda.device(index):
+            nbytes = _workspace_bytes(_native.load(), dtype_code, batch, seq_len, num_heads, head_dim, causal, index)
+            ws = _workspace(q.device, nbytes)
+    status = launch(
+        index, _native.attention_ws, q.data_ptr(), k.data_ptr(), v.data_ptr(), mask_ptr, out.data_ptr(), dtype_code,
+        batch, seq_len, num_heads, head_dim, at, at + 24, at + 48, None if mask_ptr is None else at + 96, at + 72,
+        softmax_scale, 1 if causal else 0, None if ws is None else ws.data_ptr(), nbytes)
     _native.check(status, "HIP attention")
     return out
 

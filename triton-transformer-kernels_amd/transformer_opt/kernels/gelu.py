@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 
 from .. import _native
+from .._launch import launch
 from .attention import _DTYPE_CODE
 
 
@@ -23,9 +24,8 @@ def _check(x: torch.Tensor) -> None:
 
 def _launch(src: torch.Tensor, dst: torch.Tensor) -> None:
     lib = _native.load()
-    with torch.cuda.device(src.device):
-        status = lib.ttk_gelu_fwd(src.data_ptr(), dst.data_ptr(), _DTYPE_CODE[src.dtype], src.numel(),
-                                  torch.cuda.current_stream(src.device).cuda_stream)
+    status = launch(src.get_device(), lib.ttk_gelu_fwd, src.data_ptr(), dst.data_ptr(), _DTYPE_CODE[src.dtype],
+                    src.numel())
     _native.check(status, "gelu")
 
 

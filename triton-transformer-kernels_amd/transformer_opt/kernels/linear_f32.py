@@ -20,6 +20,7 @@ from typing import Optional
 import torch
 
 from .. import _native
+from .._launch import launch
 
 
 def _float_rows(t: torch.Tensor) -> bool:
@@ -37,9 +38,7 @@ def split_weight(weight: torch.Tensor) -> Optional[torch.Tensor]:
         return None
     lib = _native.load()
     split = torch.empty(lib.ttk_linear_f32_split_bytes(n, k), dtype=torch.uint8, device=weight.device)
-    with torch.cuda.device(weight.device):
-        status = lib.ttk_linear_f32_split_weight(weight.data_ptr(), split.data_ptr(), n, k, k,
-                                                 torch.cuda.current_stream(weight.device).cuda_stream)
+    status = launch(weight.get_device(), lib.ttk_linear_f32_split_weight, weight.data_ptr(), split.data_ptr(), n, k, k)
     _native.check(status, "split weight")
     return split
 
@@ -66,10 +65,9 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor, split: torch.Tensor, bias:
     lib = _native.load()
     n, k = weight.shape
     y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
-        status = lib.ttk_linear_f32_fwd(
-            x.data_ptr(), weight.data_ptr(), split.data_ptr(), None if bias is None else bias.data_ptr(),
-            y.data_ptr(), x.numel() // k, n, k, k, k, n, _native.TTK_ACT_GELU if gelu else _native.TTK_ACT_NONE,
-            torch.cuda.current_stream(x.device).cuda_stream)
+    status = launch(
+        x.get_device(), lib.ttk_linear_f32_fwd, x.data_ptr(), weight.data_ptr(), split.data_ptr(),
+        None if bias is None else bias.data_ptr(), y.data_ptr(), x.numel() // k, n, k, k, k, n,
+        _native.TTK_ACT_GELU if gelu else _native.TTK_ACT_NONE)
     _native.check(status, "fp32 linear")
     return y

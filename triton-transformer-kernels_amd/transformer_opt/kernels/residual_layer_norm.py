@@ -18,6 +18,7 @@ from typing import Optional, Tuple
 import torch
 
 from .. import _native
+from .._launch import launch
 from ..config import LAYER_NORM_MAX_WIDTH, SUPPORTED_DTYPES
 from .attention import _DTYPE_CODE
 
@@ -25,7 +26,7 @@ from .attention import _DTYPE_CODE
 def _check_rows(x: torch.Tensor, what: str) -> None:
     if x.ndim < 2:
         raise ValueError(f"{what} must have rank two or higher")
-    if x.device.type != "cuda":
+    if not x.is_cuda:
         raise ValueError("fused residual LayerNorm requires co-located ROCm device tensors")
     if x.dtype not in SUPPORTED_DTYPES:
         raise ValueError("fused residual LayerNorm supports float32, bfloat16 and float16")
@@ -63,24 +64,20 @@ def _check_mask(x: torch.Tensor, valid_token_mask: Optional[torch.Tensor]) -> No
 
 def _launch(x, update, weight, bias, eps, mask, residual_out, normalized_out,
             zero_invalid_residual, zero_invalid_normalized) -> None:
-    lib = _native.load()
     width = x.shape[-1]
-    rows = x.numel() // width
-    with torch.cuda.device(x.device):
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        status = lib.ttk_residual_layernorm_fwd(
-            x.data_ptr(),
-            update.data_ptr() if update is not None else None,
-            weight.data_ptr(),
-            bias.data_ptr() if bias is not None else None,
-            mask.data_ptr() if mask is not None else None,
-            residual_out.data_ptr() if residual_out is not None else None,
-            normalized_out.data_ptr(),
-            _DTYPE_CODE[x.dtype], rows, width, float(eps),
-            1 if zero_invalid_residual else 0,
-            1 if zero_invalid_normalized else 0,
-            stream,
-        )
+    status = launch(
+        x.get_device(), _native.load().ttk_residual_layernorm_fwd,
+        x.data_ptr(),
+        update.data_ptr() if update is not None else None,
+        weight.data_ptr(),
+        bias.data_ptr() if bias is not None else None,
+        mask.data_ptr() if mask is not None else None,
+        residual_out.data_ptr() if residual_out is not None else None,
+        normalized_out.data_ptr(),
+        _DTYPE_CODE[x.dtype], x.numel() // width, width, float(eps),
+        1 if zero_invalid_residual else 0,
+        1 if zero_invalid_normalized else 0,
+    )
     _native.check(status, "HIP residual LayerNorm")
 
 
