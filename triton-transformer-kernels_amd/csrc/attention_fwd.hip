@@ -40,7 +40,7 @@
 //       software-pipelined.  Unmasked tiles run two phases per tile:
 //       Q.K of tile t+1 interleaved with the exp2 and 16-bit rounding of
 //       tile t's scores, then the P.V of tile t interleaved with the row max
-//       of tile t+1.  Key-masked launches run one stream interleaving the
+//       of tile t+1.  Key-masked tiles run one stream interleaving the
 //       P.V of tile t-1 with the softmax of tile t.  K and V tiles are
 //       copied global->LDS by LDS-DMA (global_load_lds_dwordx4, no register
 //       staging), spread over the MFMA groups of the pipelined loop; V stays
@@ -49,7 +49,9 @@
 // * Masking: key validity (key mask and key < S) is a wave-uniform 64-bit
 //   ballot per tile; with the lane's causal limit it becomes one bit mask per
 //   32-key sub-block.  Only tiles that need it (diagonal, ragged end, key
-//   mask) take the masked path; interior tiles run unmasked.  Causal
+//   mask) take the masked path; interior tiles run unmasked, and key
+//   blocks before the first and after the last valid key are not visited
+//   (scan_keys).  Causal
 //   workgroups stop at their diagonal (future tiles are never loaded) and a
 //   wavefront skips the 32-key sub-blocks entirely after its last query.
 //   fp32 MFMA kernel: in the last tile of a query tile, wavefront 0
@@ -84,6 +86,7 @@
 // is two transposing 8-byte LDS reads of the row-major V tile.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "bf16x3.h"
 #include "ttk_common.h"
@@ -304,13 +307,120 @@ __device__ __forceinline__ void apply_mask(f32x16 (&s)[NSB], int k0, uint64_t kv
   }
 }
 
+// Keys a masked query tile has to visit: those from the first 64-key block with
+// a valid key up to the end of the last such block.
+struct KeySpan {
+  int first;  // a multiple of 64
+  int end;
+  int full;   // 64-key blocks from the first after which one holds an invalid
+              // key (the first itself may): blocks 1 .. full - 1 are whole
+};
+constexpr int kSpanKeys = 512;  // shorter key ranges are visited whole
+constexpr int kSpanLds = 4;     // words of LDS scratch
+
+// Key span of the keys [0, end) of mask row M.  V rows
+// that drop out have weight zero, and 0 * V is left out only where V is finite:
+// with a non-finite value among them the span stays whole (and full is 0).
+//
+// Padding otherwise costs what valid keys cost, and a mask is applied to every
+// tile (about half as much VALU work again as the softmax).  With the span, the
+// 16-bit kernel runs its pipelined body on the whole blocks and applies masks
+// only where one has an invalid key.  Measured with prefixes uniform in [S / 2,
+// S]: fp16 [6, 1000, 16, 64] 50 -> 36 us, bf16 causal [4, 2048, 16, 64] 67 ->
+// 49 us, bf16 [4, 2048, 16, 128] 168 -> 123 us, fp32 [3, 777, 12, 128] (lengths
+// 470, 543, 404) 82 -> 66 us.  The scan costs 0.5 - 1 us of a launch: nothing
+// on up to 512 keys, where it gained nothing either (bf16 [2, 300, 4, 64] 9.6
+// -> 10.1 us with it), and 0 - 7 % where invalid keys are scattered over all
+// blocks (bf16 [2, 600, 8, 64] 14.6 -> 15.6 us, fp16 [6, 1000, 16, 64] 46 -> 47
+// us, bf16 [8, 1000, 16, 64] 61 -> 59 us).
+//
+// The scan is one dependent load: every wavefront reads the whole row (64 keys
+// a lane, as bytes of a bool mask with unit stride), so nothing is exchanged.
+template <typename St, unsigned INF, int D>  // INF: magnitude bits of infinity
+__device__ __forceinline__ KeySpan scan_keys(const uint8_t* M, const St* V, int64_t vs, int end, int* lds) {
+  typedef u32x4 __attribute__((aligned(1))) Bytes16;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63;
+  const int nb = (end + 63) >> 6;
+  int lo = -1, hi = -1, stop = -1;
+  for (int b = 0; b < nb; b += 64) {
+    // The last chunk of the row is read as its last 16 bytes: keys of the chunk
+    // before count twice, which at most keeps a block.
+    unsigned any = 0, zero = 0;
+    const int k = 64 * min(b + lane, nb - 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const u32x4 x = *reinterpret_cast<const Bytes16*>(M + min(k + 16 * i, end - 16));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        any |= x[e];
+        zero |= (x[e] - 0x01010101u) & ~x[e] & 0x80808080u;  // set if a byte is zero
+      }
+    }
+    const bool real = b + lane < nb;
+    const uint64_t valid = __builtin_amdgcn_ballot_w64(real && any != 0);
+    uint64_t bad = __builtin_amdgcn_ballot_w64(real && zero != 0);
+    if (valid != 0) {
+      if (lo < 0) {
+        const int f = __builtin_ctzll(valid);
+        lo = b + f;
+        bad &= ~((uint64_t{2} << f) - 1);  // blocks after the first
+      }
+      hi = b + 63 - __builtin_clzll(valid);
+    }
+    if (lo >= 0 && stop < 0 && bad != 0) stop = b + __builtin_ctzll(bad);
+  }
+  lo = max(lo, 0);  // no valid key at all: the first block
+  hi = max(hi, 0);
+  if (stop < 0) stop = nb;
+  KeySpan span = {64 * lo, min(end, 64 * (hi + 1)), stop - lo};
+  if (lo == 0 && hi == nb - 1) return span;
+
+  // 16-byte chunks of the rows that drop out: the largest magnitude bits.
+  constexpr int kChunk = 16 / sizeof(St);
+  constexpr int CPR = D / kChunk;
+  constexpr int RPP = kThreads / CPR;  // rows per pass
+  const int col = kChunk * (static_cast<int>(threadIdx.x) % CPR);
+  unsigned top = 0;
+  auto scan_v = [&](int r0, int r1) __attribute__((always_inline)) {
+    for (int r = r0; r < r1; r += 4 * RPP) {
+      u32x4 x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int row = min(r + u * RPP + static_cast<int>(threadIdx.x) / CPR, r1 - 1);
+        x[u] = *reinterpret_cast<const u32x4*>(V + static_cast<int64_t>(row) * vs + col);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (sizeof(St) == 4) {
+            top = max(top, x[u][e] & 0x7fffffffu);
+          } else {
+            typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+            top = __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(us2, top),
+                                                                         __builtin_bit_cast(us2, x[u][e] & 0x7fff7fffu)));
+          }
+        }
+    }
+  };
+  if (span.first > 0) scan_v(0, span.first);
+  if (span.end < end) scan_v(span.end, end);
+  bool odd = sizeof(St) == 4 ? top >= INF : ((top & 0xffffu) >= INF || (top >> 16) >= INF);
+  odd = __builtin_amdgcn_ballot_w64(odd) != 0;
+  if (lane == 0) lds[wave] = odd;
+  __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(lds[0] | lds[1] | lds[2] | lds[3])) span = KeySpan{0, end, 0};
+  return span;
+}
+
 // Waves per SIMD the register budget is sized for: two workgroups per CU,
 // except fp32 head_dim 128, whose live state does not fit 256 registers and
 // runs one workgroup per CU; and 16-bit head_dim <= 64, sized for three (at most 168 VGPRs; the LDS of three workgroups fits).  The 16-bit
 // loop is VALU-issue and latency bound, so the third workgroup pays: left to
 // itself the compiler gave the causal head_dim-64 kernel 176 VGPRs (two
 // workgroups per CU), and capping it at 168 - five registers spilled, reloaded
-// only on the accumulator-rescale path - made config 4's attention 5-7 %
+// only on the accumulator-rescale path - made [4, 2048, 16, 64] 5-7 %
 // faster.
 template <bool F32, int D>
 constexpr int kMinWaves = (D >= 128 && F32) ? 1 : ((!F32 && D <= 64) ? 3 : 2);
@@ -386,7 +496,7 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
   const int prio_phase = (static_cast<int>(blockIdx.x) / max(p.cu_count, 1)) & 1;
   // Folded grid: the heavy workgroup of a CU (the first CU-count workgroups)
   // keeps the high priority throughout and the light one fills its gaps
-  // (0.5 % faster than alternating at config 2, S=512).
+  // (0.5 % faster than alternating at B*H = 128, S=512).
   const bool fold_fixed = p.fold != 0;
   const bool fold_heavy = prio_phase == 0;
   int tiles_done = 0;
@@ -772,7 +882,7 @@ __global__ __launch_bounds__(kThreads, (kMinWaves<true, D>)) void attn_fwd_f32_k
 // bank conflicts): K and Q into the MFMA operand layout (key or query per lane,
 // 4 head dims per register), O back from the accumulator layout.  The MFMA
 // fragments read with a lane stride of a whole row (32 rows x 32 bytes per
-// instruction) cost ~8 % more time at config 5b than whole rows.  V is read
+// instruction) cost ~8 % more time at S = 64 than whole rows.  V is read
 // straight into its operand layout, 256 contiguous bytes per half-wavefront.
 // (fp32 MFMA: the launch is bound by HBM, 4.6 TB/s at [512, 64, 8, 64], so the
 // bf16 matrix cores would not shorten it.)
@@ -1090,6 +1200,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
   constexpr int KBUF = (BN * KS > 64 * (D + 8)) ? BN * KS : 64 * (D + 8);
   __shared__ __attribute__((aligned(16))) unsigned short smK[2][KBUF];
   __shared__ __attribute__((aligned(16))) unsigned short smV[2][BN * VS + C::VSLACK];
+  __shared__ int sm_span[HAS_MASK ? kSpanLds : 1];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1120,9 +1231,9 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
   float lag = 8.0f / c;
   // Both are wave-uniform: kept in SGPRs (a VOP3 instruction reads one SGPR
   // operand), they leave two more VGPRs to the loop.
+  const unsigned short sign = negate ? 0x8000u : 0u;
   c = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(c)));
   lag = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(lag)));
-  const unsigned short sign = negate ? 0x8000u : 0u;
 
   // K: LDS-DMA into padded rows of KCH 16-byte chunks; DMA instruction j
   // fills chunks [64j, 64j + 64) and the instructions are dealt round-robin
@@ -1177,30 +1288,26 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
     const int q0 = qb * kBM + wave * 32;
     const int qrow = q0 + m;
 
-    // B operand of S^T = K.Q^T: k-step g covers d = 16g..16g+15, lane half h
-    // holds d = 16g+8h..16g+8h+7.
-    u16x8 qf[G];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      const int d = 16 * g + 8 * h;
-      if (qrow < S && d < D) {
-        qf[g] = *reinterpret_cast<const u16x8*>(Q + qrow * p.qs + d) ^ sign;
-      } else {
-        qf[g] = u16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
-    }
+    // Keys count from `off` (0 without a key mask): SK of them exist, those
+    // from kv_end on are not visited.  Queries and keys compare as qrow - off.
+    int off = 0, SK = S;
+    int kv_end = CAUSAL ? min(S, (qb + 1) * kBM) : S;
+    int whole = 0;  // 64-key tiles 1 .. whole - 1 have no invalid key
+    auto skip_keys = [&](int n) __attribute__((always_inline)) {
+      off += n;
+      SK -= n;
+      kv_end -= n;
+    };
 
-    const int kv_end = CAUSAL ? min(S, (qb + 1) * kBM) : S;
-    const int ntiles = (kv_end + BN - 1) / BN;
 
     bool rm = false;
     auto dma_k = [&](int buf, int t) __attribute__((always_inline)) {
       if constexpr (HAS_MASK) {
         const int key = t * BN + lane;
-        rm = lane < BN && key < S && M[key * p.ms] != 0;
+        rm = lane < BN && key < SK && M[(off + key) * p.ms] != 0;
       }
-      const St* kt = K + static_cast<int64_t>(t) * BN * p.ks;
-      const bool ragged = (t + 1) * BN > S;
+      const St* kt = K + static_cast<int64_t>(off + t * BN) * p.ks;
+      const bool ragged = (t + 1) * BN > SK;
 #pragma unroll
       for (int i = 0; i < KPW; ++i) {
         const int j = wave + NW * i;
@@ -1209,10 +1316,10 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
           if (!ragged) {
             dma16(kt, koff[i], &smK[buf][512 * j]);
           } else {
-            // Keys past S copy row S-1 (at or after the tile's first key).
+            // Keys past the last copy it (at or after the tile's first key).
             const int row = pos / KCH;
             const int cc = pos - row * KCH;
-            const int rrel = min(t * BN + row, S - 1) - t * BN;
+            const int rrel = min(t * BN + row, SK - 1) - t * BN;
             dma16(kt, 2u * static_cast<unsigned>(rrel * static_cast<int>(p.ks) + 8 * (cc < CPR ? cc : 0)),
                   &smK[buf][512 * j]);
           }
@@ -1225,12 +1332,12 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       if constexpr (HAS_MASK) {
         return __builtin_amdgcn_ballot_w64(rm);
       } else {
-        return range_bits(t * BN, S);
+        return range_bits(t * BN, SK);
       }
     };
     auto dma_v = [&](int buf, int t) __attribute__((always_inline)) {
-      const St* vt = V + static_cast<int64_t>(t) * BN * p.vs;
-      const bool ragged = (t + 1) * BN > S;
+      const St* vt = V + static_cast<int64_t>(off + t * BN) * p.vs;
+      const bool ragged = (t + 1) * BN > SK;
 #pragma unroll
       for (int i = 0; i < VPW; ++i) {
         const int j = wave + NW * i;
@@ -1241,7 +1348,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
           } else {
             const int row = pos / VCH;
             const int cc = pos - row * VCH;
-            const int rrel = min(t * BN + row, S - 1) - t * BN;
+            const int rrel = min(t * BN + row, SK - 1) - t * BN;
             dma16(vt, 2u * static_cast<unsigned>(rrel * static_cast<int>(p.vs) + 8 * (cc ^ vswz(row))),
                   &smV[buf][512 * j]);
           }
@@ -1259,9 +1366,9 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
     auto dma_k_full = [&](int buf, int t) __attribute__((always_inline)) {
       if constexpr (HAS_MASK) {
         const int key = t * BN + lane;
-        rm = lane < BN && M[key * p.ms] != 0;
+        rm = lane < BN && M[(off + key) * p.ms] != 0;
       }
-      const St* kt = K + static_cast<int64_t>(t) * BN * p.ks;
+      const St* kt = K + static_cast<int64_t>(off + t * BN) * p.ks;
 #pragma unroll
       for (int i = 0; i < KPW; ++i) {
         const int j = wave + NW * i;
@@ -1271,7 +1378,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       }
     };
     auto dma_v_full = [&](int buf, int t) __attribute__((always_inline)) {
-      const St* vt = V + static_cast<int64_t>(t) * BN * p.vs;
+      const St* vt = V + static_cast<int64_t>(off + t * BN) * p.vs;
 #pragma unroll
       for (int i = 0; i < VPW; ++i) {
         const int j = wave + NW * i;
@@ -1297,6 +1404,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       return u16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     };
 
+    u16x8 qf[G];
     float m_run = -INFINITY;  // running max of RAW scores
     float m_exp = -INFINITY;  // ceil(m_run * c), kept with m_run
     float l_run = 0.0f;
@@ -1419,7 +1527,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 
     // P.V of the pending tile interleaved with the softmax of s: the first
     // half of the k-steps carries the row max, the second half the exp2 and
-    // conversion (the steady body of key-masked launches).
+    // conversion (the steady body of key-masked tiles).
     auto fused = [&](int buf, f32x16 (&s)[NSB], u16x8 (&pn)[NSB * 2]) __attribute__((always_inline)) {
       constexpr int HALF = NSTEP / 2;
       constexpr int E = NSB * 16;      // score elements per lane
@@ -1472,7 +1580,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       }
       l_run = add_packed<T>(pn, l_run);
     };
-    // Pipelined full tiles (launches without a key mask).  Q.K runs one tile
+    // Pipelined full tiles (no invalid key).  Q.K runs one tile
     // ahead, so each wavefront has matrix-core work beside its softmax VALU
     // work in both halves of a tile (Q.K on its own was the longest stretch
     // of a tile in which the wavefront could issue nothing else):
@@ -1545,16 +1653,50 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
     // of a full tile has finite scores after tile 0).
     auto ref_exp = [&]() __attribute__((always_inline)) -> float { return m_exp; };
 
-    // Key tiles [kt0, kt1) of this workgroup: all of the query tile's, or one
-    // chunk of them on the key-split grid.
-    int kt0 = 0, kt1 = ntiles;
+    // Keys of this workgroup: all of the query tile's, or one chunk of them on
+    // the key-split grid.  The copy of the first tile and the Q loads run under
+    // the mask scan (the copy is repeated if the scan moves the first key).
+    int kt0 = 0, kt1 = (kv_end + BN - 1) / BN;
     if (w.nchunk > 1) {
-      const int csz = (ntiles + w.nchunk - 1) / w.nchunk;
+      const int csz = (kt1 + w.nchunk - 1) / w.nchunk;
       kt0 = w.chunk * csz;
-      kt1 = min(ntiles, kt0 + csz);
+      kt1 = min(kt1, kt0 + csz);
+      if constexpr (HAS_MASK) {
+        kv_end = min(kv_end, kt1 * BN);
+        skip_keys(kt0 * BN);
+        kt1 -= kt0;
+        kt0 = 0;
+      }
+    }
+    dma_k(kt0 & 1, kt0);
+    // B operand of S^T = K.Q^T: k-step g covers d = 16g..16g+15, lane half h
+    // holds d = 16g+8h..16g+8h+7.
+    // Without branches, and not used before the scan: rows past S and the zero
+    // padding of head_dim 8 load other values and are cleared below.
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      qf[g] = *reinterpret_cast<const u16x8*>(Q + min(qrow, S - 1) * p.qs + min(16 * g + 8 * h, D - 8));
+    }
+    if constexpr (HAS_MASK) {
+      if (kv_end > kSpanKeys && p.ms == 1) {
+        const KeySpan span = scan_keys<St, std::is_same<T, BF16>::value ? 0x7f80u : 0x7c00u, D>(
+            M + off, V + off * p.vs, p.vs, kv_end, sm_span);
+        kv_end = __builtin_amdgcn_readfirstlane(span.end);
+        whole = __builtin_amdgcn_readfirstlane(span.full);
+        if (span.first > 0) {
+          skip_keys(__builtin_amdgcn_readfirstlane(span.first));
+          vm_wait();
+          dma_k(0, 0);
+        }
+        kt1 = (kv_end + BN - 1) / BN;
+      }
     }
 
-    dma_k(kt0 & 1, kt0);
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const bool real = qrow < S && 16 * g + 8 * h < D;
+      qf[g] = real ? qf[g] ^ sign : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
     vm_wait();
     uint64_t kvalid = key_bits(kt0);
     __syncthreads();
@@ -1565,7 +1707,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
     // tail use the generic body.  Every path executes one barrier per tile,
     // so all wavefronts meet kt1 - kt0 barriers.
     const int n_full = q0 >= S ? 0
-                               : min(kt1, min(S / BN, CAUSAL ? (q0 + 1) / BN : ntiles));
+                               : min(kt1, min(SK / BN, CAUSAL ? max(0, q0 + 1 - off) / BN : kt1));
     bool pending = false;  // a tile's P.V is still to be accumulated (uniform)
     int pend_live = 0;     // its number of live sub-blocks
 
@@ -1582,12 +1724,12 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       if (t + 1 < kt1) dma_k(kb ^ 1, t + 1);
       dma_v(kb, t);
       const int k0 = t * BN;
-      const bool live = q0 < S && (!CAUSAL || k0 <= q0 + 31);
+      const bool live = q0 < S && (!CAUSAL || k0 <= q0 + 31 - off);
       int nlive = NSB;
 #pragma unroll
       for (int sb = NSB - 1; sb >= 0; --sb) {
         const int ks = k0 + sb * 32;
-        if (ks >= S || (CAUSAL && ks > q0 + 31)) nlive = sb;
+        if (ks >= SK || (CAUSAL && ks > q0 + 31 - off)) nlive = sb;
       }
       if (pending) with_live(pend_live, [&](auto lt) __attribute__((always_inline)) { pv(kb ^ 1, lt); });
       if (live) {
@@ -1600,7 +1742,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
         with_live(nlive, [&](auto lt) __attribute__((always_inline)) {
           f32x16 s[NSB];
           qk(lt, kb, s);
-          apply_mask<NSB, CAUSAL, true, decltype(lt)::value>(s, k0, kvalid, qrow, h);
+          apply_mask<NSB, CAUSAL, true, decltype(lt)::value>(s, k0, kvalid, qrow - off, h);
           softmax(std::true_type{}, lt, s, pn);
         });
 #pragma unroll
@@ -1612,29 +1754,9 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
     };
 
     generic_tile(kt0);
-    if constexpr (HAS_MASK || BNK == 32) {
-      // Key-masked launches keep one score buffer (the second one of the
-      // pipelined body costs them an occupancy step at head_dim 64 and
-      // spills at 128, which outweighs the overlap), and so do 32-key tiles,
-      // whose three workgroups per CU leave no room for it.
-      for (int t = kt0 + 1; t < n_full; ++t) {
-        const int kb = t & 1;
-        if (t + 1 < n_full) {
-          dma_k_full(kb ^ 1, t + 1);
-        } else if (t + 1 < kt1) {
-          dma_k(kb ^ 1, t + 1);
-        }
-        dma_v_full(kb, t);
-        f32x16 s[NSB];
-        u16x8 pn[NSB * 2];
-        qk(kAllLive, kb, s);
-        if constexpr (HAS_MASK) apply_mask<NSB, false>(s, t * BN, kvalid, qrow, h);
-        fused(kb ^ 1, s, pn);
-#pragma unroll
-        for (int i = 0; i < NSB * 2; ++i) pk[i] = pn[i];
-        finish_tile(t);
-      }
-    } else if (n_full - kt0 >= 2) {
+    constexpr bool kPipe = BNK == 64 && (!HAS_MASK || D >= 64);
+    const int n_pipe = HAS_MASK ? min(n_full, whole) : n_full;
+    if constexpr (kPipe) if (n_pipe - kt0 >= 2) {
       // Every interval between two barriers copies and reads the same buffers
       // as the generic tile of that index (K(tau+1), V(tau) in; K(tau),
       // V(tau-1) read), so wavefronts on different paths stay in step.
@@ -1642,7 +1764,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       f32x16 sa[NSB], sb[NSB];
       const int t1 = kt0 + 1;
       // Tile t1: S(t1) with nothing to overlap, then P.V(kt0) with its row max.
-      if (t1 + 1 < n_full) {
+      if (t1 + 1 < n_pipe) {
         dma_k_full((t1 + 1) & 1, t1 + 1);
       } else if (t1 + 1 < kt1) {
         dma_k((t1 + 1) & 1, t1 + 1);
@@ -1651,17 +1773,17 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       qk(kAllLive, t1 & 1, sa);
       phase_b(std::false_type{}, kt0 & 1, sa, [](int) {});
       finish_tile(t1);
-      // Tile t + 1 for t = t1 .. n_full - 2.
+      // Tile t + 1 for t = t1 .. n_pipe - 2.
       auto steady = [&](int t, const f32x16 (&cur)[NSB], f32x16 (&nxt)[NSB])
           __attribute__((always_inline)) {
         const int kb = t & 1;
         // The copies of K(t+2) and V(t+1) are spread over the MFMA groups of
         // both phases instead of issued back to back at the top of the tile.
         static_assert(KPW <= G && 2 * VPW - 1 <= NSTEP, "a copy slot for every copy");
-        const bool kfull = t + 2 < n_full;
+        const bool kfull = t + 2 < n_pipe;
         if (!kfull && t + 2 < kt1) dma_k(kb, t + 2);
-        const St* kt = K + static_cast<int64_t>(t + 2) * BN * p.ks;
-        const St* vt = V + static_cast<int64_t>(t + 1) * BN * p.vs;
+        const St* kt = K + static_cast<int64_t>(off + (t + 2) * BN) * p.ks;
+        const St* vt = V + static_cast<int64_t>(off + (t + 1) * BN) * p.vs;
         phase_a(kb ^ 1, nxt, cur, ref_exp(), [&](int g) __attribute__((always_inline)) {
           if (g < KPW) {
             const int j = wave + NW * g;
@@ -1678,15 +1800,15 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
         finish_tile(t + 1);
       };
       int t = t1;
-      for (; t + 2 < n_full; t += 2) {
+      for (; t + 2 < n_pipe; t += 2) {
         steady(t, sa, sb);
         steady(t + 1, sb, sa);
       }
-      if (t + 1 < n_full) {
+      if (t + 1 < n_pipe) {
         steady(t, sa, sb);
         ++t;
       }
-      // Tile n_full - 1: its P becomes the pending P.V of the next tile.
+      // Tile n_pipe - 1: its P becomes the pending P.V of the next tile.
       const float mc = ref_exp();
       auto last_p = [&](const f32x16 (&cur)[NSB]) __attribute__((always_inline)) {
 #pragma unroll
@@ -1703,6 +1825,30 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
       l_run = add_packed<T>(pk, l_run);
       pending = true;
       pend_live = NSB;
+    }
+    if constexpr (HAS_MASK || BNK == 32) {
+      // The rest of a key-masked launch - scattered invalid keys, or head dims
+      // below 64, where the pipelined body costs an occupancy step (bf16
+      // [8, 1024, 16, 32] with scattered keys 45 -> 51 us) - and 32-key tiles,
+      // whose three workgroups per CU leave no room for it, keep one score
+      // buffer.
+      for (int t = kPipe ? max(kt0 + 1, n_pipe) : kt0 + 1; t < n_full; ++t) {
+        const int kb = t & 1;
+        if (t + 1 < n_full) {
+          dma_k_full(kb ^ 1, t + 1);
+        } else if (t + 1 < kt1) {
+          dma_k(kb ^ 1, t + 1);
+        }
+        dma_v_full(kb, t);
+        f32x16 s[NSB];
+        u16x8 pn[NSB * 2];
+        qk(kAllLive, kb, s);
+        if (HAS_MASK && kvalid != range_bits(0, BN)) apply_mask<NSB, false>(s, t * BN, kvalid, qrow, h);
+        fused(kb ^ 1, s, pn);
+#pragma unroll
+        for (int i = 0; i < NSB * 2; ++i) pk[i] = pn[i];
+        finish_tile(t);
+      }
     }
     for (int t = max(kt0 + 1, n_full); t < kt1; ++t) generic_tile(t);
     if (pending) with_live(pend_live, [&](auto lt) __attribute__((always_inline)) { pv((kt1 - 1) & 1, lt); });
@@ -1856,7 +2002,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 // at 2.0 GHz.  Against the fp32 MFMA kernel: causal [8, 1024, 16, 64] 157 ->
 // 113 us (152 TFLOP/s), [8, 4096, 16, 64] 2181 -> 1440 us (191), [8, 1024,
 // 16, 128] 376 -> 243 us, [8, 1024, 16, 32] 94 -> 69 us; non-causal key-masked
-// [3, 777, 12, 128] 132 -> 82 us.  Error against float64 at those shapes:
+// [3, 777, 12, 128] 132 -> 82 us (67 with scan_keys).  Error against float64 at those shapes:
 // 0.65-0.8 of the fp32 MFMA kernel's.
 //
 // A row with a non-finite operand in reach (or one that rounds to infinity)
@@ -1888,6 +2034,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
   using St = unsigned short;
   __shared__ __attribute__((aligned(16))) St smK[2][3 * KPL];
   __shared__ __attribute__((aligned(16))) St smV[3][3 * VPL];
+  __shared__ int sm_span[HAS_MASK ? kSpanLds : 1];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1900,9 +2047,11 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
   const int hh = w.bh - b * p.H;
   const int S = p.S;
   const float* __restrict__ Q = static_cast<const float*>(p.q) + b * p.qb + hh * p.qh;
-  const float* __restrict__ K = static_cast<const float*>(p.k) + b * p.kb + hh * p.kh;
-  const float* __restrict__ V = static_cast<const float*>(p.v) + b * p.vb + hh * p.vh;
-  const uint8_t* __restrict__ M = HAS_MASK ? p.mask + b * p.mb : nullptr;
+  const float* K = static_cast<const float*>(p.k) + b * p.kb + hh * p.kh;
+  const float* V = static_cast<const float*>(p.v) + b * p.vb + hh * p.vh;
+  const uint8_t* M = HAS_MASK ? p.mask + b * p.mb : nullptr;
+  // Keys count from `off` (0 without a key mask), SK of them exist.
+  int off = 0, SK = S;
 
   // Staging: chunk i of a thread is 4 values of row `srow + i * 256 / CPR`.
   constexpr int RPI = kThreads / CPR;  // rows per staging pass
@@ -1919,7 +2068,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
     voff[i] = (static_cast<unsigned>(srow + RPI * i) * static_cast<unsigned>(p.vs) + 4u * sc) * 4u;
   }
   auto tile_rsrc = [&](const float* base, int64_t rs, int t) __attribute__((always_inline)) {
-    const int rows = min(S - t * BN, BN);
+    const int rows = min(SK - t * BN, BN);
     const unsigned bytes = rows > 0 ? (static_cast<unsigned>(rows - 1) * static_cast<unsigned>(rs) + D) * 4u : 0u;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (rows > 0 ? static_cast<int64_t>(t) * BN * rs : 0)),
                                              static_cast<short>(0), static_cast<int>(bytes), 0x00020000);
@@ -1960,21 +2109,36 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
     const int qb = pass == 0 ? w.q_first : w.q_second;
     const int q0 = qb * kBM + wave * 32;
     const int qrow = q0 + m;
-    const int kv_end = CAUSAL ? min(S, (qb + 1) * kBM) : S;
+    int kv_end = CAUSAL ? min(S, (qb + 1) * kBM) : S;
+    if constexpr (HAS_MASK) {
+      K -= static_cast<int64_t>(off) * p.ks;
+      V -= static_cast<int64_t>(off) * p.vs;
+      M -= static_cast<int64_t>(off) * p.ms;
+      off = 0;
+      if (kv_end > kSpanKeys && p.ms == 1) {
+        const KeySpan span = scan_keys<float, 0x7f800000u, D>(M, V, p.vs, kv_end, sm_span);
+        off = span.first;
+        kv_end = span.end - off;
+        K += static_cast<int64_t>(off) * p.ks;
+        V += static_cast<int64_t>(off) * p.vs;
+        M += static_cast<int64_t>(off) * p.ms;
+      }
+      SK = S - off;
+    }
     const int ntiles = (kv_end + BN - 1) / BN;
     // Tiles with keys for this wavefront.
-    const int nlive = q0 >= S ? 0 : (CAUSAL ? min(ntiles, (q0 + 31) / BN + 1) : ntiles);
+    const int nlive = q0 >= S ? 0 : (CAUSAL ? min(ntiles, (max(-BN, q0 + 31 - off) + BN) / BN) : ntiles);
 
     bool rm = false;
     auto load_mask = [&](int t) __attribute__((always_inline)) {
       if constexpr (HAS_MASK) {
         const int key = t * BN + m;
-        rm = h == 0 && key < S && M[key * p.ms] != 0;
+        rm = h == 0 && key < SK && M[key * p.ms] != 0;
       }
     };
     auto key_bits = [&](int t) __attribute__((always_inline)) -> uint64_t {
       if constexpr (HAS_MASK) return __builtin_amdgcn_ballot_w64(rm);
-      return range_bits(t * BN, S);
+      return range_bits(t * BN, SK);
     };
 
     // Prologue: K(0) into its buffer, K(1) and V(0) into registers.
@@ -2124,12 +2288,13 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       if (t + 1 < ntiles) kvalid = key_bits(t + 1);
       __syncthreads();
       if (live) {
-        const bool need_mask = HAS_MASK || k0 + BN > S || (CAUSAL && k0 + BN - 1 > q0);
+        const bool need_mask = (HAS_MASK && static_cast<uint32_t>(kv) != ~0u) || k0 + BN > SK ||
+                               (CAUSAL && k0 + BN - 1 > q0 - off);
         constexpr int N0 = NDB >= 2 ? 4 : 2;  // MFMAs before the exponentials
 #pragma unroll
         for (int n = 0; n < N0; ++n) pv_mfma(vb, n);
         fence();
-        if (need_mask) apply_mask<1, CAUSAL>(s, k0, kv, qrow, h);
+        if (need_mask) apply_mask<1, CAUSAL>(s, k0, kv, qrow - off, h);
         float mt = s[0][0];
 #pragma unroll
         for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[0][r]);
@@ -2221,17 +2386,17 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
 #pragma unroll 1
     for (int t = 0; t < nlive; ++t) {
       const int k0 = t * BN;
-      const float* kp = K + static_cast<int64_t>(min(k0 + m, S - 1)) * p.ks + h;
+      const float* kp = K + static_cast<int64_t>(min(k0 + m, SK - 1)) * p.ks + h;
       const float* qp = Q + static_cast<int64_t>(min(qrow, S - 1)) * p.qs + h;
       f32x16 s[1];
       s[0] = f32x16{};
 #pragma unroll 1
       for (int d = 0; d < D; d += 2) s[0] = mfma_f32(kp[d], qp[d] * p.scale_log2, s[0]);
-      uint64_t valid = range_bits(k0, S);
+      uint64_t valid = range_bits(k0, SK);
       if constexpr (HAS_MASK) {
-        valid = __builtin_amdgcn_ballot_w64(h == 0 && k0 + m < S && M[(k0 + m) * p.ms] != 0);
+        valid = __builtin_amdgcn_ballot_w64(h == 0 && k0 + m < SK && M[(k0 + m) * p.ms] != 0);
       }
-      apply_mask<1, CAUSAL>(s, k0, valid, qrow, h);
+      apply_mask<1, CAUSAL>(s, k0, valid, qrow - off, h);
       float mt = s[0][0];
 #pragma unroll
       for (int r = 0; r < 16; ++r) mt = fmaxf(mt, s[0][r]);
@@ -2252,9 +2417,9 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int key = k0 + acc_row(r, h);
-        const float* vp = V + static_cast<int64_t>(min(key, S - 1)) * p.vs + m;
+        const float* vp = V + static_cast<int64_t>(min(key, SK - 1)) * p.vs + m;
 #pragma unroll
-        for (int i = 0; i < NDB; ++i) acc[i] = mfma_f32(key < S ? vp[32 * i] : 0.0f, s[0][r], acc[i]);
+        for (int i = 0; i < NDB; ++i) acc[i] = mfma_f32(key < SK ? vp[32 * i] : 0.0f, s[0][r], acc[i]);
       }
     }
     store(sum_with_other_half(l_run));
@@ -2306,7 +2471,7 @@ SplitPlan plan_key_split(int dtype, int D, bool causal, int64_t BH, int64_t S) {
   total *= BH;
   const int64_t limit = std::max<int64_t>(8, (total + slots - 1) / slots);
   // Split only when the heaviest query tile carries over 1.5x the average
-  // load of a workgroup slot.  Measured on the MI355X: config 4's attention
+  // load of a workgroup slot.  Measured on the MI355X: a long-sequence layer
   // (B=4, H=16, S=2048, D=64; 1.41x) ran slower split (62.4 -> 66.6 us: the
   // extra prologues and the state exchange outweigh the shorter tail), as
   // did B=8, H=16, S=1024 (1.33x); B=1, H=4, S=4096 (11.6x) went 51.9 ->
@@ -2383,14 +2548,16 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
   }
   if constexpr ((D == 64 || D == 32) && CAUSAL) {
     // 16-bit head_dim 64 and 32, causal, not key-split: 32-key tiles at four
-    // workgroups per CU up to S = 1024 (head_dim 64 with a key mask: 2048).
+    // workgroups per CU up to S = 1024 (not key-masked head_dim 32, whose
+    // 64-key kernel has four workgroups per CU too).
     // Measured against the 64-key kernel (same box, alternating):
-    // [16, 512, 16, 64] -13 %, [8, 1024, 16, 64] -4.5 %, key-masked fp16
-    // [4, 2048, 16, 64] -2.5 %; config 4 (S = 2048, no mask) +6 %,
-    // [1, 8192, 16, 64] +12 %, non-causal launches 6-9 % slower.  Head dim
-    // 32: [32, 256, 16, 32] -15 %, [16, 512] -15 %, [8, 1024] -4 %, key-masked
-    // fp16 [8, 1024] +2.7 %.
-    const int bn32_max = HAS_MASK ? (D == 64 ? 2048 : 0) : 1024;
+    // [16, 512, 16, 64] -13 %, [8, 1024, 16, 64] -4.5 % (key-masked the same
+    // time), [4, 2048, 16, 64] +6 % (key-masked +10 to +17 %), key-masked
+    // [8, 1500, 16, 64] +4 to +8 %, [1, 8192, 16, 64] +12 %, non-causal
+    // launches 6-9 % slower.  Head dim 32: [32, 256, 16, 32] -15 %, [16, 512]
+    // -15 %, [8, 1024] -4 %; key-masked [8, 1024, 16, 32] +15 %, [4, 700, 8,
+    // 32] +20 %.
+    const int bn32_max = HAS_MASK && D == 32 ? 0 : 1024;
     if (dtype != 0 && !p.split && p.S <= bn32_max) {
       const dim3 g(static_cast<unsigned>(p.units) * static_cast<unsigned>(p.BH)), blk(kThreads);
       if (dtype == 1) {
@@ -2403,14 +2570,14 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
   }
   if constexpr (D == 128) {
     // 16-bit head_dim 128, not key-split: 32-key tiles, three workgroups per
-    // CU, for causal or key-masked launches up to S = 4096 and unmasked
-    // non-causal ones up to 1024.  Measured against the 64-key kernel (same
-    // box, alternating): causal [16, 512, 16, 128] -19 %, [8, 1024, 16, 128]
-    // -9.5 % (key-masked fp16 -19 %), [4, 2048, 16, 128] key-masked fp16
-    // -14 %, [4, 4096, 16, 128] -4 %; non-causal [16, 512, 16, 128] -4 %,
-    // [8, 1024, 16, 128] +0.7 %, [4, 2048, 16, 128] +4.6 % (key-masked fp16
-    // -1 %), [4, 4096, 16, 128] +4.6 %; causal S = 16384 +3.6 %.
-    const int bn32_max = (CAUSAL || HAS_MASK) ? 4096 : 1024;
+    // CU, for causal launches up to S = 4096 and non-causal ones up to 1024.
+    // Measured against the 64-key kernel (same box, alternating): causal
+    // [16, 512, 16, 128] -19 %, [8, 1024, 16, 128] -9.5 %, [4, 4096, 16, 128]
+    // -4 %; non-causal [16, 512, 16, 128] -4 %, [8, 1024, 16, 128] +0.7 %,
+    // [4, 2048, 16, 128] +4.6 % (key-masked +7 to +12 %), [4, 4096, 16, 128]
+    // +4.6 %, key-masked [8, 1200, 16, 128] +7 to +13 %; causal S = 16384
+    // +3.6 %.
+    const int bn32_max = CAUSAL ? 4096 : 1024;
     if (dtype != 0 && !p.split && p.S <= bn32_max) {
       const dim3 g(static_cast<unsigned>(p.units) * static_cast<unsigned>(p.BH)), blk(kThreads);
       if (dtype == 1) {

@@ -263,7 +263,7 @@ class UserOptimizedTransformer(nn.Module):
         self.fused_residual_layer_norm_calls = 0
         # True: in bf16/fp16 models of width 1024, each block's attention
         # output projection and its first residual + LayerNorm run as one HIP
-        # kernel.  Off by default: at config 4 the library GEMM plus the
+        # kernel.  Off by default: at 8192 rows the library GEMM plus the
         # residual + LayerNorm kernel is faster.
         self.fuse_out_projection_norm = False
         # Captures, packed projections and the lock: derived inference state,
