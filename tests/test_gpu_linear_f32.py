@@ -96,14 +96,27 @@ def test_split_weight_declines_what_the_kernel_cannot_take(gpu_ready):
         assert not linear_f32_supported(x, ok, None)
 
 
-def test_split_terms_follow_the_weights_across_streams(gpu_ready):
-    # A weight edited in place is split again, and an eager call on another
-    # stream is ordered after the split.
+def _model(execution_mode, layers=2):
     from transformer_opt.submission import TransformerConfig, UserOptimizedTransformer
 
     torch.manual_seed(5)
-    model = UserOptimizedTransformer(TransformerConfig(2, 96, 128, 4, 256, 2, True), execution_mode="eager")
-    model = model.cuda().eval()
+    model = UserOptimizedTransformer(TransformerConfig(2, 96, 128, 4, 256, layers, True),
+                                     execution_mode=execution_mode)
+    return model.cuda().eval()
+
+
+def _fresh(model, x):
+    """What a model that never saw other weights gives."""
+    fresh = _model("eager")
+    fresh.load_state_dict(model.state_dict())
+    with torch.inference_mode():
+        return fresh(x)
+
+
+def test_edited_weights_are_seen_on_every_stream(gpu_ready):
+    # In-place edits, eager calls on the editing stream and on one ordered
+    # after it.
+    model = _model("eager")
     x = torch.randn(2, 96, 128, device="cuda")
     side = torch.cuda.Stream()
     with torch.inference_mode():
@@ -111,10 +124,8 @@ def test_split_terms_follow_the_weights_across_streams(gpu_ready):
     with torch.no_grad():
         model.layers[0].ffn_out.weight.mul_(-1.0)
         model.layers[1].attention.k_proj.weight.mul_(0.5)
-    fresh = UserOptimizedTransformer(model.config, execution_mode="eager").cuda().eval()
-    fresh.load_state_dict(model.state_dict())
+    expected = _fresh(model, x)
     with torch.inference_mode():
-        expected = fresh(x)
         edited = model(x).clone()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
@@ -122,3 +133,45 @@ def test_split_terms_follow_the_weights_across_streams(gpu_ready):
         torch.cuda.current_stream().wait_stream(side)
     assert torch.equal(edited, expected) and torch.equal(again, expected)
     assert not torch.allclose(first, expected)
+
+
+@pytest.mark.parametrize("execution_mode", ["eager", "auto"])
+@pytest.mark.parametrize("name", ["attention.out_proj", "ffn_in", "ffn_out"])
+def test_writes_that_leave_no_trace_reach_the_projections(gpu_ready, execution_mode, name):
+    # ``.data`` writes change neither the parameter's identity nor its
+    # version: eager calls and replays read the parameter itself.
+    model = _model(execution_mode)
+    x = torch.randn(2, 96, 128, device="cuda")
+    weight = model.get_submodule(f"layers.0.{name}").weight
+    with torch.inference_mode():
+        before = model(x).clone()
+        weight.data.copy_(weight.data.flip(0) * 1.5)
+        after = model(x).clone()
+    assert not torch.allclose(before, after)
+    assert torch.equal(after, _fresh(model, x))
+
+
+def test_a_callers_graph_follows_in_place_edits(gpu_ready):
+    # The caller's own capture after a warm-up: it reads the parameters
+    # themselves and memory that lives as long as the graph.
+    model = _model("eager")
+    x = torch.randn(2, 96, 128, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.inference_mode(False), torch.no_grad():
+        with torch.cuda.stream(side):
+            model(x)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(x)
+        for scale in (-1.0, 0.5, 3.0):
+            model.layers[0].ffn_in.weight.mul_(scale)
+            model.layers[1].ffn_out.weight.mul_(scale)
+            model.layers[1].attention.out_proj.weight.mul_(scale)
+            eager = model(x)
+            # Whatever an edit let go of is somebody else's memory by now.
+            junk = [torch.full((n,), float("nan"), device="cuda") for n in (1 << 12, 1 << 14, 1 << 16, 1 << 18)]
+            graph.replay()
+            assert torch.equal(out, eager) and torch.equal(eager, _fresh(model, x))
+            del junk

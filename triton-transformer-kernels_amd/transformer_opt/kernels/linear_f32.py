@@ -5,12 +5,13 @@ bias)``, or its exact GELU, of fp32 tensors: the projections of the fp32
 encoder (reference transformer_opt/submission.py:484-508).  The products run on
 the bf16 matrix cores, each operand as three bf16 terms that sum to it exactly,
 with an error below that of a plain fp32 GEMM (``ttk_linear_f32_fwd``).
-``split`` is the weight's terms in the order the kernel reads, made once per
-weight by ``split_weight``.
+``split`` is the weight's terms in the order the kernel reads, made by
+``split_weight``: a caller that keeps them owes a new split after every change
+of the weight.
 
-The encoder model uses it (``submission.UserOptimizedTransformer``); where
-``split_weight`` or ``linear_f32_supported`` declines, the model's library
-route runs.
+The encoder model uses it (``submission.UserOptimizedTransformer``) and splits
+in every forward; where ``split_weight`` or ``linear_f32_supported`` declines,
+the model's library route runs.
 """
 
 from __future__ import annotations

@@ -10,8 +10,6 @@ what outlives a call:
 * ``CapturedForward`` - one forward captured as a ``torch.cuda.CUDAGraph``
   (a hipGraph on ROCm) over static input buffers, replayed with fresh inputs
   copied in and a clone of the static output returned;
-* ``SplitWeight`` - a projection weight's bf16 terms for the fp32 linear
-  kernel, under the same rule;
 * ``ReplayCache`` - the captures of one model fingerprint, least recently
   used first, keyed by input geometry, plus the packed projections and the
   lock that serialises capture and replay.
@@ -115,25 +113,6 @@ class PackedOut:
         return self.stamp is not None and self.stamp == PackedQKV.stamp_of((weight,))
 
 
-class SplitWeight:
-    """A projection weight's bf16 terms for the fp32 linear kernel, rebuilt
-    whenever the weight changes (same rule as ``PackedQKV``).  ``terms`` is
-    None when that kernel cannot take the weight."""
-
-    __slots__ = ("sources", "stamp", "terms")
-
-    def __init__(self, weight: torch.Tensor, sources: Sequence[torch.Tensor]):
-        from .kernels.linear_f32 import split_weight
-
-        self.sources = tuple(sources)
-        self.stamp = PackedQKV.stamp_of(self.sources)
-        with torch.no_grad():
-            self.terms = split_weight(weight.detach())
-
-    def serves(self, sources: Sequence[torch.Tensor]) -> bool:
-        return self.stamp is not None and self.stamp == PackedQKV.stamp_of(tuple(sources))
-
-
 _CAPTURE_STREAMS: Dict[int, torch.cuda.Stream] = {}
 _CAPTURE_STREAMS_LOCK = threading.Lock()
 
@@ -229,9 +208,6 @@ class ReplayCache:
         self.last: Optional[CapturedForward] = None
         self.packs: Dict[int, PackedQKV] = {}
         self.out_packs: Dict[int, PackedOut] = {}
-        self.splits: Dict[Hashable, SplitWeight] = {}
-        # The stream the last split ran on and the event after it.
-        self.splits_ready = None
         # The model's module-tree layout and the operands resolved from it,
         # with the (layout epoch, tensor stamps, scalars) key they were
         # resolved under; owned by the model, cached here so copies start
@@ -258,8 +234,6 @@ class ReplayCache:
             self.drop_captures()
             self.packs.clear()
             self.out_packs.clear()
-            self.splits.clear()
-            self.splits_ready = None
             self.layout = None
             self.operands = None
             self.operands_key = None
@@ -277,42 +251,6 @@ class ReplayCache:
             pack = PackedOut(weight)
             self.out_packs[slot] = pack
         return pack
-
-    def split_for(self, slot: Hashable, weight: torch.Tensor,
-                  sources: Sequence[torch.Tensor]) -> Optional[torch.Tensor]:
-        """The bf16 terms of a projection weight (``sources``: the parameters
-        it comes from), or None for the library route: weights that are not
-        fp32 on a ROCm device, that cannot be stamped, or whose terms are not
-        there yet while the caller captures a graph (they would exist only
-        after its first replay)."""
-        if not weight.is_cuda or weight.dtype != torch.float32 or any(t.is_inference() for t in sources):
-            self.splits.pop(slot, None)
-            return None
-        split = self.splits.get(slot)
-        if split is None or not split.serves(sources):
-            if torch.cuda.is_current_stream_capturing():
-                return None
-            split = SplitWeight(weight, sources)
-            self.splits[slot] = split
-            if split.terms is not None:
-                stream = torch.cuda.current_stream(weight.device)
-                event = torch.cuda.Event()
-                event.record(stream)
-                self.splits_ready = (stream, event)
-        return split.terms
-
-    def order_splits(self) -> None:
-        """Orders the current stream after the last split if it ran on another,
-        and keeps the terms' memory for it."""
-        if self.splits_ready is None or torch.cuda.is_current_stream_capturing():
-            return
-        made_on, event = self.splits_ready
-        stream = torch.cuda.current_stream(made_on.device)
-        if stream != made_on:
-            stream.wait_event(event)
-            for split in self.splits.values():
-                if split.terms is not None:
-                    split.terms.record_stream(stream)
 
     def entry(self, fingerprint: Hashable, geometry: Hashable,
               build: Callable[[], CapturedForward]) -> CapturedForward:

@@ -39,13 +39,14 @@ restricted it); graph replay is eligible for every supported shape and dtype
 instead of a measured shape set (submission.py:582-590), with up to
 ``max_cuda_graphs`` captures kept, one per input geometry.  fp32 projections
 run on the HIP kernel that forms them on the bf16 matrix cores from three-term
-splits of both operands (the weights' terms are kept beside the packed QKV
-projection); 16-bit ones, and widths that kernel does not take, are library
-GEMMs (hipBLASLt through ``F.linear``).  In fp32 and bf16 the FFN's input
-projection and exact GELU are one HIP kernel (GELU in the GEMM epilogue),
-otherwise the GELU runs in place on the HIP elementwise kernel.  The model is
-forward-inference only: with gradients enabled on parameters that require
-them the kernels raise, as there is no backward kernel.
+splits of both operands (the weight's terms are made again by every forward,
+so that it follows every write to the weight); 16-bit ones, and widths that
+kernel does not take, are library GEMMs (hipBLASLt through ``F.linear``).  In
+fp32 and bf16 the FFN's input projection and exact GELU are one HIP kernel
+(GELU in the GEMM epilogue), otherwise the GELU runs in place on the HIP
+elementwise kernel.  The model is forward-inference only: with gradients
+enabled on parameters that require them the kernels raise, as there is no
+backward kernel.
 """
 
 from __future__ import annotations
@@ -60,7 +61,7 @@ from .config import ATTENTION_BACKENDS, SUPPORTED_DTYPES
 from .dispatch import attention_forward
 from .kernels.gelu import gelu_
 from .kernels.linear import linear_gelu, linear_supported
-from .kernels.linear_f32 import linear_f32, linear_f32_supported
+from .kernels.linear_f32 import linear_f32, linear_f32_supported, split_weight
 from .kernels.linear_ln import linear_ln_supported, linear_residual_layer_norm
 from .kernels.linear_ln import workspace_bytes as linear_ln_workspace_bytes
 from .kernels.residual_layer_norm import fused_residual_layer_norm, layer_norm
@@ -97,12 +98,6 @@ class _Block(NamedTuple):
     # out_weight packed for the fused projection + residual + LayerNorm
     # kernel, or None when that kernel cannot take it.
     out_packed: Optional[torch.Tensor]
-    # bf16 terms of the fp32 projection weights for the fp32 linear kernel
-    # (None: the library GEMM).
-    qkv_split: Optional[torch.Tensor]
-    out_split: Optional[torch.Tensor]
-    ffn_in_split: Optional[torch.Tensor]
-    ffn_out_split: Optional[torch.Tensor]
 
 
 class _Operands(NamedTuple):
@@ -195,29 +190,40 @@ class _Layout:
             qkv = entry["qkv"]
             pack = cache.pack_for(index, qkv[:3], qkv[3:])
             out_packed = cache.out_pack_for(index, entry["out"][0]).packed if fuse_out else None
-            splits = [cache.split_for((index, "qkv"), pack.weight, qkv[:3])]
-            splits += [cache.split_for((index, name), entry[name][0], entry[name][:1])
-                       for name in ("out", "ffn_in", "ffn_out")]
             blocks.append(_Block(
                 pack.weight, pack.bias, attn.num_heads, attn.head_dim, attn.scale,
                 *entry["out"], _Norm(*entry["norm2"], eps[2 * index + 1]),
-                *entry["ffn_in"], *entry["ffn_out"], exits[index + 1], out_packed, *splits,
+                *entry["ffn_in"], *entry["ffn_out"], exits[index + 1], out_packed,
             ))
         if not fuse_out:
             cache.out_packs.clear()
         keepalive = (self.tensors, tuple(cache.packs.values()),
-                     tuple(p.packed for p in cache.out_packs.values()),
-                     tuple(s.terms for s in cache.splits.values()))
+                     tuple(p.packed for p in cache.out_packs.values()))
         return _Operands(exits[0], tuple(blocks), None, keepalive)
 
 
-def _project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
-             split: Optional[torch.Tensor]) -> torch.Tensor:
-    """``F.linear(x, weight, bias)``: the fp32 kernel on the weight's split
-    terms where it takes the call, else the library GEMM."""
-    if split is not None and linear_f32_supported(x, weight, bias):
-        return linear_f32(x, weight, split, bias)
-    return F.linear(x, weight, bias)
+def _project_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
+                 gelu: bool = False) -> Optional[torch.Tensor]:
+    """``F.linear(x, weight, bias)`` or its exact GELU on the fp32 kernel, or
+    None where that kernel does not take the call.
+
+    The weight's bf16 terms are made by every call, on the call's stream (and
+    inside a capture, into the capture's memory): nothing derived from a
+    parameter outlives the call, so a write to the parameter, in whatever way
+    it is done, is seen by the next forward or replay as the library GEMM
+    would see it.
+    """
+    if not linear_f32_supported(x, weight, bias):
+        return None
+    split = split_weight(weight)
+    return None if split is None else linear_f32(x, weight, split, bias, gelu=gelu)
+
+
+def _project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
+    """``F.linear(x, weight, bias)``: the fp32 kernel where it takes the call,
+    else the library GEMM."""
+    y = _project_f32(x, weight, bias)
+    return F.linear(x, weight, bias) if y is None else y
 
 
 class _ModelTally:
@@ -332,10 +338,7 @@ class UserOptimizedTransformer(nn.Module):
         ops = cache.operands
         if ops is None or stamps is None or cache.operands_key != key:
             ops = layout.resolve(cache, fuse_out)
-            # Operands resolved while the caller captures a graph may lack
-            # weight terms: resolved again by the next call.
-            keep = not (layout.tensors[0].is_cuda and torch.cuda.is_current_stream_capturing())
-            cache.operands, cache.operands_key = (ops, key) if keep else (None, None)
+            cache.operands, cache.operands_key = ops, key
         fingerprint = None
         if stamps is not None and settled:
             fingerprint = key + (self.config, torch.backends.cuda.matmul.allow_tf32)
@@ -377,7 +380,7 @@ class UserOptimizedTransformer(nn.Module):
                                                   workspace=workspace)
                 tally.count_fused_norm()
             else:
-                update = _project(context, block.out_weight, block.out_bias, block.out_split)
+                update = _project(context, block.out_weight, block.out_bias)
                 x, h = self._fused_norm(x, update, norm, mask, tally)
             x, h = self._fused_norm(x, self._feed_forward(block, h), block.exit_norm, mask, tally,
                                     zero_residual=masked, zero_output=masked and index == last)
@@ -387,7 +390,7 @@ class UserOptimizedTransformer(nn.Module):
         """Multi-head attention of one block up to its output projection:
         the context ``[B, S, width]`` that out_proj maps."""
         batch, seq_len, width = h.shape
-        qkv = _project(h, block.qkv_weight, block.qkv_bias, block.qkv_split)
+        qkv = _project(h, block.qkv_weight, block.qkv_bias)
         q, k, v = qkv.view(batch, seq_len, 3, block.num_heads, block.head_dim).unbind(2)
         context, record = attention_forward(q, k, v, mask, causal=self.config.causal,
                                             scale=block.scale, backend=self.attention_backend)
@@ -407,11 +410,11 @@ class UserOptimizedTransformer(nn.Module):
         w, b = block.ffn_in_weight, block.ffn_in_bias
         if h.dtype == torch.bfloat16 and linear_supported(h, w, b) is None:
             inner = linear_gelu(h, w, b)
-        elif block.ffn_in_split is not None and linear_f32_supported(h, w, b):
-            inner = linear_f32(h, w, block.ffn_in_split, b, gelu=True)
         else:
-            inner = gelu_(F.linear(h, w, b))
-        return _project(inner, block.ffn_out_weight, block.ffn_out_bias, block.ffn_out_split)
+            inner = _project_f32(h, w, b, gelu=True)
+            if inner is None:
+                inner = gelu_(F.linear(h, w, b))
+        return _project(inner, block.ffn_out_weight, block.ffn_out_bias)
 
     @staticmethod
     def _fused_norm(x, update, norm: _Norm, mask, tally, *, zero_residual=False,
@@ -431,7 +434,6 @@ class UserOptimizedTransformer(nn.Module):
         # every capture and replay; the eager forward itself runs outside it.
         with self._replay.lock:
             ops = self._operands()
-            self._replay.order_splits()
         return self._encode(ops, x.contiguous(), mask, _ModelTally(self))
 
     def forward(self, x: torch.Tensor, valid_token_mask: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -452,12 +454,11 @@ class UserOptimizedTransformer(nn.Module):
         # The lock orders host-side capture and replay; the capture's event
         # orders its static buffers between caller streams.
         with cache.lock:
-
-            def capture() -> CapturedForward:
-                cache.order_splits()
-                return CapturedForward(lambda xs, ms, t: self._encode(ops, xs, ms, t), x, mask, ops.keepalive)
-
-            captured = cache.entry((ops.fingerprint, self.attention_backend), geometry, capture)
+            captured = cache.entry(
+                (ops.fingerprint, self.attention_backend), geometry,
+                lambda: CapturedForward(lambda xs, ms, t: self._encode(ops, xs, ms, t), x, mask,
+                                        ops.keepalive),
+            )
             result = captured.replay(x, mask)
             for selected, count in captured.tally.attention.items():
                 self.attention_backend_counts[selected] = (
