@@ -323,3 +323,36 @@ def test_replay_of_a_key_split_attention_is_bitwise_eager(gpu_ready):
             assert torch.equal(out, reference), step
     assert model.cuda_graph_replays == 3
     assert model._inference_graph is not None
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
+def test_packs_of_a_callers_capture_stay_with_it(gpu_ready, dtype):
+    """What the caller's capture packs is filled by its replays only: an eager
+    call before the first of them does not see it.  And the capture holds no
+    kept pack: after an edit and an eager call, which replace those, its
+    replays still read memory of their own and follow the edit."""
+    from transformer_opt.submission import UserOptimizedTransformer
+
+    model, eager = twin(dtype=dtype, execution_mode="eager")
+    x = sample(dtype=dtype)
+    with torch.no_grad():
+        if dtype != torch.float32:  # library GEMMs allocate at their first call
+            eager(x)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = model(x)
+        assert not model._packed_qkv_cache
+        assert torch.equal(model(x), eager(x))
+        for scale in (-0.5, 2.0, 1.5):
+            for m in (model, eager):
+                m.layers[0].attention.q_proj.weight.mul_(scale)
+                m.layers[2].attention.v_proj.weight.mul_(scale)
+            again = model(x)
+            junk = [torch.full((n,), float("nan"), dtype=dtype, device="cuda") for n in (1 << 14, 1 << 16, 1 << 18)]
+            graph.replay()
+            # A model that has seen no other weights.
+            fresh = UserOptimizedTransformer(CFG, execution_mode="eager").to("cuda", dtype).eval()
+            fresh.load_state_dict(model.state_dict(), strict=True)
+            expected = fresh(x)
+            assert torch.equal(again, expected) and torch.equal(out, expected)
+            del junk

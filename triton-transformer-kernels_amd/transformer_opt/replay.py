@@ -238,14 +238,23 @@ class ReplayCache:
             self.operands = None
             self.operands_key = None
 
-    def pack_for(self, slot: int, weights, biases) -> PackedQKV:
+    # ``keep=False`` (the caller captures a graph) packs anew, inside that
+    # capture, and leaves the cache alone: the copy runs with every replay, into
+    # memory of the graph's own.  A pack kept from a capture would hold nothing
+    # before its first replay, and a kept pack's address in the caller's graph
+    # would outlive the pack.
+    def pack_for(self, slot: int, weights, biases, keep: bool = True) -> PackedQKV:
+        if not keep:
+            return PackedQKV(weights, biases)
         pack = self.packs.get(slot)
         if pack is None or not pack.serves(weights, biases):
             pack = PackedQKV(weights, biases)
             self.packs[slot] = pack
         return pack
 
-    def out_pack_for(self, slot: int, weight: torch.Tensor) -> PackedOut:
+    def out_pack_for(self, slot: int, weight: torch.Tensor, keep: bool = True) -> PackedOut:
+        if not keep:
+            return PackedOut(weight)
         pack = self.out_packs.get(slot)
         if pack is None or not pack.serves(weight):
             pack = PackedOut(weight)

@@ -178,18 +178,19 @@ class _Layout:
         return (tuple([n.eps for n in self.norms]),
                 tuple([(a.num_heads, a.head_dim, a.d_model, a.scale) for a in self.attentions]))
 
-    def resolve(self, cache: ReplayCache, fuse_out: bool) -> _Operands:
+    def resolve(self, cache: ReplayCache, fuse_out: bool, keep: bool = True) -> _Operands:
         """Operands of every block; the out-projection weights are packed for
         the fused projection + residual + LayerNorm kernel only with
-        ``fuse_out`` (otherwise the packs are dropped)."""
+        ``fuse_out`` (otherwise the packs are dropped).  ``keep``: packs come
+        from and stay in the cache."""
         eps = [n.eps for n in self.norms]
         exits = [_Norm(*entry["norm1"], eps[2 * i]) for i, entry in enumerate(self.layers)]
         exits.append(_Norm(*self.final_norm, eps[-1]))
         blocks = []
         for index, (entry, attn) in enumerate(zip(self.layers, self.attentions)):
             qkv = entry["qkv"]
-            pack = cache.pack_for(index, qkv[:3], qkv[3:])
-            out_packed = cache.out_pack_for(index, entry["out"][0]).packed if fuse_out else None
+            pack = cache.pack_for(index, qkv[:3], qkv[3:], keep)
+            out_packed = cache.out_pack_for(index, entry["out"][0], keep).packed if fuse_out else None
             blocks.append(_Block(
                 pack.weight, pack.bias, attn.num_heads, attn.head_dim, attn.scale,
                 *entry["out"], _Norm(*entry["norm2"], eps[2 * index + 1]),
@@ -336,7 +337,11 @@ class UserOptimizedTransformer(nn.Module):
         fuse_out = bool(self.fuse_out_projection_norm)
         key = (layout.epoch, stamps, scalars, fuse_out)
         ops = cache.operands
-        if ops is None or stamps is None or cache.operands_key != key:
+        # A capture of the caller's gets operands of its own.
+        keep = not (layout.tensors[0].is_cuda and torch.cuda.is_current_stream_capturing())
+        if not keep:
+            ops = layout.resolve(cache, fuse_out, keep)
+        elif ops is None or stamps is None or cache.operands_key != key:
             ops = layout.resolve(cache, fuse_out)
             cache.operands, cache.operands_key = ops, key
         fingerprint = None
