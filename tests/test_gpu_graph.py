@@ -356,3 +356,40 @@ def test_packs_of_a_callers_capture_stay_with_it(gpu_ready, dtype):
             expected = fresh(x)
             assert torch.equal(again, expected) and torch.equal(out, expected)
             del junk
+
+
+@pytest.mark.parametrize("mode", ["eager", "auto"])
+def test_kept_packs_are_ordered_before_calls_on_other_streams(gpu_ready, mode):
+    """The packs are made behind a queue of work on one stream; calls on
+    streams that nothing else orders after it read them whole, and so does a
+    third stream after a single weight was replaced on the second."""
+    model, eager = twin(execution_mode=mode)
+    x = sample()
+    busy = torch.randn(4096, 4096, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    with torch.inference_mode():
+        expected = eager(x)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[0]):
+            for _ in range(40):
+                busy = busy @ busy * 1e-3
+            model._operands()  # the packs, some milliseconds from now
+        with torch.cuda.stream(streams[1]):
+            got = model(x)
+    torch.cuda.synchronize()
+    assert torch.equal(got, expected)
+    for m in (model, eager):
+        attention = m.layers[1].attention
+        attention.k_proj.weight = nn.Parameter(attention.k_proj.weight.detach() * -2.0)
+    torch.cuda.synchronize()
+    with torch.inference_mode():
+        expected = eager(x)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[1]):
+            for _ in range(40):
+                busy = busy @ busy * 1e-3
+            model._operands()
+        with torch.cuda.stream(streams[2]):
+            got = model(x)
+    torch.cuda.synchronize()
+    assert torch.equal(got, expected)

@@ -30,6 +30,8 @@ from typing import Callable, Dict, Hashable, Optional, Sequence
 
 import torch
 
+from ._launch import raw_stream
+
 
 class CallTally:
     """Kernel launches one forward performs, by kind."""
@@ -58,6 +60,33 @@ def tensor_stamp(t: torch.Tensor) -> tuple:
     return (id(t), t.data_ptr(), t._version)
 
 
+class _Made:
+    """Where and when derived tensors were made: the stream of their last
+    write and an event after it."""
+
+    __slots__ = ("tensors", "device", "handle", "event")
+
+    def __init__(self, tensors: Sequence[Optional[torch.Tensor]]):
+        self.tensors = tuple(t for t in tensors if t is not None and t.is_cuda)
+        self.event = None
+        if self.tensors and not torch.cuda.is_current_stream_capturing():
+            self.device = self.tensors[0].device
+            stream = torch.cuda.current_stream(self.device)
+            self.handle = stream.cuda_stream
+            self.event = torch.cuda.Event()
+            self.event.record(stream)
+
+    def use_here(self) -> None:
+        """Orders the current stream after the making, and keeps the memory
+        until work queued on it by the time of the free is done."""
+        if self.event is None or raw_stream(self.device.index) == self.handle:
+            return
+        stream = torch.cuda.current_stream(self.device)
+        stream.wait_event(self.event)
+        for t in self.tensors:
+            t.record_stream(stream)
+
+
 class PackedQKV:
     """``cat(Wq, Wk, Wv)`` and ``cat(bq, bk, bv)`` for one packed projection GEMM.
 
@@ -67,7 +96,7 @@ class PackedQKV:
     so such a pack is never reused.
     """
 
-    __slots__ = ("sources", "stamp", "weight", "bias")
+    __slots__ = ("sources", "stamp", "weight", "bias", "made")
 
     def __init__(self, weights: Sequence[torch.Tensor], biases: Sequence[Optional[torch.Tensor]]):
         filled = [b if b is not None else w.new_zeros(w.shape[0]) for w, b in zip(weights, biases)]
@@ -76,6 +105,7 @@ class PackedQKV:
         with torch.no_grad():
             self.weight = torch.cat(tuple(weights), dim=0).detach()
             self.bias = torch.cat(filled, dim=0).detach()
+        self.made = _Made((self.weight, self.bias))
 
     @staticmethod
     def stamp_of(sources: Sequence[Optional[torch.Tensor]]) -> Optional[tuple]:
@@ -96,7 +126,7 @@ class PackedOut:
     kernel cannot take the weight (not a 16-bit [1024, K] ROCm tensor with K a
     multiple of 128)."""
 
-    __slots__ = ("sources", "stamp", "packed")
+    __slots__ = ("sources", "stamp", "packed", "made")
 
     def __init__(self, weight: torch.Tensor):
         from .kernels.linear_ln import WIDTH, pack_weight
@@ -108,6 +138,7 @@ class PackedOut:
                 and weight.shape[0] == WIDTH and weight.shape[1] % 128 == 0):
             with torch.no_grad():
                 self.packed = pack_weight(weight.detach())
+        self.made = _Made((self.packed,))
 
     def serves(self, weight: torch.Tensor) -> bool:
         return self.stamp is not None and self.stamp == PackedQKV.stamp_of((weight,))
@@ -260,6 +291,14 @@ class ReplayCache:
             pack = PackedOut(weight)
             self.out_packs[slot] = pack
         return pack
+
+    def use_packs_here(self) -> None:
+        """Call with ``lock`` held, before work that reads the kept packs is
+        queued on the current stream (not while it captures: such work has
+        packs of its own)."""
+        for packs in (self.packs, self.out_packs):
+            for pack in packs.values():
+                pack.made.use_here()
 
     def entry(self, fingerprint: Hashable, geometry: Hashable,
               build: Callable[[], CapturedForward]) -> CapturedForward:

@@ -320,7 +320,8 @@ class UserOptimizedTransformer(nn.Module):
         read once and re-checked per call with one identity pass; tensor
         stamps (storage pointer, version) and the scalar settings (eps,
         heads, scale) are re-read per call.  Operands are rebuilt only when
-        one of these moved.
+        one of these moved.  What the packs hold is ordered before the work
+        that the caller queues next on the current stream.
         """
         cache = self._replay
         layout = cache.layout
@@ -344,6 +345,8 @@ class UserOptimizedTransformer(nn.Module):
         elif ops is None or stamps is None or cache.operands_key != key:
             ops = layout.resolve(cache, fuse_out)
             cache.operands, cache.operands_key = ops, key
+        if keep:
+            cache.use_packs_here()
         fingerprint = None
         if stamps is not None and settled:
             fingerprint = key + (self.config, torch.backends.cuda.matmul.allow_tf32)
