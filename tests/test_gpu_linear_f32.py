@@ -96,6 +96,21 @@ def test_split_weight_declines_what_the_kernel_cannot_take(gpu_ready):
         assert not linear_f32_supported(x, ok, None)
 
 
+def test_terms_that_are_not_the_weights_are_refused(gpu_ready):
+    from transformer_opt.kernels.linear_f32 import linear_f32, split_weight
+
+    x, w = torch.zeros(5, 64, device="cuda"), torch.zeros(64, 64, device="cuda")
+    split = split_weight(w)
+    smaller, larger = split_weight(w[:32]), split_weight(torch.zeros(68, 64, device="cuda"))
+    for bad in (smaller, larger, split.cpu(), split.view(torch.float32), split[::2], split[16:], w):
+        with pytest.raises(ValueError, match="split"):
+            linear_f32(x, w, bad, None)
+    for weight in (w.t(), w.bfloat16(), w.double(), w.cpu(), w[0]):
+        with pytest.raises(ValueError, match="unsupported"):
+            linear_f32(x, weight, split, None)
+    assert torch.equal(linear_f32(x, w, split, None), torch.zeros_like(x))
+
+
 def _model(execution_mode, layers=2):
     from transformer_opt.submission import TransformerConfig, UserOptimizedTransformer
 

@@ -61,10 +61,13 @@ def linear_f32_supported(x: torch.Tensor, weight: torch.Tensor, bias: Optional[t
 def linear_f32(x: torch.Tensor, weight: torch.Tensor, split: torch.Tensor, bias: Optional[torch.Tensor],
                gelu: bool = False) -> torch.Tensor:
     """``F.linear(x, weight, bias)``, with ``gelu`` its exact GELU, in one kernel."""
-    if not linear_f32_supported(x, weight, bias):
+    if weight.ndim != 2 or not _float_rows(weight) or not linear_f32_supported(x, weight, bias):
         raise ValueError("unsupported HIP fp32 linear input")
     lib = _native.load()
     n, k = weight.shape
+    if (split.device != weight.device or split.dtype != torch.uint8 or not split.is_contiguous()
+            or split.numel() != lib.ttk_linear_f32_split_bytes(n, k)):
+        raise ValueError("split is not what split_weight gives for a weight of this shape and device")
     y = torch.empty(*x.shape[:-1], n, dtype=x.dtype, device=x.device)
     status = launch(
         x.get_device(), lib.ttk_linear_f32_fwd, x.data_ptr(), weight.data_ptr(), split.data_ptr(),
