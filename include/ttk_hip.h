@@ -261,8 +261,11 @@ ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, 
  * X [M, K] (row stride ldx elements), W [N, K] (row stride ldw) and the same
  * W as split by ttk_linear_f32_split_weight, bias [N] or NULL, Y [M, N] (row
  * stride ldy), all fp32.  Each operand enters as its three bf16 terms and the
- * six products of terms above 2^-22 are accumulated in fp32, the leading ones
- * apart from the rest: the error is below that of an fp32 fma chain over K.
+ * six products with the leading terms are accumulated in fp32, the leading ones
+ * apart from the rest.  What is left out of a product is at most 2^-24 of it
+ * and of either sign.  Against float64 the error (2-norm, N(0, 1) operands) is
+ * 0.2 - 0.4 of an fp32 GEMM's from K = 32 to 4096; rows of X with one nonzero
+ * value, which an fp32 GEMM rounds once, come within 1.03 of its error.
  * A result that is not finite is recomputed from the fp32 operands.
  *
  * Requirements (TTK_EUNSUPPORTED otherwise): K a multiple of 32 below 2^22, N

@@ -49,6 +49,22 @@ def test_error_against_float64(gpu_ready, seq_len, head_dim, causal, masked):
     assert bool(((out.double() - exact).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("seq_len", [128, 1024])
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+def test_no_pull_towards_zero(gpu_ready, seq_len, head_dim):
+    # All products of P.V positive: what is left out of them has either sign,
+    # so the mean error stays below half a unit in the last place (2^-24).
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (torch.randn(4, seq_len, 4, head_dim, device="cuda", generator=g) for _ in range(3))
+    v = v.abs() + 0.5
+    with torch.inference_mode():
+        out = hip_attention(q, k, v, causal=False)
+        exact, _ = _exact(q, k, v, None, False, head_dim ** -0.5)
+    assert abs((out.double() / exact - 1.0).mean().item()) <= 2.0 ** -24
+
+
 def test_rows_that_overlap_and_broadcast(gpu_ready):
     from transformer_opt.kernels import hip_attention
 

@@ -44,7 +44,7 @@ def test_linear_f32_against_float64(gpu_ready, rows, out_features, in_features, 
         if bias:
             exact, scale = exact + b.double(), scale + b.double().abs()
         err = (y.double() - exact).abs()
-        # Products left out: 3 * 2^-22 of |x||w|; two roundings per 16 values
+        # Products left out: 2^-24 of |x||w|; two roundings per 16 values
         # of K and sum, and a few at the end.
         assert bool((err <= (2.0 * in_features / 16 + 24) * 2.0 ** -24 * scale).all())
         # No less accurate than the library's fp32 GEMM (2-norm).
@@ -54,6 +54,22 @@ def test_linear_f32_against_float64(gpu_ready, rows, out_features, in_features, 
         torch.testing.assert_close(z, gelu(y), rtol=1e-6, atol=1e-7)
         # The same call gives the same bits.
         assert torch.equal(linear_f32(x, w, split, b), y)
+
+
+@pytest.mark.parametrize("rows,out_features,in_features", [(128, 256, 64), (2048, 512, 512), (8192, 4096, 1024)])
+def test_a_single_product_is_rounded_about_once(gpu_ready, rows, out_features, in_features):
+    # Rows with one nonzero value: 2^-24 of the product left out, 2^-24 in the
+    # last addition, and the small products' own roundings (2^-8 of that each).
+    from transformer_opt.kernels.linear_f32 import linear_f32, split_weight
+
+    x, w, _ = _inputs(rows, out_features, in_features, 11)
+    at = torch.arange(rows, device="cuda")
+    one = torch.zeros_like(x)
+    one[at, at % in_features] = x[at, at % in_features]
+    with torch.inference_mode():
+        y = linear_f32(one, w, split_weight(w), None).double()
+        exact = torch.matmul(one.double(), w.double().t().contiguous())
+    assert bool(((y - exact).abs() <= (2.0 + 2.0 ** -5) * 2.0 ** -24 * exact.abs()).all())
 
 
 @pytest.mark.parametrize("rows,out_features,in_features", [(40, 64, 64), (2048, 512, 512), (4096, 1024, 1024)])

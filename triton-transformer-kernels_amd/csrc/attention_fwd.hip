@@ -77,8 +77,8 @@
 // * Output: the 16-bit kernel stages each wavefront's 32 x D tile in LDS so
 //   that each store covers whole rows; fp32 stores straight from registers.
 //
-// fp32 path: fp32 products, exact to 2^-22 of each where they are formed from
-// bf16 terms, fp32 accumulate.  Q is pre-multiplied by scale*log2(e) so scores
+// fp32 path: fp32 products, exact to 2^-24 of each where they are formed from
+// bf16 terms (bf16x3.h), fp32 accumulate.  Q is pre-multiplied by scale*log2(e) so scores
 // are already in the exp2 domain.  bf16/fp16 path: v_mfma_f32_32x32x16_{bf16,f16}; scores stay fp32,
 // the row max is taken on raw scores and the scale is folded into one fma per
 // element before exp2; P is rounded to the input type (v_cvt_pk_bf16_f32 /
@@ -1979,8 +1979,7 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 // kernel ran at up to 0.79 of its peak.  Here every operand - scaled Q, K, V
 // and the probabilities - is the sum of three bf16 terms (bf16x3.h) and each
 // product the six products of terms that matter, 16/6 of the fp32 MFMA's rate
-// at best.  Q's terms are rounded to nearest and K's, V's and P's truncated;
-// small products are accumulated before the leading ones of a Q.K, so its sum
+// at best.  Small products are accumulated before the leading ones of a Q.K, so its sum
 // is rounded D / 16 times.
 //
 // One workgroup = 4 wavefronts x 32 queries; 32-key tiles.  A tile's K and V
@@ -2158,10 +2157,10 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
         a = *reinterpret_cast<const f32x4*>(Q + qrow * p.qs + 16 * g + 8 * h) * p.scale_log2;
         c = *reinterpret_cast<const f32x4*>(Q + qrow * p.qs + 16 * g + 8 * h + 4) * p.scale_log2;
       }
-      split_pair_rn(qf[g], 0, a[0], a[1]);
-      split_pair_rn(qf[g], 1, a[2], a[3]);
-      split_pair_rn(qf[g], 2, c[0], c[1]);
-      split_pair_rn(qf[g], 3, c[2], c[3]);
+      split_pair(qf[g], 0, a[0], a[1]);
+      split_pair(qf[g], 1, a[2], a[3]);
+      split_pair(qf[g], 2, c[0], c[1]);
+      split_pair(qf[g], 3, c[2], c[3]);
     }
     {
       const auto k1 = tile_rsrc(K, p.ks, 1), v0 = tile_rsrc(V, p.vs, 0);

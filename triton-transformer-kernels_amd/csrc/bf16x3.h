@@ -1,10 +1,21 @@
-// fp32 values as three bf16 terms, for fp32 products on the bf16 matrix cores.
+// fp32 values as three bf16 terms, for fp32 products on the bf16 matrix cores
+// (the splitting of Henry, Tang and Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", ARITH
+// 2019).
 //
 // A float's 24 significant bits are the sum of three bf16 numbers exactly
-// (8 + 8 + 8 bits; values below 2^-110 may lose their last bits).  Products of
-// bf16 pairs are exact in fp32, so a product of two fp32 values is the sum of
-// nine exact ones; the six with the leading terms are kept (terms 0.0, 0.1,
-// 1.0, 1.1, 0.2, 2.0), the other three are below 2^-22 of the product.
+// (8 + 8 + 8 bits; values below 2^-110 may lose their last bits).  Every term
+// is rounded to nearest, so the second is at most 2^-8 and the third at most
+// 2^-17 of the value, both of either sign.  Products of bf16 pairs are exact in
+// fp32, so a product of two fp32 values is the sum of nine exact ones; the six
+// with the leading terms are kept (terms 0.0, 0.1, 1.0, 1.1, 0.2, 2.0).  The
+// other three (1.2, 2.1, 2.2) come to at most 2^-24 + 2^-34 of the product, of
+// random sign.  Terms cut off instead would all have the value's sign: the
+// products left out come to 2^-22, and where both operands are cut off, they
+// pull every sum towards zero: attention over 1024 keys with positive V had a
+// mean error of -3.1e-7 (rms 5.8e-7; the fp32 MFMA's 4.7e-7), and has -3e-8
+// (3.4e-7) as rounded.  Either split takes 11 VALU operations a pair; the
+// conversions cost 2 - 4 % of the attention kernels, nothing of the linear ones.
 // Infinities, NaN and values that round to infinity leave NaN in a sum of such
 // products: callers recompute non-finite results from the fp32 operands.
 #pragma once
@@ -31,16 +42,23 @@ __device__ __forceinline__ float high_half(float a) {
 __device__ __forceinline__ unsigned pack_high(float a, float b) {
   return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
 }
-// The three terms of the pair (a, b), by truncation: 11 VALU operations.
+// The three terms of the pair (a, b): 11 VALU operations.
 // (v_dot2_f32_bf16 would subtract a term in one instruction but holds up the
 // matrix pipe: beside four simple VALU operations an MFMA took 14.6 ns, beside
 // four dot2 28 ns.)
 __device__ __forceinline__ void split_pair(float a, float b, unsigned& t0, unsigned& t1, unsigned& t2) {
-  const float a1 = a - high_half(a), b1 = b - high_half(b);
-  const float a2 = a1 - high_half(a1), b2 = b1 - high_half(b1);
-  t0 = pack_high(a, b);
-  t1 = pack_high(a1, b1);
-  t2 = pack_high(a2, b2);
+  auto round = [](float& u, float& v) __attribute__((always_inline)) -> unsigned {
+    const x3bf16x2 r = {static_cast<__bf16>(u), static_cast<__bf16>(v)};
+    unsigned bits = __builtin_bit_cast(unsigned, r);
+    asm("" : "+v"(bits));  // one conversion of the pair, not another of its lower half
+    u -= __uint_as_float(bits << 16);
+    v -= high_half(__uint_as_float(bits));
+    return bits;
+  };
+  t0 = round(a, b);
+  t1 = round(a, b);
+  const x3bf16x2 r = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
+  t2 = __builtin_bit_cast(unsigned, r);
   // Opaque here, so that the split stays where it is written: between the
   // MFMAs before the ones that use it.
   asm volatile("" : "+v"(t2));
@@ -52,16 +70,4 @@ __device__ __forceinline__ void split_pair(Split8& s, int d, float a, float b) {
   s.t[1][d] = t1;
   s.t[2][d] = t2;
 }
-// The same with every term rounded to nearest: the terms' signs are then
-// independent of the value's, and so are those of the products left out.
-__device__ __forceinline__ void split_pair_rn(Split8& s, int d, float a, float b) {
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const x3bf16x2 r = {static_cast<__bf16>(a), static_cast<__bf16>(b)};
-    s.t[i][d] = __builtin_bit_cast(unsigned, r);
-    a -= static_cast<float>(r.x);
-    b -= static_cast<float>(r.y);
-  }
-}
-
 }  // namespace ttk

@@ -11,8 +11,8 @@
 // each operand is written as the sum of three bf16 numbers, which is exact
 // (8 + 8 + 8 significant bits), and the product is formed from the six
 // products of terms that matter: x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0 (the
-// three left out are below 2^-22 of |x w|, and of random sign: W's terms are
-// rounded to nearest).  Products of bf16 pairs are exact in fp32, and the
+// three left out come to at most 2^-24 of |x w|, of random sign: see
+// bf16x3.h).  Products of bf16 pairs are exact in fp32, and the
 // leading products and the five small ones have an fp32 accumulator each, so
 // the leading sum is rounded K / 16 times instead of K / 2 times by the fp32
 // MFMA.  Relative error against float64 (2-norm): 1.8e-7 at K = 1024 and
@@ -27,10 +27,8 @@
 //
 // W is split once (launch_split_weight), in MFMA fragment order: 6 bytes a
 // weight, one contiguous 1 KB copy per fragment, no work on it in the main
-// loop.  X is split in registers: truncation, 5.5 VALU operations per value
-// in the shadow of the MFMAs (v_dot2_f32_bf16, which would subtract a term in
-// one instruction, holds up the matrix pipe: a probe measured 14.6 ns per
-// MFMA with four other VALU operations beside it and 28 ns with four dot2).
+// loop.  X is split in registers: 5.5 VALU operations per value, in the shadow
+// of the MFMAs.
 //
 // Tiled kernel (one workgroup = 4 wavefronts, two workgroups per CU; a 128 x
 // 128 tile): a wavefront owns 32 tokens x 128 features, as C^T = W . X^T with
@@ -523,8 +521,7 @@ hipError_t launch_tiled(LinearF32Params& p, bool gelu, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// W [N, K] fp32 into its three bf16 terms (round to nearest even at every
-// step, so the terms' signs are independent), in MFMA fragment order: 16-byte
+// W [N, K] fp32 into its three bf16 terms, in MFMA fragment order: 16-byte
 // chunk ((fb * K/16 + q) * 3 + t) * 64 + l holds term t of
 // W[32 fb + l % 32][16 q + 8 (l / 32) .. + 7]; rows past N are zero.
 __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4* wp, int N, int K, int64_t ldw) {
@@ -544,7 +541,7 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4
     }
     Split8 t;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) split_pair_rn(t, d, v[d >> 1][2 * (d & 1)], v[d >> 1][2 * (d & 1) + 1]);
+    for (int d = 0; d < 4; ++d) split_pair(t, d, v[d >> 1][2 * (d & 1)], v[d >> 1][2 * (d & 1) + 1]);
 #pragma unroll
     for (int i = 0; i < 3; ++i) wp[(frag * 3 + i) * 64 + l] = t.t[i];
   }
