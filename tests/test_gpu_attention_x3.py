@@ -65,6 +65,37 @@ def test_no_pull_towards_zero(gpu_ready, seq_len, head_dim):
     assert abs((out.double() / exact - 1.0).mean().item()) <= 2.0 ** -24
 
 
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+def test_scores_of_one_product_are_rounded_about_once(gpu_ready, head_dim):
+    # Scores up to 220 in exp2 units from one product each, neighbours close
+    # enough to share a row's weight: the error is the score's rounding.  As
+    # much of it as products that are rounded once give, 8 % for the 2^-24 of
+    # each that is left out, and 2^-24 for the sums.
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(head_dim)
+    seq, scale = 512, head_dim ** -0.5
+    at = torch.arange(seq, device="cuda").float()[None, :, None]
+    got = rounded = 0.0
+    for column in range(4):
+        q, k = torch.zeros(2, 1, seq, 4, head_dim, device="cuda")
+        q[..., column] = 1.0 + 0.1 * torch.rand(1, seq, 4, device="cuda", generator=g)
+        k[..., column] = 0.3 / scale * at * (1.0 + 1e-3 * torch.rand(1, seq, 4, device="cuda", generator=g))
+        v = torch.randn(1, seq, 4, head_dim, device="cuda", generator=g)
+        with torch.inference_mode():
+            exact, _ = _exact(q, k, v, None, True, scale)
+            out = hip_attention(q, k, v, causal=True)
+            s = (q[..., column] * (scale * math.log2(math.e))).permute(0, 2, 1)[..., None] \
+                * k[..., column].permute(0, 2, 1)[:, :, None]
+            s = s.double().masked_fill(torch.ones(seq, seq, dtype=torch.bool, device="cuda").triu(1), -math.inf)
+            weights = torch.softmax(s * math.log(2.0), -1)
+            plain = torch.matmul(weights, v.double().permute(0, 2, 1, 3).contiguous()).permute(0, 2, 1, 3)
+        got += ((out.double() - exact).norm() / exact.norm()).item()
+        rounded += ((plain - exact).norm() / exact.norm()).item()
+    print(f"head_dim {head_dim}: {got / 4:.3e}, rounded products {rounded / 4:.3e}")
+    assert got <= 1.08 * rounded + 4 * 2.0 ** -24
+
+
 def test_rows_that_overlap_and_broadcast(gpu_ready):
     from transformer_opt.kernels import hip_attention
 

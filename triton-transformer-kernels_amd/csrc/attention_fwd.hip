@@ -1979,8 +1979,12 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 // kernel ran at up to 0.79 of its peak.  Here every operand - scaled Q, K, V
 // and the probabilities - is the sum of three bf16 terms (bf16x3.h) and each
 // product the six products of terms that matter, 16/6 of the fp32 MFMA's rate
-// at best.  Small products are accumulated before the leading ones of a Q.K, so its sum
-// is rounded D / 16 times.
+// at best.  The small and the leading products of a Q.K have an accumulator
+// each, so its sum is rounded D / 16 times, and once more where a VALU addition
+// joins the two.  (Leading products accumulated onto the small ones lose more
+// than a rounding in the matrix core's alignment: scores of one product each,
+// rising to 220 over 512 keys, gave 1.2 - 1.35 times the error of rounded
+// products, 1.02 - 1.05 in two sums.  The additions cost no measurable time.)
 //
 // One workgroup = 4 wavefronts x 32 queries; 32-key tiles.  A tile's K and V
 // rows are loaded into registers a tile ahead (16 bytes a lane, through a
@@ -2249,8 +2253,10 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       const bool live = t < nlive;
       f32x16 s[1];
       if (live) {
-        // The small products of every k-step first, then the leading ones.
+        // The small products of every k-step first, then the leading ones, in
+        // a sum of their own.
         s[0] = f32x16{};
+        f32x16 hi;
         constexpr int NQK = 6 * G;
         constexpr int kQT[5] = {0, 1, 0, 2, 1};
 #pragma unroll
@@ -2260,7 +2266,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
             s[0] = mfma_x3(pr == 0 ? kr[g & 1][0] : (pr < 3 ? kr[g & 1][1] : k0f[g]), qf[g].t[kQT[pr]], s[0]);
             if (pr == 0 && g + 1 < G) k_frag(kb, g + 1);
           } else {
-            s[0] = mfma_x3(k0f[n - 5 * G], qf[n - 5 * G].t[0], s[0]);
+            hi = mfma_x3(k0f[n - 5 * G], qf[n - 5 * G].t[0], n == 5 * G ? f32x16{} : hi);
           }
           // 2 CPT chunks over 6 G = 12 CPT MFMAs: one per six.
           if (n % 6 == 1) stage(n / 6, 0);
@@ -2270,6 +2276,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
           if (n == NQK - 2) v_frag(vb, 1);
           fence();
         }
+        s[0] += hi;
       } else {
 #pragma unroll
         for (int c = 0; c < 2 * CPT; ++c) {
