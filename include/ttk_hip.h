@@ -266,7 +266,8 @@ ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, 
  * and of either sign.  Against float64 the error (2-norm, N(0, 1) operands) is
  * 0.2 - 0.4 of an fp32 GEMM's from K = 32 to 4096; rows of X with one nonzero
  * value, which an fp32 GEMM rounds once, come within 1.03 of its error.
- * A result that is not finite is recomputed from the fp32 operands.
+ * A result that is not finite, or not zero and below 2^-80 in magnitude, is
+ * recomputed from the fp32 operands.
  *
  * Requirements (TTK_EUNSUPPORTED otherwise): K a multiple of 32 below 2^22, N
  * a multiple of 4; x, w, w_split, bias and y 16-byte aligned; ldx, ldw and

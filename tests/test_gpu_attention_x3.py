@@ -96,6 +96,34 @@ def test_scores_of_one_product_are_rounded_about_once(gpu_ready, head_dim):
     assert got <= 1.08 * rounded + 4 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("exponent", [-90, -118])
+@pytest.mark.parametrize("head_dim", [32, 64, 128])
+def test_values_below_the_range_of_three_terms(gpu_ready, head_dim, exponent):
+    # Values too small for three bf16 terms, and ordinary ones under weights as
+    # small (every other value zero): the results of plain fp32 arithmetic.
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(head_dim)
+    q, k, v = (torch.randn(2, 150, 3, head_dim, device="cuda", generator=g) for _ in range(3))
+    with torch.inference_mode():
+        out = hip_attention(q, k, v * 2.0 ** exponent, causal=True).double()
+        exact, spread = _exact(q, k, v * 2.0 ** exponent, None, True, head_dim ** -0.5)
+    bound = (8 + 4 + 150 / 32) * 2.0 ** -23 * spread + 2.0 ** -146
+    assert bool(((out - exact).abs() <= bound).all())
+    # Scores in exp2 units: -exponent at key 3, whose value is zero; 0 at the
+    # others.
+    q, k = torch.zeros(2, 2, 150, 3, head_dim, device="cuda")
+    q[..., 0] = 1.0
+    k[:, 3, :, 0] = -exponent * math.log(2.0)
+    v[:, 3] = 0.0
+    with torch.inference_mode():
+        out = hip_attention(q, k, v, scale=1.0, causal=False).double()
+        exact, spread = _exact(q, k, v, None, False, 1.0)
+    # The score is -exponent in magnitude: its rounding moves a weight by 2^-17.
+    bound = (2.0 ** -17 + 150 / 2 * 2.0 ** -24) * spread + 2.0 ** -146
+    assert bool(((out - exact).abs() <= bound).all())
+
+
 def test_rows_that_overlap_and_broadcast(gpu_ready):
     from transformer_opt.kernels import hip_attention
 

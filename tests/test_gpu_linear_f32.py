@@ -72,6 +72,27 @@ def test_a_single_product_is_rounded_about_once(gpu_ready, rows, out_features, i
     assert bool(((y - exact).abs() <= (2.0 + 2.0 ** -5) * 2.0 ** -24 * exact.abs()).all())
 
 
+@pytest.mark.parametrize("exponent", [-90, -118, -124])
+@pytest.mark.parametrize("rows,out_features,in_features", [(40, 64, 64), (2048, 512, 512), (4096, 1024, 1024)])
+def test_operands_below_the_range_of_three_terms(gpu_ready, rows, out_features, in_features, exponent):
+    # Below 2^-110 a value loses bits as three bf16 terms: rows of such values
+    # (the others stay ordinary) and weights, the results plain fp32's.
+    from transformer_opt.kernels.linear_f32 import linear_f32, split_weight
+
+    x, w, _ = _inputs(rows, out_features, in_features, 17)
+    x[::3] *= 2.0 ** exponent
+    w[1::5] *= 2.0 ** -20
+    x[1] = 0.0
+    for a, b in ((x, w), (x[2::3].contiguous(), w * 2.0 ** exponent)):
+        with torch.inference_mode():
+            y = linear_f32(a, b, split_weight(b), None).double()
+            exact = torch.matmul(a.double(), b.double().t().contiguous())
+            scale = torch.matmul(a.double().abs(), b.double().abs().t().contiguous())
+        # A sum of K rounded products, and the spacing of subnormal numbers.
+        bound = (in_features / 2 + 2) * 2.0 ** -24 * scale + in_features * 2.0 ** -149
+        assert bool(((y - exact).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("rows,out_features,in_features", [(40, 64, 64), (2048, 512, 512), (4096, 1024, 1024)])
 def test_non_finite_results_are_those_of_the_fp32_operands(gpu_ready, rows, out_features, in_features):
     from transformer_opt.kernels.linear_f32 import linear_f32, split_weight

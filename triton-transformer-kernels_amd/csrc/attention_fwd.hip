@@ -2009,9 +2009,9 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 // 0.65-0.8 of the fp32 MFMA kernel's.
 //
 // A row with a non-finite operand in reach (or one that rounds to infinity)
-// comes out non-finite; its wavefront then computes its 32 rows again on the
-// fp32 MFMA straight from global memory, which gives what plain fp32
-// arithmetic gives.
+// comes out non-finite, and one of values too small for three terms below
+// 2^-80; its wavefront then computes its 32 rows again on the fp32 MFMA
+// straight from global memory, which gives what plain fp32 arithmetic gives.
 template <int D>
 struct X3Cfg {
   static constexpr int BN = 32;              // keys per tile
@@ -2373,17 +2373,25 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       }
     };
     const float lt = sum_with_other_half(l_run);
-    float bad = lt * 0.0f;
+    RedoWatch watch;
+    watch.see(lt);
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bad = __builtin_fmaf(acc[db][r], 0.0f, bad);
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) == 0, 1)) {
+      for (int r = 0; r < 16; ++r) watch.see(acc[db][r]);
+    bool redo = watch.any();
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) != 0, 0)) {
+      redo = redo_x3(lt);
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) redo |= redo_x3(acc[db][r]);
+    }
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) == 0, 1)) {
       store(lt);
       continue;
     }
-    // Non-finite operands (or results): these rows again on the fp32 MFMA,
-    // straight from global memory.
+    // These rows again on the fp32 MFMA, straight from global memory.
     if (q0 >= S) continue;
     m_run = -INFINITY;
     l_run = 0.0f;

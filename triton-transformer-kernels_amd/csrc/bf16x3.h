@@ -17,7 +17,8 @@
 // (3.4e-7) as rounded.  Either split takes 11 VALU operations a pair; the
 // conversions cost 2 - 4 % of the attention kernels, nothing of the linear ones.
 // Infinities, NaN and values that round to infinity leave NaN in a sum of such
-// products: callers recompute non-finite results from the fp32 operands.
+// products, and values below 2^-110 fewer bits: callers recompute results that
+// are not finite, or nonzero and below 2^-80, from the fp32 operands (redo_x3).
 #pragma once
 
 #include "ttk_common.h"
@@ -70,4 +71,25 @@ __device__ __forceinline__ void split_pair(Split8& s, int d, float a, float b) {
   s.t[1][d] = t1;
   s.t[2][d] = t2;
 }
+// Whether a result has to be formed again from the fp32 operands.  Bits that a
+// value below 2^-110 loses are at most 2^-134 in magnitude: 2^-54 of a result
+// of 2^-80 times the other operand, which keeps fp32 accuracy up to operands of
+// 2^28.
+constexpr float kRedoBelow = 0x1p-80f;
+__device__ __forceinline__ bool redo_x3(float v) {
+  return !(v * 0.0f == 0.0f) || (v != 0.0f && __builtin_fabsf(v) < kRedoBelow);
+}
+// A first look over many results, 1.5 VALU operations each: without `any()`
+// none is to be formed again.  Zeros, which are not but count here, are told
+// apart by redo_x3.
+struct RedoWatch {
+  float bad = 0.0f;         // NaN once a value was not finite
+  float least = INFINITY;   // smallest magnitude
+  __device__ __forceinline__ void see(float v) {
+    bad = __builtin_fmaf(v, 0.0f, bad);
+    least = __builtin_fminf(least, __builtin_fabsf(v));
+  }
+  __device__ __forceinline__ bool any() const { return !(bad == 0.0f) || least < kRedoBelow; }
+};
+
 }  // namespace ttk

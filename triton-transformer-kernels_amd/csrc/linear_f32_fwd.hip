@@ -21,9 +21,10 @@
 // limit holds bf16 MFMAs to about 1.85 PFLOP/s, i.e. 308.
 //
 // What a bf16 split cannot carry - infinities, values that round to infinity,
-// NaN - makes the sum NaN or infinite, so every non-finite result is
-// recomputed from the fp32 operands (fp32 MFMA or fma): those results are
-// what a plain fp32 product gives.
+// NaN - makes the sum NaN or infinite, and values below 2^-110, which lose
+// bits, matter in results as small only: every result that is not finite, or
+// not zero and below 2^-80, is recomputed from the fp32 operands (fp32 MFMA or
+// fma), which gives what a plain fp32 product gives.
 //
 // W is split once (launch_split_weight), in MFMA fragment order: 6 bytes a
 // weight, one contiguous 1 KB copy per fragment, no work on it in the main
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
         lo[i] = mfma_x3(terms, ones, lo[i]);
       }
     }
-    float bad = 0.0f;
+    RedoWatch watch;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -293,12 +294,18 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           v[e] = hi[i][4 * g + e] + lo[i][4 * g + e];
-          bad = __builtin_fmaf(v[e], 0.0f, bad);
+          watch.see(v[e]);
         }
         put(i, g, v);
         __builtin_amdgcn_sched_barrier(0);
       }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(bad == 0.0f)) != 0, 0)) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(watch.any()) == 0, 1)) return;
+    bool redo = false;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) redo |= redo_x3(hi[i][e] + lo[i][e]);
+    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
       fl_vm_wait<0>();
 #pragma unroll 1
       for (int i = 0; i < TN; ++i) {
@@ -454,9 +461,11 @@ __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_
     f32x4 v = part[0][c][lane];
 #pragma unroll
     for (int s = 1; s < NW; ++s) v += part[s][c][lane];
-    const float bad = __builtin_fmaf(v[0], 0.0f, v[1] * 0.0f) + __builtin_fmaf(v[2], 0.0f, v[3] * 0.0f);
+    bool redo = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) redo |= redo_x3(v[e]);
     if (m >= p.M || f >= p.N) continue;
-    if (__builtin_expect(!(bad == 0.0f), 0)) {
+    if (__builtin_expect(redo, 0)) {
       const float* xr = p.x + static_cast<int64_t>(m) * p.ldx;
 #pragma unroll 1
       for (int e = 0; e < 4; ++e) {
