@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define TTK_ABI_VERSION 10
+#define TTK_ABI_VERSION 11
 
 /* Bytes of the arrival-counter block that leads every attention workspace
  * (and the library's static scratch): the same for every launch shape. */
@@ -248,7 +248,8 @@ int64_t ttk_linear_f32_split_bytes(int64_t N, int64_t K);
  * W[32 fb + l % 32][16 q + 8 (l / 32) .. + 7], rows past N zero.
  * Requirements (TTK_EUNSUPPORTED otherwise): K a multiple of 32 below 2^22, w
  * and w_split 16-byte aligned, ldw a multiple of 4 and >= K; w_split must not
- * overlap w (TTK_EINVAL).  A weight that does not change is split once.
+ * overlap w (TTK_EINVAL).  A weight that does not change may be split once:
+ * whoever keeps the terms makes them again after every change of W.
  */
 ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, int64_t K, int64_t ldw,
                                        void* stream);
@@ -275,12 +276,34 @@ ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, 
  * M and N below 2^31.  y must not overlap an input (TTK_EINVAL).  M == 0 is a
  * no-op.
  *
+ * Small products read W alone.
+ *
  * Replaces the fp32 library GEMMs of the encoder's projections and the GELU
  * pass after the FFN input (reference transformer_opt/submission.py:484-508).
  */
 ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split, const void* bias, void* y,
                               int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy,
                               int activation, void* stream);
+
+/*
+ * Workspace bytes of ttk_linear_f32_fwd_ws: ttk_linear_f32_split_bytes(N, K)
+ * where the call makes W's terms first, 0 for small products (which read W
+ * alone) and for sizes it does not take.  Asked for with the device of the
+ * launch current.
+ */
+int64_t ttk_linear_f32_workspace_size(int64_t M, int64_t N, int64_t K);
+
+/*
+ * ttk_linear_f32_fwd that reads W as it is at the time of the launch: its
+ * terms, where the product wants them, are made by the call in `workspace`
+ * (workspace_bytes >= ttk_linear_f32_workspace_size(M, N, K), 16-byte aligned,
+ * apart from every other argument; TTK_EINVAL otherwise), whose contents
+ * before the call do not matter.  workspace may be NULL where that size is 0.
+ * Nothing is kept between calls.
+ */
+ttk_status ttk_linear_f32_fwd_ws(const void* x, const void* w, const void* bias, void* y, int64_t M, int64_t N,
+                                 int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, int activation, void* workspace,
+                                 int64_t workspace_bytes, void* stream);
 
 /* Bytes of the counter block that leads every ttk_linear_residual_ln_fwd
  * workspace: the same for every M (one counter per 64 rows of the largest M

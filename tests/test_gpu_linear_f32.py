@@ -56,6 +56,36 @@ def test_linear_f32_against_float64(gpu_ready, rows, out_features, in_features, 
         assert torch.equal(linear_f32(x, w, split, b), y)
 
 
+@pytest.mark.parametrize("rows,out_features,in_features", SHAPES + [(16, 1024, 4096), (8192, 768, 256)])
+@pytest.mark.parametrize("gelu", [False, True], ids=["linear", "gelu"])
+def test_terms_made_by_the_call(gpu_ready, rows, out_features, in_features, gelu):
+    # Small products split W in registers, the tiled kernel reads terms made
+    # beforehand: the same terms, so the same bits where both take one form.
+    from transformer_opt.kernels import gelu as exact_gelu
+    from transformer_opt.kernels.linear_f32 import linear_f32, split_weight
+
+    x, w, b = _inputs(rows, out_features, in_features, rows + out_features)
+    with torch.inference_mode():
+        split = split_weight(w)
+        y = linear_f32(x, w, None, b, gelu=gelu)
+        exact = torch.addmm(b.double(), x.double(), w.double().t().contiguous())
+        scale = torch.matmul(x.double().abs(), w.double().abs().t().contiguous()) + b.double().abs()
+        bound = (2.0 * in_features / 16 + 24) * 2.0 ** -24 * scale
+        given = linear_f32(x, w, split, b, gelu=gelu)
+        if not gelu:
+            assert bool(((y.double() - exact).abs() <= bound).all())
+            assert bool(((y - given).double().abs() <= 2 * bound).all())
+        else:
+            torch.testing.assert_close(y, exact_gelu(linear_f32(x, w, None, b)), rtol=1e-6, atol=1e-7)
+        if in_features <= 96 or rows >= 32768:
+            assert torch.equal(y, given)
+        # Following the weight: no terms are left over.  (The same bound: the
+        # matrix core's sums are not the same bits with every sign turned.)
+        w.mul_(-1.0)
+        again = linear_f32(x, w, None, -b)
+        assert bool(((again.double() + exact).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("rows,out_features,in_features", [(128, 256, 64), (2048, 512, 512), (8192, 4096, 1024)])
 def test_a_single_product_is_rounded_about_once(gpu_ready, rows, out_features, in_features):
     # Rows with one nonzero value: 2^-24 of the product left out, 2^-24 in the

@@ -51,6 +51,34 @@ def test_split_weight_arguments_and_sizes():
     assert split(1 << 20, 2 << 20, 64, 64, 32, None) == _native.TTK_EUNSUPPORTED
 
 
+def test_workspace_arguments():
+    lib = _native.load()
+    size, split_bytes = lib.ttk_linear_f32_workspace_size, lib.ttk_linear_f32_split_bytes
+    assert size(32, 64, 64) == size(256, 1024, 256) == 0  # small products read W alone
+    assert size(8192, 4096, 1024) == split_bytes(4096, 1024)
+    assert size(0, 64, 64) == size(-1, 64, 64) == size(1 << 31, 64, 64) == size(64, 64, 1 << 22) == 0
+
+    def call(**over):
+        m, n, k = 8192, 4096, 1024
+        a = dict(x=1 << 30, w=2 << 30, b=None, y=3 << 30, M=m, N=n, K=k, ws=4 << 30, bytes=split_bytes(n, k))
+        a.update(over)
+        return lib.ttk_linear_f32_fwd_ws(a["x"], a["w"], a["b"], a["y"], a["M"], a["N"], a["K"], a["K"], a["K"], a["N"],
+                                         _native.TTK_ACT_NONE, a["ws"], a["bytes"], None)
+
+    for over, status, message in (
+        (dict(ws=None), _native.TTK_EINVAL, "NULL"),
+        (dict(bytes=split_bytes(4096, 1024) - 1), _native.TTK_EINVAL, "must hold"),
+        (dict(ws=(4 << 30) + 8), _native.TTK_EUNSUPPORTED, "16-byte aligned"),
+        (dict(ws=(2 << 30) + 16), _native.TTK_EINVAL, "overlaps w"),
+        (dict(ws=(1 << 30) + 16), _native.TTK_EINVAL, "overlaps an input"),
+        (dict(b=(4 << 30) + 32), _native.TTK_EINVAL, "overlaps an input"),
+        (dict(y=(4 << 30) + 32), _native.TTK_EINVAL, "y overlaps"),
+        (dict(M=0), _native.TTK_OK, ""),
+    ):
+        assert call(**over) == status
+        assert message in _native.last_error()
+
+
 def test_m0_is_only_written_by_the_inline_copies(tmp_path):
     in_asm, inside, outside = False, 0, 0
     for line in _assembly(CSRC / "linear_f32_fwd.hip", tmp_path).splitlines():

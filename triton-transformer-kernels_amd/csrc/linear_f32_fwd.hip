@@ -26,9 +26,9 @@
 // not zero and below 2^-80, is recomputed from the fp32 operands (fp32 MFMA or
 // fma), which gives what a plain fp32 product gives.
 //
-// W is split once (launch_split_weight), in MFMA fragment order: 6 bytes a
-// weight, one contiguous 1 KB copy per fragment, no work on it in the main
-// loop.  X is split in registers: 5.5 VALU operations per value, in the shadow
+// For the tiled kernel W is split by a launch of its own (launch_split_weight),
+// in MFMA fragment order: 6 bytes a weight, one contiguous 1 KB copy per
+// fragment, no work on it in the main loop.  X is split in registers: 5.5 VALU operations per value, in the shadow
 // of the MFMAs.
 //
 // Tiled kernel (one workgroup = 4 wavefronts, two workgroups per CU; a 128 x
@@ -378,9 +378,14 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
 }
 
 // Small products: one workgroup of four wavefronts per TB*32 x TB*32 tile, the
-// wavefronts splitting K.  Fragments come straight from global memory (W as
-// packed, X as two 16-byte halves of a row's 8 values); the wavefronts' sums
-// are added in order through LDS.
+// wavefronts splitting K.  Fragments come straight from global memory, X and W
+// alike as two 16-byte halves of a row's 8 values, and are split in registers:
+// no terms of W have to be made first.  The wavefronts' sums are added in order
+// through LDS.
+// Against the same kernel on terms made beforehand 0.8 us more at K = 256 (256
+// x 768: 4.1 -> 4.9 us) and up to 35 % where the full chip runs (64 x 1024 x
+// 4096 22 -> 30 us, 1024 x 1024 x 1024 18 -> 21 us); making the terms is a
+// launch of 2.4 us for 256 x 256 weights, 7.5 us for 1024 x 4096.
 template <int TB, bool GELU, bool BIAS>
 __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_kernel(LinearF32Params p) {
   constexpr int NW = kFlThreads / 64;
@@ -394,12 +399,11 @@ __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_
   const int KQ = p.K / 16;
   const int q0 = KQ * wave / NW, q1 = KQ * (wave + 1) / NW;
   const float* xrow[TB];
-  const u32x4* wf[TB];
+  const float* wrow[TB];
 #pragma unroll
   for (int b = 0; b < TB; ++b) {
     xrow[b] = p.x + static_cast<int64_t>(min(m0 + 32 * b + r32, p.M - 1)) * p.ldx + 8 * h;
-    wf[b] = static_cast<const u32x4*>(p.wp) +
-            static_cast<int64_t>(min((n0 >> 5) + b, (p.N - 1) >> 5)) * KQ * 192 + lane;
+    wrow[b] = p.w + static_cast<int64_t>(min(n0 + 32 * b + r32, p.N - 1)) * p.ldw + 8 * h;
   }
   f32x16 hi[TB][TB], lo[TB][TB];
 #pragma unroll
@@ -408,28 +412,30 @@ __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_
     for (int j = 0; j < TB; ++j) hi[i][j] = lo[i][j] = f32x16{};
   constexpr int UN = TB == 1 ? 4 : 2;  // k-steps whose loads are in flight together
   for (int q = q0; q < q1; q += UN) {
-    f32x4 rx[UN][TB][2];
-    Split8 w[UN][TB];
+    f32x4 rx[UN][TB][2], rw[UN][TB][2];
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       const int qq = min(q + u, q1 - 1);
 #pragma unroll
       for (int b = 0; b < TB; ++b) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) rx[u][b][j] = *reinterpret_cast<const f32x4*>(xrow[b] + 16 * qq + 4 * j);
-#pragma unroll
-        for (int t = 0; t < 3; ++t) w[u][b].t[t] = wf[b][(qq * 3 + t) * 64];
+        for (int j = 0; j < 2; ++j) {
+          rx[u][b][j] = *reinterpret_cast<const f32x4*>(xrow[b] + 16 * qq + 4 * j);
+          rw[u][b][j] = *reinterpret_cast<const f32x4*>(wrow[b] + 16 * qq + 4 * j);
+        }
       }
     }
 #pragma unroll
     for (int u = 0; u < UN; ++u) {
       if (q + u < q1) {
-        Split8 x[TB];
+        Split8 x[TB], w[TB];
 #pragma unroll
         for (int b = 0; b < TB; ++b)
 #pragma unroll
-          for (int d = 0; d < 4; ++d)
+          for (int d = 0; d < 4; ++d) {
             split_pair(x[b], d, rx[u][b][d >> 1][2 * (d & 1)], rx[u][b][d >> 1][2 * (d & 1) + 1]);
+            split_pair(w[b], d, rw[u][b][d >> 1][2 * (d & 1)], rw[u][b][d >> 1][2 * (d & 1) + 1]);
+          }
 #pragma unroll
         for (int pr = 0; pr < 6; ++pr)
 #pragma unroll
@@ -437,7 +443,7 @@ __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_
 #pragma unroll
             for (int i = 0; i < TB; ++i) {
               f32x16& c = pr == 2 ? hi[i][j] : lo[i][j];
-              c = mfma_x3(w[u][i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
+              c = mfma_x3(w[i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
             }
       }
     }
@@ -558,21 +564,32 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4
 
 }  // namespace
 
-hipError_t launch_linear_f32(LinearF32Params& p, bool gelu, hipStream_t stream) {
+LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, bool terms_ready) {
   // The form with the least expected time (us) on 256 CUs, from the measured
-  // times of the three over products from 100 x 132 x 64 to 32768 x 2048 x
+  // times of the three over products from 16 x 3072 x 1024 to 32768 x 2048 x
   // 512: a launch's fixed cost, then the longest chain of k-steps or the rate
-  // at which the full chip runs, whichever lasts longer.  E.g. 256 x 256 x
-  // 256: 3.7 us for 32 x 32 tiles, 6.6 for 64 x 64, 13.4 for 128 x 128; 2048
-  // x 512 x 512: 14.5, 11.6, 22.2; 4096 x 1024 x 1024: 93, 56, 49.
-  const double flops = 2.0 * p.M * p.N * p.K;
-  const double rounds = std::ceil(std::ceil(p.M / 128.0) * std::ceil(p.N / 128.0) / 256.0);
-  const double t32 = 3.2 + std::max(flops / 105e6, p.K / 256.0);
-  const double t64 = 4.0 + std::max(flops / 150e6, p.K / 102.0);
-  const double t128 = 5.0 + p.K / kFlBK * 1.37 * rounds;
-  if (t32 <= t64 && t32 <= t128) return launch_small<1>(p, gelu, stream);
-  if (t64 <= t128) return launch_small<2>(p, gelu, stream);
-  return launch_tiled(p, gelu, stream);
+  // at which the full chip runs, whichever lasts longer; for the tiled form
+  // also the launch that makes W's terms, unless they are there.  E.g. 256 x
+  // 256 x 256: 4.7 us for 32 x 32 tiles, 8.8 for 64 x 64, 15.3 for 128 x 128;
+  // 2048 x 512 x 512: 18.8, 13.8, 23.9; 4096 x 1024 x 1024: 117, 71, 50.
+  const double flops = 2.0 * static_cast<double>(M) * N * K;
+  const double tiles = std::ceil(M / 128.0) * std::ceil(N / 128.0);
+  const double rounds = std::ceil(tiles / 256.0);
+  const double t32 = 3.2 + std::max(flops / 74e6, K / 160.0);
+  const double t64 = 4.5 + std::max(flops / 112e6, K / 73.0);
+  double t128 = 5.0 + static_cast<double>(K / kFlBK) * (rounds > 1.0 ? 1.37 * rounds : 0.85 + 0.52 * tiles / 256.0);
+  if (!terms_ready) t128 += 3.0 + static_cast<double>(N) * K / 0.6e6;
+  if (t32 <= t64 && t32 <= t128) return LinearF32Form::kTiles32;
+  return t64 <= t128 ? LinearF32Form::kTiles64 : LinearF32Form::kTiles128;
+}
+
+hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream) {
+  switch (form) {
+    case LinearF32Form::kTiles32: return launch_small<1>(p, gelu, stream);
+    case LinearF32Form::kTiles64: return launch_small<2>(p, gelu, stream);
+    case LinearF32Form::kTiles128: return launch_tiled(p, gelu, stream);
+  }
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_split_weight(const float* w, void* wp, int N, int K, int64_t ldw, hipStream_t stream) {

@@ -453,55 +453,68 @@ extern "C" int64_t ttk_linear_f32_split_bytes(int64_t N, int64_t K) {
   return (N + 31) / 32 * 32 * K * 6;
 }
 
+extern "C" int64_t ttk_linear_f32_workspace_size(int64_t M, int64_t N, int64_t K) {
+  const int64_t bytes = ttk_linear_f32_split_bytes(N, K);
+  if (M <= 0 || M >= (int64_t{1} << 31) || bytes == 0) return 0;
+  return ttk::linear_f32_form(M, N, K, false) == ttk::LinearF32Form::kTiles128 ? bytes : 0;
+}
+
 namespace {
 
-// What both fp32 linear entry points ask of W.
-ttk_status check_linear_f32_weight(const char* what, const void* w, const void* w_split, int64_t N, int64_t K,
-                                   int64_t ldw) {
+// What the fp32 linear entry points ask of W.
+ttk_status check_linear_f32_weight(const char* what, const void* w, int64_t N, int64_t K, int64_t ldw) {
   if (N <= 0 || K <= 0) {
     return fail(TTK_EINVAL, "%s: N and K must be positive (N=%lld K=%lld)", what, (long long)N, (long long)K);
   }
-  if (!w || !w_split) return fail(TTK_EINVAL, "%s: w and w_split must not be NULL", what);
+  if (!w) return fail(TTK_EINVAL, "%s: w must not be NULL", what);
   if (K % 32 != 0 || K >= (int64_t{1} << 22) || N >= (int64_t{1} << 31)) {
     return fail(TTK_EUNSUPPORTED, "%s: K=%lld must be a multiple of 32 below 2^22 and N=%lld below 2^31", what,
                 (long long)K, (long long)N);
   }
-  if (!aligned16(w) || !aligned16(w_split) || ldw % 4 != 0 || ldw < K || ldw >= (int64_t{1} << 31)) {
-    return fail(TTK_EUNSUPPORTED,
-                "%s: w and w_split must be 16-byte aligned, ldw a multiple of 4 and >= K (ldw=%lld)", what,
+  if (!aligned16(w) || ldw % 4 != 0 || ldw < K || ldw >= (int64_t{1} << 31)) {
+    return fail(TTK_EUNSUPPORTED, "%s: w must be 16-byte aligned, ldw a multiple of 4 and >= K (ldw=%lld)", what,
                 (long long)ldw);
   }
   return TTK_OK;
 }
 
-}  // namespace
-
-extern "C" ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, int64_t K,
-                                                  int64_t ldw, void* stream) {
-  g_error[0] = '\0';
-  const ttk_status st = check_linear_f32_weight("split weight", w, w_split, N, K, ldw);
-  if (st != TTK_OK) return st;
+// The buffer of W's terms: made by the call (`writable`) or given.
+ttk_status check_linear_f32_terms(const char* what, const void* terms, const void* w, int64_t N, int64_t K,
+                                  int64_t ldw, bool writable) {
+  if (!terms) return fail(TTK_EINVAL, "%s: the buffer of W's terms must not be NULL", what);
+  if (!aligned16(terms)) return fail(TTK_EUNSUPPORTED, "%s: the buffer of W's terms must be 16-byte aligned", what);
   const uint64_t wbytes = (static_cast<uint64_t>(N - 1) * ldw + K) * 4;
-  if (overlaps(w_split, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K)), w, wbytes)) {
-    return fail(TTK_EINVAL, "split weight: w_split overlaps w");
+  if (writable && overlaps(terms, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K)), w, wbytes)) {
+    return fail(TTK_EINVAL, "%s: the buffer of W's terms overlaps w", what);
   }
-  const hipError_t err = ttk::launch_split_weight(static_cast<const float*>(w), w_split, static_cast<int>(N),
-                                                  static_cast<int>(K), ldw, static_cast<hipStream_t>(stream));
-  if (err != hipSuccess) return fail(TTK_ELAUNCH, "split weight: launch failed: %s", hipGetErrorString(err));
   return TTK_OK;
 }
 
-extern "C" ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split, const void* bias,
-                                         void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
-                                         int64_t ldy, int activation, void* stream) {
+ttk_status split_weight(const char* what, const void* w, void* terms, int64_t N, int64_t K, int64_t ldw,
+                        void* stream) {
+  const hipError_t err = ttk::launch_split_weight(static_cast<const float*>(w), terms, static_cast<int>(N),
+                                                  static_cast<int>(K), ldw, static_cast<hipStream_t>(stream));
+  if (err != hipSuccess) return fail(TTK_ELAUNCH, "%s: launch failed: %s", what, hipGetErrorString(err));
+  return TTK_OK;
+}
+
+// Y = act(X W^T + bias).  W's terms are in `terms` (make_terms: made there by
+// the call, in the form that reads them).
+ttk_status linear_f32(const void* x, const void* w, void* terms, bool make_terms, int64_t terms_bytes,
+                      const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                      int64_t ldy, int activation, void* stream) {
   g_error[0] = '\0';
   if (activation != TTK_ACT_NONE && activation != TTK_ACT_GELU) {
     return fail(TTK_EINVAL, "fp32 linear: unknown activation code %d", activation);
   }
   if (M < 0) return fail(TTK_EINVAL, "fp32 linear: M must be >= 0 (M=%lld)", (long long)M);
   if (M == 0) return TTK_OK;
-  const ttk_status st = check_linear_f32_weight("fp32 linear", w, w_split, N, K, ldw);
+  ttk_status st = check_linear_f32_weight("fp32 linear", w, N, K, ldw);
   if (st != TTK_OK) return st;
+  if (!make_terms) {
+    st = check_linear_f32_terms("fp32 linear", terms, w, N, K, ldw, false);
+    if (st != TTK_OK) return st;
+  }
   if (!x || !y) return fail(TTK_EINVAL, "fp32 linear: x and y must not be NULL");
   if (N % 4 != 0 || M >= (int64_t{1} << 31)) {
     return fail(TTK_EUNSUPPORTED, "fp32 linear: N=%lld must be a multiple of 4 and M=%lld below 2^31", (long long)N,
@@ -517,18 +530,37 @@ extern "C" ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const voi
                 "(ldx=%lld ldy=%lld)",
                 (long long)ldx, (long long)ldy);
   }
+  const ttk::LinearF32Form form = ttk::linear_f32_form(M, N, K, !make_terms);
+  const bool reads_terms = form == ttk::LinearF32Form::kTiles128;
+  const uint64_t tbytes = static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K));
   const uint64_t xbytes = (static_cast<uint64_t>(M - 1) * ldx + K) * 4;
   const uint64_t wbytes = (static_cast<uint64_t>(N - 1) * ldw + K) * 4;
   const uint64_t ybytes = (static_cast<uint64_t>(M - 1) * ldy + N) * 4;
+  if (make_terms && reads_terms) {
+    if (terms_bytes < static_cast<int64_t>(tbytes)) {
+      return fail(TTK_EINVAL, "fp32 linear: the workspace must hold %lld bytes (got %lld)", (long long)tbytes,
+                  (long long)terms_bytes);
+    }
+    st = check_linear_f32_terms("fp32 linear", terms, w, N, K, ldw, true);
+    if (st != TTK_OK) return st;
+    if (overlaps(terms, tbytes, x, xbytes) ||
+        (bias != nullptr && overlaps(terms, tbytes, bias, static_cast<uint64_t>(N) * 4))) {
+      return fail(TTK_EINVAL, "fp32 linear: the workspace overlaps an input");
+    }
+  }
   if (overlaps(y, ybytes, x, xbytes) || overlaps(y, ybytes, w, wbytes) ||
-      overlaps(y, ybytes, w_split, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K))) ||
+      ((reads_terms || !make_terms) && overlaps(y, ybytes, terms, tbytes)) ||
       (bias != nullptr && overlaps(y, ybytes, bias, static_cast<uint64_t>(N) * 4))) {
     return fail(TTK_EINVAL, "fp32 linear: y overlaps an input");
+  }
+  if (make_terms && reads_terms) {
+    st = split_weight("fp32 linear", w, terms, N, K, ldw, stream);
+    if (st != TTK_OK) return st;
   }
   ttk::LinearF32Params p{};
   p.x = static_cast<const float*>(x);
   p.w = static_cast<const float*>(w);
-  p.wp = w_split;
+  p.wp = reads_terms ? terms : nullptr;
   p.bias = static_cast<const float*>(bias);
   p.y = static_cast<float*>(y);
   p.ldx = ldx;
@@ -538,9 +570,32 @@ extern "C" ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const voi
   p.N = static_cast<int>(N);
   p.K = static_cast<int>(K);
   const hipError_t err =
-      ttk::launch_linear_f32(p, activation == TTK_ACT_GELU, static_cast<hipStream_t>(stream));
+      ttk::launch_linear_f32(p, form, activation == TTK_ACT_GELU, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(TTK_ELAUNCH, "fp32 linear: launch failed: %s", hipGetErrorString(err));
   return TTK_OK;
+}
+
+}  // namespace
+
+extern "C" ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, int64_t N, int64_t K,
+                                                  int64_t ldw, void* stream) {
+  g_error[0] = '\0';
+  ttk_status st = check_linear_f32_weight("split weight", w, N, K, ldw);
+  if (st == TTK_OK) st = check_linear_f32_terms("split weight", w_split, w, N, K, ldw, true);
+  return st == TTK_OK ? split_weight("split weight", w, w_split, N, K, ldw, stream) : st;
+}
+
+extern "C" ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split, const void* bias,
+                                         void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                         int64_t ldy, int activation, void* stream) {
+  return linear_f32(x, w, const_cast<void*>(w_split), false, 0, bias, y, M, N, K, ldx, ldw, ldy, activation, stream);
+}
+
+extern "C" ttk_status ttk_linear_f32_fwd_ws(const void* x, const void* w, const void* bias, void* y, int64_t M,
+                                            int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy,
+                                            int activation, void* workspace, int64_t workspace_bytes,
+                                            void* stream) {
+  return linear_f32(x, w, workspace, true, workspace_bytes, bias, y, M, N, K, ldx, ldw, ldy, activation, stream);
 }
 
 namespace {

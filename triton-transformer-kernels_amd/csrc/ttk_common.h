@@ -176,7 +176,7 @@ struct LinearLnParams {
 struct LinearF32Params {
   const float* x;
   const float* w;
-  const void* wp;     // W's three bf16 terms as packed by launch_split_weight
+  const void* wp;     // W's three bf16 terms as packed by launch_split_weight, or null
   const float* bias;  // [N] or null
   float* y;
   int64_t ldx, ldw, ldy;
@@ -210,9 +210,14 @@ hipError_t launch_gelu(int dtype, const void* x, void* y, int64_t n, hipStream_t
 // fills the tile fields of p and sizes the grid.
 hipError_t launch_linear(int dtype, int activation, LinearParams& p, hipStream_t stream);
 
+// Kernel of an fp32 Linear launch (see linear_f32_fwd.hip): only the one with
+// 128 x 128 tiles reads W as terms (LinearF32Params::wp).
+enum class LinearF32Form { kTiles32, kTiles64, kTiles128 };
+// The fastest form; `terms_ready`: W's terms are there already.
+LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, bool terms_ready);
 // fp32 Linear, optionally with the exact GELU; fills the tile fields of p and
 // sizes the grid.  K a multiple of 32, N of 4.
-hipError_t launch_linear_f32(LinearF32Params& p, bool gelu, hipStream_t stream);
+hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream);
 // W [N, K] fp32 (row stride ldw, K a multiple of 16) as three bf16 terms in
 // MFMA fragment order: ceil(N / 32) * 32 * K * 6 bytes.
 hipError_t launch_split_weight(const float* w, void* wp, int N, int K, int64_t ldw, hipStream_t stream);

@@ -27,6 +27,14 @@ def launch(index: int, entry, *args) -> int:
         return entry(*args, raw_stream(index))
 
 
+def query(index: int, entry, *args):
+    """``entry(*args)`` with device ``index`` current."""
+    if _current_device() == index:
+        return entry(*args)
+    with torch.cuda.device(index):
+        return entry(*args)
+
+
 def vector_ready(t: torch.Tensor) -> bool:
     """Rows of a 4-D tensor start on 16-byte boundaries (128-bit accesses)."""
     s = t.stride()

@@ -42,11 +42,13 @@ EXPORTED_SYMBOLS = (
     "ttk_linear_f32_split_bytes",
     "ttk_linear_f32_split_weight",
     "ttk_linear_f32_fwd",
+    "ttk_linear_f32_workspace_size",
+    "ttk_linear_f32_fwd_ws",
     "ttk_linear_residual_ln_workspace_size",
     "ttk_linear_pack_weight",
     "ttk_linear_residual_ln_fwd",
 )
-ABI_VERSION = 10
+ABI_VERSION = 11
 # TTK_ATTENTION_WS_COUNTER_BYTES: the zero-initialised counter block that
 # leads every attention workspace, the same for every launch shape.
 ATTENTION_WS_COUNTER_BYTES = 16384
@@ -112,6 +114,11 @@ def _configure(lib: ctypes.CDLL) -> None:
     lib.ttk_linear_f32_fwd.restype = ctypes.c_int
     lib.ttk_linear_f32_fwd.argtypes = [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64,
                                        ctypes.c_int, _vp]
+    lib.ttk_linear_f32_workspace_size.restype = _i64
+    lib.ttk_linear_f32_workspace_size.argtypes = [_i64, _i64, _i64]
+    lib.ttk_linear_f32_fwd_ws.restype = ctypes.c_int
+    lib.ttk_linear_f32_fwd_ws.argtypes = [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, ctypes.c_int,
+                                          _vp, _i64, _vp]
     lib.ttk_linear_residual_ln_workspace_size.restype = _i64
     lib.ttk_linear_residual_ln_workspace_size.argtypes = [_i64]
     lib.ttk_linear_pack_weight.restype = ctypes.c_int

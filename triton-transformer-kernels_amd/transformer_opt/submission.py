@@ -39,8 +39,8 @@ restricted it); graph replay is eligible for every supported shape and dtype
 instead of a measured shape set (submission.py:582-590), with up to
 ``max_cuda_graphs`` captures kept, one per input geometry.  fp32 projections
 run on the HIP kernel that forms them on the bf16 matrix cores from three-term
-splits of both operands (the weight's terms are made again by every forward,
-so that it follows every write to the weight); 16-bit ones, and widths that
+splits of both operands (the weight's are made again by every forward, so that
+it follows every write to the weight); 16-bit ones, and widths that
 kernel does not take, are library GEMMs (hipBLASLt through ``F.linear``).  In
 fp32 and bf16 the FFN's input projection and exact GELU are one HIP kernel
 (GELU in the GEMM epilogue), otherwise the GELU runs in place on the HIP
@@ -61,7 +61,7 @@ from .config import ATTENTION_BACKENDS, SUPPORTED_DTYPES
 from .dispatch import attention_forward
 from .kernels.gelu import gelu_
 from .kernels.linear import linear_gelu, linear_supported
-from .kernels.linear_f32 import linear_f32, linear_f32_supported, split_weight
+from .kernels.linear_f32 import linear_f32, linear_f32_supported
 from .kernels.linear_ln import linear_ln_supported, linear_residual_layer_norm
 from .kernels.linear_ln import workspace_bytes as linear_ln_workspace_bytes
 from .kernels.residual_layer_norm import fused_residual_layer_norm, layer_norm
@@ -203,28 +203,18 @@ class _Layout:
         return _Operands(exits[0], tuple(blocks), None, keepalive)
 
 
-def _project_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
-                 gelu: bool = False) -> Optional[torch.Tensor]:
-    """``F.linear(x, weight, bias)`` or its exact GELU on the fp32 kernel, or
-    None where that kernel does not take the call.
-
-    The weight's bf16 terms are made by every call, on the call's stream (and
-    inside a capture, into the capture's memory): nothing derived from a
-    parameter outlives the call, so a write to the parameter, in whatever way
-    it is done, is seen by the next forward or replay as the library GEMM
-    would see it.
-    """
-    if not linear_f32_supported(x, weight, bias):
-        return None
-    split = split_weight(weight)
-    return None if split is None else linear_f32(x, weight, split, bias, gelu=gelu)
-
-
 def _project(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> torch.Tensor:
     """``F.linear(x, weight, bias)``: the fp32 kernel where it takes the call,
-    else the library GEMM."""
-    y = _project_f32(x, weight, bias)
-    return F.linear(x, weight, bias) if y is None else y
+    else the library GEMM.
+
+    That kernel's terms of the weight are made by the call (inside a capture,
+    in the capture's memory): nothing derived from a parameter outlives the
+    call, so a write to the parameter, in whatever way it is done, is seen by
+    the next forward or replay as the library GEMM would see it.
+    """
+    if linear_f32_supported(x, weight, bias):
+        return linear_f32(x, weight, None, bias)
+    return F.linear(x, weight, bias)
 
 
 class _ModelTally:
@@ -418,10 +408,10 @@ class UserOptimizedTransformer(nn.Module):
         w, b = block.ffn_in_weight, block.ffn_in_bias
         if h.dtype == torch.bfloat16 and linear_supported(h, w, b) is None:
             inner = linear_gelu(h, w, b)
+        elif linear_f32_supported(h, w, b):
+            inner = linear_f32(h, w, None, b, gelu=True)
         else:
-            inner = _project_f32(h, w, b, gelu=True)
-            if inner is None:
-                inner = gelu_(F.linear(h, w, b))
+            inner = gelu_(F.linear(h, w, b))
         return _project(inner, block.ffn_out_weight, block.ffn_out_bias)
 
     @staticmethod
