@@ -299,6 +299,7 @@ int64_t ttk_linear_f32_workspace_size(int64_t M, int64_t N, int64_t K);
  * (workspace_bytes >= ttk_linear_f32_workspace_size(M, N, K), 16-byte aligned,
  * apart from every other argument; TTK_EINVAL otherwise), whose contents
  * before the call do not matter.  workspace may be NULL where that size is 0.
+ * ldw below 2^22 as well (TTK_EUNSUPPORTED otherwise).
  * Nothing is kept between calls.
  */
 ttk_status ttk_linear_f32_fwd_ws(const void* x, const void* w, const void* bias, void* y, int64_t M, int64_t N,

@@ -58,6 +58,7 @@ namespace ttk {
 namespace {
 
 constexpr int kFlThreads = 256;  // 4 wavefronts, one per SIMD
+constexpr int kFsThreads = 512;  // small products: 8 wavefronts
 constexpr int kFlBK = 32;        // k per stage: 128-byte rows of X
 constexpr int kFlTile = 128;     // tokens and features per tile
 constexpr int kFlFrag = 1024;    // bytes of one fragment (32 rows x 16 k of one term)
@@ -377,77 +378,116 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
   fl_vm_wait<0>();
 }
 
-// Small products: one workgroup of four wavefronts per TB*32 x TB*32 tile, the
-// wavefronts splitting K.  Fragments come straight from global memory, X and W
-// alike as two 16-byte halves of a row's 8 values, and are split in registers:
-// no terms of W have to be made first.  The wavefronts' sums are added in order
-// through LDS.
-// Against the same kernel on terms made beforehand 0.8 us more at K = 256 (256
-// x 768: 4.1 -> 4.9 us) and up to 35 % where the full chip runs (64 x 1024 x
-// 4096 22 -> 30 us, 1024 x 1024 x 1024 18 -> 21 us); making the terms is a
-// launch of 2.4 us for 256 x 256 weights, 7.5 us for 1024 x 4096.
+// Small products: one workgroup of eight wavefronts per TB*32 x TB*32 tile, the
+// wavefronts splitting K; X and W are both split in registers, so that no terms
+// of W have to be made first (a launch of 2.4 us for 256 x 256 weights, 7.5 us
+// for 1024 x 4096).  Each wavefront copies its k-steps' 64-byte row pieces by
+// LDS-DMA into a ring of its own (no barriers), four lanes a piece: fragments
+// loaded straight into registers have every lane in another row, and the L1
+// served one of them per cycle (230 cycles a k-step and CU in 32 x 32 tiles,
+// 512 in 64 x 64).  Row r's 16-byte chunk c sits at c ^ ((r >> 2) & 3), so the
+// 16 rows of a fragment read cover all banks.  The wavefronts' sums are added
+// in order through LDS.
+// Before -> here: 64 x 1024 x 4096 31 -> 20 us, 256 x 1024 x 1024 10.9 -> 9.9,
+// 512 x 1024 x 1024 18.9 -> 15.6, 1024 x 1024 x 1024 21.5 -> 19.1, 256 x 256 x
+// 1024 10.0 -> 7.7, 256 x 256 x 256 4.8 -> 4.5.  Bound by the splits' VALU work
+// and the MFMAs one after the other (2600 cycles a k-step and SIMD in 64 x 64
+// tiles, 1536 of them MFMA): the next k-step's splits between this one's MFMAs
+// gained 5 - 13 % from K = 2048 up in few tiles and lost 5 - 20 % elsewhere.
+// The library's fp32 GEMM is faster where few tiles meet a long K (64 x 1024 x
+// 4096 11 us, 64 x 1024 x 1024 6.0 against 7.7), at three times the error.
 template <int TB, bool GELU, bool BIAS>
-__global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_kernel(LinearF32Params p) {
-  constexpr int NW = kFlThreads / 64;
-  __shared__ f32x4 part[NW][TB * TB * 4][64];
+__global__ __launch_bounds__(kFsThreads, 2) void linear_f32_small_kernel(LinearF32Params p) {
+  constexpr int NW = kFsThreads / 64;
+  constexpr int R = TB == 1 ? 4 : 2;           // ring depth
+  constexpr int kHalf = 32 * TB * 64;          // X (then W) of a k-step: rows of 64 bytes
+  constexpr int kRing = R * 2 * kHalf;
+  constexpr int XC = kHalf / 1024;             // copies of X (and of W) per k-step
+  static_assert(TB * TB * 4096 <= kRing, "a wavefront's sums fit its ring");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[NW * kRing];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r32 = lane & 31;
   const int h = lane >> 5;
-  const int m0 = static_cast<int>(blockIdx.x) / p.tiles_n * (32 * TB);
-  const int n0 = static_cast<int>(blockIdx.x) % p.tiles_n * (32 * TB);
+  // Workgroups are dealt round-robin to the 8 XCDs: each gets a contiguous run
+  // of tiles, in bands of group_m rows of tiles, and keeps their operands in
+  // its L2 (up to 10 % from two rounds of tiles on).
+  const int o = static_cast<int>(blockIdx.x & 7) * p.per_xcd + static_cast<int>(blockIdx.x >> 3);
+  if (o >= p.tiles) return;
+  const int span = p.group_m * p.tiles_n;
+  const int first = o / span * p.group_m;
+  const int gs = min(p.group_m, p.tiles_m - first);
+  const int rem = o % span;
+  const int m0 = (first + rem % gs) * (32 * TB);
+  const int n0 = rem / gs * (32 * TB);
   const int KQ = p.K / 16;
   const int q0 = KQ * wave / NW, q1 = KQ * (wave + 1) / NW;
-  const float* xrow[TB];
-  const float* wrow[TB];
+
+  // Copy c fills rows 16 c .. + 15; rows past the last repeat it.
+  const unsigned chunk = static_cast<unsigned>((lane & 3) ^ ((lane >> 4) & 3)) * 16u;
+  unsigned xoff[XC], woff[XC];
 #pragma unroll
-  for (int b = 0; b < TB; ++b) {
-    xrow[b] = p.x + static_cast<int64_t>(min(m0 + 32 * b + r32, p.M - 1)) * p.ldx + 8 * h;
-    wrow[b] = p.w + static_cast<int64_t>(min(n0 + 32 * b + r32, p.N - 1)) * p.ldw + 8 * h;
+  for (int c = 0; c < XC; ++c) {
+    const int row = 16 * c + (lane >> 2);
+    xoff[c] = static_cast<unsigned>(__umul24(min(row, p.M - 1 - m0), static_cast<unsigned>(p.ldx) * 4u)) + chunk;
+    woff[c] = static_cast<unsigned>(__umul24(min(row, p.N - 1 - n0), static_cast<unsigned>(p.ldw) * 4u)) + chunk;
   }
+  const float* xbase = p.x + static_cast<int64_t>(m0) * p.ldx;
+  const float* wbase = p.w + static_cast<int64_t>(n0) * p.ldw;
+  unsigned char* const ring = smem + wave * kRing;
+  const unsigned ring_lds = static_cast<unsigned>(reinterpret_cast<size_t>(TTK_FL_LDS(smem))) + wave * kRing;
+  auto issue = [&](int q, int slot) __attribute__((always_inline)) {
+    const int k = 16 * min(q, q1 - 1);  // past the last: again, into a slot that nobody reads
+#pragma unroll
+    for (int c = 0; c < XC; ++c) fl_dma16(xbase + k, xoff[c], ring_lds + slot * (2 * kHalf) + c * 1024);
+#pragma unroll
+    for (int c = 0; c < XC; ++c) fl_dma16(wbase + k, woff[c], ring_lds + slot * (2 * kHalf) + kHalf + c * 1024);
+  };
+  // This lane's 8 values of row 32 b + r32, k = 8 h .. + 7, from row block `at`.
+  auto read_split = [&](Split8& d, const unsigned char* at) __attribute__((always_inline)) {
+    f32x4 v[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      v[j] = *reinterpret_cast<const f32x4*>(at + r32 * 64 + 16 * ((2 * h + j) ^ ((r32 >> 2) & 3)));
+#pragma unroll
+    for (int u = 0; u < 4; ++u) split_pair(d, u, v[u >> 1][2 * (u & 1)], v[u >> 1][2 * (u & 1) + 1]);
+  };
+
   f32x16 hi[TB][TB], lo[TB][TB];
 #pragma unroll
   for (int i = 0; i < TB; ++i)
 #pragma unroll
     for (int j = 0; j < TB; ++j) hi[i][j] = lo[i][j] = f32x16{};
-  constexpr int UN = TB == 1 ? 4 : 2;  // k-steps whose loads are in flight together
-  for (int q = q0; q < q1; q += UN) {
-    f32x4 rx[UN][TB][2], rw[UN][TB][2];
+  if (q0 < q1) {
 #pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      const int qq = min(q + u, q1 - 1);
+    for (int s = 0; s < R - 1; ++s) issue(q0 + s, s);
+    int slot = 0;
+    for (int q = q0; q < q1; ++q) {
+      // K-step q has to be in LDS (younger: the copies of q + 1 .. q + R - 2),
+      // and the reads of k-step q - 1, whose slot is filled next, done.
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * 2 * XC) : "memory");
+      issue(q + R - 1, slot == 0 ? R - 1 : slot - 1);
+      const unsigned char* at = ring + slot * (2 * kHalf);
+      Split8 x[TB], w[TB];
 #pragma unroll
       for (int b = 0; b < TB; ++b) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          rx[u][b][j] = *reinterpret_cast<const f32x4*>(xrow[b] + 16 * qq + 4 * j);
-          rw[u][b][j] = *reinterpret_cast<const f32x4*>(wrow[b] + 16 * qq + 4 * j);
-        }
+        read_split(x[b], at + b * 2048);
+        read_split(w[b], at + kHalf + b * 2048);
       }
-    }
 #pragma unroll
-    for (int u = 0; u < UN; ++u) {
-      if (q + u < q1) {
-        Split8 x[TB], w[TB];
+      for (int pr = 0; pr < 6; ++pr)
 #pragma unroll
-        for (int b = 0; b < TB; ++b)
+        for (int j = 0; j < TB; ++j)
 #pragma unroll
-          for (int d = 0; d < 4; ++d) {
-            split_pair(x[b], d, rx[u][b][d >> 1][2 * (d & 1)], rx[u][b][d >> 1][2 * (d & 1) + 1]);
-            split_pair(w[b], d, rw[u][b][d >> 1][2 * (d & 1)], rw[u][b][d >> 1][2 * (d & 1) + 1]);
+          for (int i = 0; i < TB; ++i) {
+            f32x16& c = pr == 2 ? hi[i][j] : lo[i][j];
+            c = mfma_x3(w[i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
           }
-#pragma unroll
-        for (int pr = 0; pr < 6; ++pr)
-#pragma unroll
-          for (int j = 0; j < TB; ++j)
-#pragma unroll
-            for (int i = 0; i < TB; ++i) {
-              f32x16& c = pr == 2 ? hi[i][j] : lo[i][j];
-              c = mfma_x3(w[i].t[kTermW[pr]], x[j].t[kTermX[pr]], c);
-            }
-      }
+      slot = slot == R - 1 ? 0 : slot + 1;
     }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   }
+  f32x4* const sums = reinterpret_cast<f32x4*>(ring) + lane;  // of this wavefront, 64 to a chunk
 #pragma unroll
   for (int i = 0; i < TB; ++i)
 #pragma unroll
@@ -457,16 +497,17 @@ __global__ __launch_bounds__(kFlThreads, TB == 1 ? 4 : 2) void linear_f32_small_
         f32x4 v;
 #pragma unroll
         for (int e = 0; e < 4; ++e) v[e] = hi[i][j][4 * g + e] + lo[i][j][4 * g + e];
-        part[wave][(i * TB + j) * 4 + g][lane] = v;
+        sums[((i * TB + j) * 4 + g) * 64] = v;
       }
   __syncthreads();
 #pragma unroll
   for (int c = wave; c < TB * TB * 4; c += NW) {
     const int i = c / (4 * TB), j = (c >> 2) % TB, g = c & 3;
     const int m = m0 + 32 * j + r32, f = n0 + 32 * i + 8 * g + 4 * h;
-    f32x4 v = part[0][c][lane];
+    const f32x4* part = reinterpret_cast<const f32x4*>(smem) + c * 64 + lane;
+    f32x4 v = part[0];
 #pragma unroll
-    for (int s = 1; s < NW; ++s) v += part[s][c][lane];
+    for (int s = 1; s < NW; ++s) v += part[s * (kRing / 16)];
     bool redo = false;
 #pragma unroll
     for (int e = 0; e < 4; ++e) redo |= redo_x3(v[e]);
@@ -495,7 +536,12 @@ template <int TB>
 hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
   p.tiles_n = (p.N + 32 * TB - 1) / (32 * TB);
   p.tiles_m = (p.M + 32 * TB - 1) / (32 * TB);
-  const dim3 grid(static_cast<unsigned>(p.tiles_n) * static_cast<unsigned>(p.tiles_m)), blk(kFlThreads);
+  p.tiles = p.tiles_m * p.tiles_n;
+  p.per_xcd = (p.tiles + 7) / 8;
+  // A band is as square as an XCD's share allows.
+  p.group_m = 1;
+  while (2 * p.group_m <= p.tiles_m && 4 * p.group_m * p.group_m <= p.per_xcd) p.group_m *= 2;
+  const dim3 grid(8 * static_cast<unsigned>(p.per_xcd)), blk(kFsThreads);
   if (gelu) {
     if (p.bias) linear_f32_small_kernel<TB, true, true><<<grid, blk, 0, stream>>>(p);
     else linear_f32_small_kernel<TB, true, false><<<grid, blk, 0, stream>>>(p);
@@ -564,21 +610,23 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4
 
 }  // namespace
 
-LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, bool terms_ready) {
+LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready) {
+  if (ldw >= int64_t{1} << 22) return LinearF32Form::kTiles128;
   // The form with the least expected time (us) on 256 CUs, from the measured
-  // times of the three over products from 16 x 3072 x 1024 to 32768 x 2048 x
-  // 512: a launch's fixed cost, then the longest chain of k-steps or the rate
-  // at which the full chip runs, whichever lasts longer; for the tiled form
+  // times of the three over products from 1 x 256 x 256 to 8192 x 4096 x 1024:
+  // a launch's fixed cost and the chain of k-steps in one round of tiles, which
+  // runs slower the more CUs have a tile, or whole rounds; for the tiled form
   // also the launch that makes W's terms, unless they are there.  E.g. 256 x
-  // 256 x 256: 4.7 us for 32 x 32 tiles, 8.8 for 64 x 64, 15.3 for 128 x 128;
-  // 2048 x 512 x 512: 18.8, 13.8, 23.9; 4096 x 1024 x 1024: 117, 71, 50.
-  const double flops = 2.0 * static_cast<double>(M) * N * K;
-  const double tiles = std::ceil(M / 128.0) * std::ceil(N / 128.0);
-  const double rounds = std::ceil(tiles / 256.0);
-  const double t32 = 3.2 + std::max(flops / 74e6, K / 160.0);
-  const double t64 = 4.5 + std::max(flops / 112e6, K / 73.0);
-  double t128 = 5.0 + static_cast<double>(K / kFlBK) * (rounds > 1.0 ? 1.37 * rounds : 0.85 + 0.52 * tiles / 256.0);
-  if (!terms_ready) t128 += 3.0 + static_cast<double>(N) * K / 0.6e6;
+  // 256 x 256: 4.5 us for 32 x 32 tiles, 7.2 for 64 x 64, 15.2 for 128 x 128;
+  // 1024 x 1024 x 1024: 33, 19, 45; 4096 x 1024 x 1024: 119, 67, 54.
+  constexpr double kCus = 256.0;
+  auto tiles = [&](double t) { return std::ceil(M / t) * std::ceil(N / t); };
+  const double k = static_cast<double>(K), n32 = tiles(32.0), n64 = tiles(64.0), n128 = tiles(128.0);
+  const double r32 = std::ceil(n32 / kCus), r64 = std::ceil(n64 / kCus), r128 = std::ceil(n128 / kCus);
+  const double t32 = r32 > 1.0 ? 2.6 + r32 * (1.6 + k / 180.0) : 3.2 + k / 250.0 + n32 / kCus * (0.6 + k / 700.0);
+  const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 75.0) : 4.6 + k / 113.0 + n64 / kCus * (0.9 + k / 230.0);
+  double t128 = 5.0 + k / kFlBK * (r128 > 1.0 ? 1.37 * r128 : 0.85 + 0.52 * n128 / kCus);
+  if (!terms_ready) t128 += 3.0 + N * k / 0.6e6;
   if (t32 <= t64 && t32 <= t128) return LinearF32Form::kTiles32;
   return t64 <= t128 ? LinearF32Form::kTiles64 : LinearF32Form::kTiles128;
 }

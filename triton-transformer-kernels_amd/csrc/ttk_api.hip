@@ -456,7 +456,7 @@ extern "C" int64_t ttk_linear_f32_split_bytes(int64_t N, int64_t K) {
 extern "C" int64_t ttk_linear_f32_workspace_size(int64_t M, int64_t N, int64_t K) {
   const int64_t bytes = ttk_linear_f32_split_bytes(N, K);
   if (M <= 0 || M >= (int64_t{1} << 31) || bytes == 0) return 0;
-  return ttk::linear_f32_form(M, N, K, false) == ttk::LinearF32Form::kTiles128 ? bytes : 0;
+  return ttk::linear_f32_form(M, N, K, K, false) == ttk::LinearF32Form::kTiles128 ? bytes : 0;
 }
 
 namespace {
@@ -524,13 +524,13 @@ ttk_status linear_f32(const void* x, const void* w, void* terms, bool make_terms
     return fail(TTK_EUNSUPPORTED, "fp32 linear: x, bias and y must be 16-byte aligned");
   }
   if (ldx % 4 != 0 || ldy % 4 != 0 || ldx < K || ldy < N || ldx >= (int64_t{1} << 22) ||
-      ldy >= (int64_t{1} << 22)) {
+      ldy >= (int64_t{1} << 22) || (make_terms && ldw >= (int64_t{1} << 22))) {
     return fail(TTK_EUNSUPPORTED,
                 "fp32 linear: ldx and ldy must be multiples of 4 below 2^22 with ldx >= K and ldy >= N "
                 "(ldx=%lld ldy=%lld)",
                 (long long)ldx, (long long)ldy);
   }
-  const ttk::LinearF32Form form = ttk::linear_f32_form(M, N, K, !make_terms);
+  const ttk::LinearF32Form form = ttk::linear_f32_form(M, N, K, ldw, !make_terms);
   const bool reads_terms = form == ttk::LinearF32Form::kTiles128;
   const uint64_t tbytes = static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K));
   const uint64_t xbytes = (static_cast<uint64_t>(M - 1) * ldx + K) * 4;

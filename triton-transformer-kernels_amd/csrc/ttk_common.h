@@ -213,8 +213,9 @@ hipError_t launch_linear(int dtype, int activation, LinearParams& p, hipStream_t
 // Kernel of an fp32 Linear launch (see linear_f32_fwd.hip): only the one with
 // 128 x 128 tiles reads W as terms (LinearF32Params::wp).
 enum class LinearF32Form { kTiles32, kTiles64, kTiles128 };
-// The fastest form; `terms_ready`: W's terms are there already.
-LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, bool terms_ready);
+// The fastest form; `terms_ready`: W's terms are there already.  Row strides of W
+// from 2^22 up take 128 x 128 tiles.
+LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready);
 // fp32 Linear, optionally with the exact GELU; fills the tile fields of p and
 // sizes the grid.  K a multiple of 32, N of 4.
 hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream);
