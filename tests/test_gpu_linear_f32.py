@@ -11,7 +11,7 @@ import torch.nn.functional as F
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    # 32 x 32 tiles, K split over eight wavefronts (some without a k-step).
+    # 32 x 32 tiles, K split over four or eight wavefronts (some without a k-step).
     (1, 4, 32), (31, 36, 64), (33, 32, 96), (129, 132, 224),
     # 64 x 64 tiles, ragged both ways.
     (2047, 516, 544), (2049, 1540, 512),
@@ -57,7 +57,7 @@ def test_linear_f32_against_float64(gpu_ready, rows, out_features, in_features, 
 
 
 @pytest.mark.parametrize("rows,out_features,in_features", SHAPES + [
-    (16, 1024, 4096), (8192, 768, 256), (1000, 516, 544), (700, 1540, 512)])
+    (16, 1024, 4096), (8192, 768, 256), (1000, 516, 544), (700, 1540, 512), (300, 1020, 288)])
 @pytest.mark.parametrize("gelu", [False, True], ids=["linear", "gelu"])
 def test_terms_made_by_the_call(gpu_ready, rows, out_features, in_features, gelu):
     # Small products split W in registers, the tiled kernel reads terms made

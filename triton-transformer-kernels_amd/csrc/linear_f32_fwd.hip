@@ -58,7 +58,6 @@ namespace ttk {
 namespace {
 
 constexpr int kFlThreads = 256;  // 4 wavefronts, one per SIMD
-constexpr int kFsThreads = 512;  // small products: 8 wavefronts
 constexpr int kFlBK = 32;        // k per stage: 128-byte rows of X
 constexpr int kFlTile = 128;     // tokens and features per tile
 constexpr int kFlFrag = 1024;    // bytes of one fragment (32 rows x 16 k of one term)
@@ -378,7 +377,7 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
   fl_vm_wait<0>();
 }
 
-// Small products: one workgroup of eight wavefronts per TB*32 x TB*32 tile, the
+// Small products: one workgroup of NW wavefronts per TB*32 x TB*32 tile, the
 // wavefronts splitting K; X and W are both split in registers, so that no terms
 // of W have to be made first (a launch of 2.4 us for 256 x 256 weights, 7.5 us
 // for 1024 x 4096).  Each wavefront copies its k-steps' 64-byte row pieces by
@@ -388,17 +387,19 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
 // 512 in 64 x 64).  Row r's 16-byte chunk c sits at c ^ ((r >> 2) & 3), so the
 // 16 rows of a fragment read cover all banks.  The wavefronts' sums are added
 // in order through LDS.
-// Before -> here: 64 x 1024 x 4096 31 -> 20 us, 256 x 1024 x 1024 10.9 -> 9.9,
-// 512 x 1024 x 1024 18.9 -> 15.6, 1024 x 1024 x 1024 21.5 -> 19.1, 256 x 256 x
-// 1024 10.0 -> 7.7, 256 x 256 x 256 4.8 -> 4.5.  Bound by the splits' VALU work
+// Eight wavefronts, which fill a CU's LDS, or four where two tiles of 32 x 32
+// share a CU or K is short: 512 x 1024 x 256 8.0 -> 6.1 us, 512 x 512 x 64 3.9
+// -> 3.5; 64 x 1024 x 1024 takes 7.5 with eight and 10.1 with four.
+// Fragments in registers -> here: 64 x 1024 x 4096 31 -> 20 us, 256 x 1024 x
+// 1024 10.9 -> 9.6, 512 x 1024 x 1024 18.9 -> 14.4, 1024 x 1024 x 1024 21.5 ->
+// 18.5, 256 x 256 x 1024 10.0 -> 7.6, 256 x 256 x 256 4.8 -> 4.3.  Bound by the splits' VALU work
 // and the MFMAs one after the other (2600 cycles a k-step and SIMD in 64 x 64
 // tiles, 1536 of them MFMA): the next k-step's splits between this one's MFMAs
 // gained 5 - 13 % from K = 2048 up in few tiles and lost 5 - 20 % elsewhere.
 // The library's fp32 GEMM is faster where few tiles meet a long K (64 x 1024 x
 // 4096 11 us, 64 x 1024 x 1024 6.0 against 7.7), at three times the error.
-template <int TB, bool GELU, bool BIAS>
-__global__ __launch_bounds__(kFsThreads, 2) void linear_f32_small_kernel(LinearF32Params p) {
-  constexpr int NW = kFsThreads / 64;
+template <int TB, int NW, bool GELU, bool BIAS>
+__global__ __launch_bounds__(64 * NW, 2) void linear_f32_small_kernel(LinearF32Params p) {
   constexpr int R = TB == 1 ? 4 : 2;           // ring depth
   constexpr int kHalf = 32 * TB * 64;          // X (then W) of a k-step: rows of 64 bytes
   constexpr int kRing = R * 2 * kHalf;
@@ -437,7 +438,7 @@ __global__ __launch_bounds__(kFsThreads, 2) void linear_f32_small_kernel(LinearF
   unsigned char* const ring = smem + wave * kRing;
   const unsigned ring_lds = static_cast<unsigned>(reinterpret_cast<size_t>(TTK_FL_LDS(smem))) + wave * kRing;
   auto issue = [&](int q, int slot) __attribute__((always_inline)) {
-    const int k = 16 * min(q, q1 - 1);  // past the last: again, into a slot that nobody reads
+    const int k = 16 * q;
 #pragma unroll
     for (int c = 0; c < XC; ++c) fl_dma16(xbase + k, xoff[c], ring_lds + slot * (2 * kHalf) + c * 1024);
 #pragma unroll
@@ -460,13 +461,19 @@ __global__ __launch_bounds__(kFsThreads, 2) void linear_f32_small_kernel(LinearF
     for (int j = 0; j < TB; ++j) hi[i][j] = lo[i][j] = f32x16{};
   if (q0 < q1) {
 #pragma unroll
-    for (int s = 0; s < R - 1; ++s) issue(q0 + s, s);
+    for (int s = 0; s < R - 1; ++s)
+      if (q0 + s < q1) issue(q0 + s, s);
     int slot = 0;
     for (int q = q0; q < q1; ++q) {
-      // K-step q has to be in LDS (younger: the copies of q + 1 .. q + R - 2),
-      // and the reads of k-step q - 1, whose slot is filled next, done.
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * 2 * XC) : "memory");
-      issue(q + R - 1, slot == 0 ? R - 1 : slot - 1);
+      // K-step q has to be in LDS (younger: the copies of q + 1 .. q + R - 2, or
+      // up to the last), and the reads of k-step q - 1, whose slot is filled
+      // next, done.
+      if (q + R - 2 < q1) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((R - 2) * 2 * XC) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      }
+      if (q + R - 1 < q1) issue(q + R - 1, slot == 0 ? R - 1 : slot - 1);
       const unsigned char* at = ring + slot * (2 * kHalf);
       Split8 x[TB], w[TB];
 #pragma unroll
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(kFsThreads, 2) void linear_f32_small_kernel(LinearF
           }
       slot = slot == R - 1 ? 0 : slot + 1;
     }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
   f32x4* const sums = reinterpret_cast<f32x4*>(ring) + lane;  // of this wavefront, 64 to a chunk
 #pragma unroll
@@ -532,7 +539,7 @@ __global__ __launch_bounds__(kFsThreads, 2) void linear_f32_small_kernel(LinearF
   }
 }
 
-template <int TB>
+template <int TB, int NW>
 hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
   p.tiles_n = (p.N + 32 * TB - 1) / (32 * TB);
   p.tiles_m = (p.M + 32 * TB - 1) / (32 * TB);
@@ -541,13 +548,13 @@ hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
   // A band is as square as an XCD's share allows.
   p.group_m = 1;
   while (2 * p.group_m <= p.tiles_m && 4 * p.group_m * p.group_m <= p.per_xcd) p.group_m *= 2;
-  const dim3 grid(8 * static_cast<unsigned>(p.per_xcd)), blk(kFsThreads);
+  const dim3 grid(8 * static_cast<unsigned>(p.per_xcd)), blk(64 * NW);
   if (gelu) {
-    if (p.bias) linear_f32_small_kernel<TB, true, true><<<grid, blk, 0, stream>>>(p);
-    else linear_f32_small_kernel<TB, true, false><<<grid, blk, 0, stream>>>(p);
+    if (p.bias) linear_f32_small_kernel<TB, NW, true, true><<<grid, blk, 0, stream>>>(p);
+    else linear_f32_small_kernel<TB, NW, true, false><<<grid, blk, 0, stream>>>(p);
   } else {
-    if (p.bias) linear_f32_small_kernel<TB, false, true><<<grid, blk, 0, stream>>>(p);
-    else linear_f32_small_kernel<TB, false, false><<<grid, blk, 0, stream>>>(p);
+    if (p.bias) linear_f32_small_kernel<TB, NW, false, true><<<grid, blk, 0, stream>>>(p);
+    else linear_f32_small_kernel<TB, NW, false, false><<<grid, blk, 0, stream>>>(p);
   }
   return hipGetLastError();
 }
@@ -610,31 +617,44 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4
 
 }  // namespace
 
+namespace {
+
+double tile_count(double M, double N, double side) { return std::ceil(M / side) * std::ceil(N / side); }
+constexpr double kCus = 256.0;
+
+// Wavefronts of a 32 x 32 tile (see linear_f32_small_kernel).
+bool four_wavefronts(int64_t M, int64_t N, int64_t K) { return K <= 64 || tile_count(M, N, 32.0) > kCus; }
+
+}  // namespace
+
 LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready) {
   if (ldw >= int64_t{1} << 22) return LinearF32Form::kTiles128;
   // The form with the least expected time (us) on 256 CUs, from the measured
   // times of the three over products from 1 x 256 x 256 to 8192 x 4096 x 1024:
   // a launch's fixed cost and the chain of k-steps in one round of tiles, which
-  // runs slower the more CUs have a tile, or whole rounds; for the tiled form
-  // also the launch that makes W's terms, unless they are there.  E.g. 256 x
-  // 256 x 256: 4.5 us for 32 x 32 tiles, 7.2 for 64 x 64, 15.2 for 128 x 128;
-  // 1024 x 1024 x 1024: 33, 19, 45; 4096 x 1024 x 1024: 119, 67, 54.
-  constexpr double kCus = 256.0;
-  auto tiles = [&](double t) { return std::ceil(M / t) * std::ceil(N / t); };
-  const double k = static_cast<double>(K), n32 = tiles(32.0), n64 = tiles(64.0), n128 = tiles(128.0);
-  const double r32 = std::ceil(n32 / kCus), r64 = std::ceil(n64 / kCus), r128 = std::ceil(n128 / kCus);
-  const double t32 = r32 > 1.0 ? 2.6 + r32 * (1.6 + k / 180.0) : 3.2 + k / 250.0 + n32 / kCus * (0.6 + k / 700.0);
-  const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 75.0) : 4.6 + k / 113.0 + n64 / kCus * (0.9 + k / 230.0);
-  double t128 = 5.0 + k / kFlBK * (r128 > 1.0 ? 1.37 * r128 : 0.85 + 0.52 * n128 / kCus);
-  if (!terms_ready) t128 += 3.0 + N * k / 0.6e6;
+  // runs slower the more CUs have a tile, or whole rounds (of two 32 x 32 tiles
+  // a CU); for the tiled form also the launch that makes W's terms, unless they
+  // are there.  E.g. 256 x 256 x 256: 4.3 us for 32 x 32 tiles, 7.0 for 64 x
+  // 64, 15.2 for 128 x 128; 512 x 1024 x 1024: 14.4, 15.7, 46; 1024 x 1024 x
+  // 1024: 25.6, 18.5, 45; 4096 x 1024 x 1024: 88, 65, 54.
+  const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
+  const double n32 = tile_count(m, n, 32.0), n64 = tile_count(m, n, 64.0), n128 = tile_count(m, n, 128.0);
+  const double r64 = std::ceil(n64 / kCus), r128 = std::min(std::ceil(n128 / kCus), 1.12 * n128 / kCus);
+  const double t32 = n32 > kCus ? 2.4 + std::ceil(n32 / (2.0 * kCus)) * (1.6 + k / 100.0)
+                                : 3.0 + k / 250.0 + n32 / kCus * (0.3 + k / 700.0);
+  const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 78.0) : 4.5 + k / 113.0 + n64 / kCus * (0.9 + k / 230.0);
+  double t128 = 5.0 + k / kFlBK * (n128 > kCus ? 1.37 * r128 : 0.85 + 0.52 * n128 / kCus);
+  if (!terms_ready) t128 += 3.0 + n * k / 0.6e6;
   if (t32 <= t64 && t32 <= t128) return LinearF32Form::kTiles32;
   return t64 <= t128 ? LinearF32Form::kTiles64 : LinearF32Form::kTiles128;
 }
 
 hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream) {
   switch (form) {
-    case LinearF32Form::kTiles32: return launch_small<1>(p, gelu, stream);
-    case LinearF32Form::kTiles64: return launch_small<2>(p, gelu, stream);
+    case LinearF32Form::kTiles32:
+      if (four_wavefronts(p.M, p.N, p.K)) return launch_small<1, 4>(p, gelu, stream);
+      return launch_small<1, 8>(p, gelu, stream);
+    case LinearF32Form::kTiles64: return launch_small<2, 8>(p, gelu, stream);
     case LinearF32Form::kTiles128: return launch_tiled(p, gelu, stream);
   }
   return hipErrorInvalidValue;
