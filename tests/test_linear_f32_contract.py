@@ -58,6 +58,12 @@ def test_workspace_arguments():
     assert size(8192, 4096, 1024) == split_bytes(4096, 1024)
     assert size(0, 64, 64) == size(-1, 64, 64) == size(1 << 31, 64, 64) == size(64, 64, 1 << 22) == 0
 
+    # One tile more than a launch takes workgroups goes to the persistent grid,
+    # however little work a tile has (the rule alone: nothing is launched).
+    last = (2 ** 32 - 1) // 512 - 8
+    for rows in (32 * last + 1, 64 * last + 1, (1 << 31) - 1):
+        assert size(rows, 4, 32) == split_bytes(4, 32)
+
     def call(**over):
         m, n, k = 8192, 4096, 1024
         a = dict(x=1 << 30, w=2 << 30, b=None, y=3 << 30, M=m, N=n, K=k, ws=4 << 30, bytes=split_bytes(n, k))

@@ -541,8 +541,8 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_f32_small_kernel(LinearF32P
 
 template <int TB, int NW>
 hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
-  p.tiles_n = (p.N + 32 * TB - 1) / (32 * TB);
-  p.tiles_m = (p.M + 32 * TB - 1) / (32 * TB);
+  p.tiles_n = (p.N - 1) / (32 * TB) + 1;
+  p.tiles_m = (p.M - 1) / (32 * TB) + 1;
   p.tiles = p.tiles_m * p.tiles_n;
   p.per_xcd = (p.tiles + 7) / 8;
   // A band is as square as an XCD's share allows.
@@ -572,8 +572,8 @@ int fl_cu_count() {
 }
 
 hipError_t launch_tiled(LinearF32Params& p, bool gelu, hipStream_t stream) {
-  p.tiles_m = (p.M + kFlTile - 1) / kFlTile;
-  p.tiles_n = (p.N + kFlTile - 1) / kFlTile;
+  p.tiles_m = (p.M - 1) / kFlTile + 1;
+  p.tiles_n = (p.N - 1) / kFlTile + 1;
   p.tiles = p.tiles_m * p.tiles_n;
   p.per_xcd = (p.tiles + 7) / 8;
   p.group_m = std::max(1, std::min(p.tiles_m, p.per_xcd / p.tiles_n));
@@ -645,8 +645,12 @@ LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool
   const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 78.0) : 4.5 + k / 113.0 + n64 / kCus * (0.9 + k / 230.0);
   double t128 = 5.0 + k / kFlBK * (n128 > kCus ? 1.37 * r128 : 0.85 + 0.52 * n128 / kCus);
   if (!terms_ready) t128 += 3.0 + n * k / 0.6e6;
-  if (t32 <= t64 && t32 <= t128) return LinearF32Form::kTiles32;
-  return t64 <= t128 ? LinearF32Form::kTiles64 : LinearF32Form::kTiles128;
+  // The small forms have a workgroup per tile: within HIP's limit of 2^32 - 1
+  // work-items (the tiled form's grid is persistent).
+  constexpr double kMaxTiles = 4294967295.0 / 512.0 - 8.0;
+  const bool fits32 = n32 <= kMaxTiles, fits64 = n64 <= kMaxTiles;
+  if (fits32 && (t32 <= t64 || !fits64) && t32 <= t128) return LinearF32Form::kTiles32;
+  return fits64 && t64 <= t128 ? LinearF32Form::kTiles64 : LinearF32Form::kTiles128;
 }
 
 hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream) {
