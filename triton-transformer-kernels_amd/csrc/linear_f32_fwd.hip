@@ -620,16 +620,15 @@ __global__ __launch_bounds__(256) void split_weight_kernel(const float* w, u32x4
 namespace {
 
 double tile_count(double M, double N, double side) { return std::ceil(M / side) * std::ceil(N / side); }
-constexpr double kCus = 256.0;
 
 // Wavefronts of a 32 x 32 tile (see linear_f32_small_kernel).
-bool four_wavefronts(int64_t M, int64_t N, int64_t K) { return K <= 64 || tile_count(M, N, 32.0) > kCus; }
+bool four_wavefronts(int64_t M, int64_t N, int64_t K) { return K <= 64 || tile_count(M, N, 32.0) > fl_cu_count(); }
 
 }  // namespace
 
 LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready) {
   if (ldw >= int64_t{1} << 22) return LinearF32Form::kTiles128;
-  // The form with the least expected time (us) on 256 CUs, from the measured
+  // The form with the least expected time (us), from the measured (256 CUs)
   // times of the three over products from 1 x 256 x 256 to 8192 x 4096 x 1024:
   // a launch's fixed cost and the chain of k-steps in one round of tiles, which
   // runs slower the more CUs have a tile, or whole rounds (of two 32 x 32 tiles
@@ -637,13 +636,14 @@ LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool
   // are there.  E.g. 256 x 256 x 256: 4.3 us for 32 x 32 tiles, 7.0 for 64 x
   // 64, 15.2 for 128 x 128; 512 x 1024 x 1024: 14.4, 15.7, 46; 1024 x 1024 x
   // 1024: 25.6, 18.5, 45; 4096 x 1024 x 1024: 88, 65, 54.
+  const double cus = fl_cu_count();
   const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
   const double n32 = tile_count(m, n, 32.0), n64 = tile_count(m, n, 64.0), n128 = tile_count(m, n, 128.0);
-  const double r64 = std::ceil(n64 / kCus), r128 = std::min(std::ceil(n128 / kCus), 1.12 * n128 / kCus);
-  const double t32 = n32 > kCus ? 2.4 + std::ceil(n32 / (2.0 * kCus)) * (1.6 + k / 100.0)
-                                : 3.0 + k / 250.0 + n32 / kCus * (0.3 + k / 700.0);
-  const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 78.0) : 4.5 + k / 113.0 + n64 / kCus * (0.9 + k / 230.0);
-  double t128 = 5.0 + k / kFlBK * (n128 > kCus ? 1.37 * r128 : 0.85 + 0.52 * n128 / kCus);
+  const double r64 = std::ceil(n64 / cus), r128 = std::min(std::ceil(n128 / cus), 1.12 * n128 / cus);
+  const double t32 = n32 > cus ? 2.4 + std::ceil(n32 / (2.0 * cus)) * (1.6 + k / 100.0)
+                                : 3.0 + k / 250.0 + n32 / cus * (0.3 + k / 700.0);
+  const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 78.0) : 4.5 + k / 113.0 + n64 / cus * (0.9 + k / 230.0);
+  double t128 = 5.0 + k / kFlBK * (n128 > cus ? 1.37 * r128 : 0.85 + 0.52 * n128 / cus);
   if (!terms_ready) t128 += 3.0 + n * k / 0.6e6;
   // The small forms have a workgroup per tile: within HIP's limit of 2^32 - 1
   // work-items (the tiled form's grid is persistent).
