@@ -61,6 +61,34 @@ def test_against_float64(gpu_ready, seq, head_dim, causal, dtype):
         assert bool(((out.double() - exact).abs() <= bound).all()), name
 
 
+@pytest.mark.parametrize("heads", [5, 6, 7, 8, 9, 12], ids=lambda h: f"groups{90 * h}")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_tile_rule_of_long_masked_launches(gpu_ready, dtype, heads):
+    # 90 workgroups a head: up to 512 of them (256 CUs) 64-key tiles, up to 640
+    # 32-key tiles, then 64-key ones unless the rows are strided and a round is
+    # saved (8 heads: one instead of two; 9: two either way; 12: two instead of
+    # three).
+    from transformer_opt.kernels import hip_attention
+
+    seq, head_dim = 1100, 128
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    mask = _rows(seq).cuda()
+    q, k, v = (torch.randn(len(mask), seq, heads, head_dim, device="cuda", generator=g).to(dtype) for _ in range(3))
+    wide = torch.zeros(len(mask), 2 * seq, dtype=torch.bool, device="cuda")
+    wide[:, ::2] = mask
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]  # the bound of test_against_float64
+    with torch.inference_mode():
+        outs = {"span": hip_attention(q, k, v, mask), "strided": hip_attention(q, k, v, wide[:, ::2])}
+        for b in range(len(mask)):
+            qh, kt, vh = (t[b].double().permute(p).contiguous() for t, p in ((q, (1, 0, 2)), (k, (1, 2, 0)), (v, (1, 0, 2))))
+            s = torch.matmul(qh, kt).mul_(head_dim ** -0.5).masked_fill_(~mask[b], -math.inf)
+            weights = torch.softmax(s, -1) if bool(mask[b].any()) else torch.zeros_like(s)
+            exact, spread = torch.matmul(weights, vh), torch.matmul(weights, vh.abs())
+            bound = (2.5 * eps + (8 + 4 + seq / 32) * 2.0 ** -23) * spread + eps * exact.abs() + 2.0 ** -24
+            for name, out in outs.items():
+                assert bool(((out[b].permute(1, 0, 2).double() - exact).abs() <= bound).all()), (name, b)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["fp32", "bf16", "fp16"])
 @pytest.mark.parametrize("value", [math.inf, math.nan])
 @pytest.mark.parametrize("row", [3, 600, 767])

@@ -2588,10 +2588,26 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
     // Measured against the 64-key kernel (same box, alternating): causal
     // [16, 512, 16, 128] -19 %, [8, 1024, 16, 128] -9.5 %, [4, 4096, 16, 128]
     // -4 %; non-causal [16, 512, 16, 128] -4 %, [8, 1024, 16, 128] +0.7 %,
-    // [4, 2048, 16, 128] +4.6 % (key-masked +7 to +12 %), [4, 4096, 16, 128]
-    // +4.6 %, key-masked [8, 1200, 16, 128] +7 to +13 %; causal S = 16384
+    // [4, 2048, 16, 128] +4.6 %, [4, 4096, 16, 128] +4.6 %; causal S = 16384
     // +3.6 %.
-    const int bn32_max = CAUSAL ? 4096 : 1024;
+    // Key-masked and non-causal from there to 4096, where three workgroups per
+    // CU save a round of the grid: without a key span (mask rows of other than
+    // unit stride) the 64-key kernel has no whole blocks to run its pipelined
+    // body on ([4, 1200, 16, 128] 74.9 us against 63.7, [8, 1800, 16, 128] 256
+    // against 244).  With one, the mask decides - prefixes run 1-12 % faster on
+    // 64-key tiles, scattered keys 2-15 % slower ([6, 1500, 16, 128] 104.8 us
+    // against 113.1 and 147 against 138) - so 32-key tiles are taken only where
+    // the second 64-key round would be at most a quarter full: [3, 1500, 16,
+    // 128] prefix 65.1 us against 66.1, scattered 95.6 against 82.2; [4, 1200,
+    // 16, 128] 54.5 against 57.2, 77.7 against 67.5.  In grids that save no
+    // round 64-key tiles win under any mask ([2, 2048, 16, 128] 60.3 against
+    // 70.7, 78.7 against 85.2).
+    int bn32_max = CAUSAL ? 4096 : 1024;
+    if constexpr (HAS_MASK && !CAUSAL) {
+      const int64_t groups = static_cast<int64_t>(p.units) * p.BH, cus = p.cu_count;
+      const bool saves = (groups + 3 * cus - 1) / (3 * cus) < (groups + 2 * cus - 1) / (2 * cus);
+      if (saves && (p.ms != 1 || 2 * groups <= 5 * cus)) bn32_max = 4096;
+    }
     if (dtype != 0 && !p.split && p.S <= bn32_max) {
       const dim3 g(static_cast<unsigned>(p.units) * static_cast<unsigned>(p.BH)), blk(kThreads);
       if (dtype == 1) {
