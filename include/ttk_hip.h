@@ -287,9 +287,9 @@ ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split,
 
 /*
  * Workspace bytes of ttk_linear_f32_fwd_ws: ttk_linear_f32_split_bytes(N, K)
- * where the call makes W's terms first, 0 for small products (which read W
- * alone) and for sizes it does not take.  Asked for with the device of the
- * launch current.
+ * where the call makes W's terms first, the workgroups' sums where several
+ * share a tile's K (few rows, long K), 0 for other small products and for sizes
+ * it does not take.  Asked for with the device of the launch current.
  */
 int64_t ttk_linear_f32_workspace_size(int64_t M, int64_t N, int64_t K);
 

@@ -87,6 +87,44 @@ def test_terms_made_by_the_call(gpu_ready, rows, out_features, in_features, gelu
         assert bool(((again.double() + exact).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("rows,out_features,in_features", [
+    (1, 4, 1024), (16, 2048, 8192), (33, 100, 2080), (64, 1020, 4000), (31, 260, 1056), (128, 2048, 8192), (65, 516, 5152)])
+@pytest.mark.parametrize("bias", [True, False], ids=["bias", "nobias"])
+def test_workgroups_that_share_a_tile(gpu_ready, rows, out_features, in_features, bias):
+    # Few tiles of long K, in 32 x 32 and 64 x 64 tiles, k-steps that do not
+    # divide among the wavefronts; the workspace holds NaN before the call.
+    from transformer_opt import _native
+    from transformer_opt.kernels import gelu
+    from transformer_opt.kernels.linear_f32 import linear_f32
+
+    need = _native.load().ttk_linear_f32_workspace_size(rows, out_features, in_features)
+    tiles = -(-rows // 32) * -(-out_features // 32)
+    assert 0 < need != _native.load().ttk_linear_f32_split_bytes(out_features, in_features) and need % 4096 == 0
+    assert need >= 2 * 4096 * min(tiles, 256)
+    x, w, b = _inputs(rows, out_features, in_features, rows + out_features)
+    b = b if bias else None
+    x[0, 3] = float("inf")
+    if rows > 2:
+        x[1] *= 2.0 ** -118
+        x[2] = 0.0
+    with torch.inference_mode():
+        junk = torch.full((need // 4,), float("nan"), device="cuda")
+        del junk
+        y = linear_f32(x, w, None, b)
+        assert torch.equal(linear_f32(x, w, None, b).nan_to_num(1.0), y.nan_to_num(1.0))
+        z = linear_f32(x, w, None, b, gelu=True)
+        torch.testing.assert_close(z, gelu(y), rtol=1e-6, atol=1e-7, equal_nan=True)
+        exact = torch.matmul(x.double(), w.double().t().contiguous())
+        scale = torch.matmul(x.double().abs(), w.double().abs().t().contiguous())
+        if bias:
+            exact, scale = exact + b.double(), scale + b.double().abs()
+    assert torch.equal(y[0].double(), exact[0])  # infinities of either sign
+    # Row 1 is a plain fp32 sum: K roundings, and the spacing of subnormal numbers.
+    bound = (2.0 * in_features / 16 + 24) * 2.0 ** -24 * scale
+    bound[1:2] = (in_features / 2 + 2) * 2.0 ** -24 * scale[1:2] + in_features * 2.0 ** -149
+    assert bool(((y.double() - exact).abs() <= bound)[1:].all())
+
+
 @pytest.mark.parametrize("rows,out_features,in_features", [(128, 256, 64), (2048, 512, 512), (8192, 4096, 1024)])
 def test_a_single_product_is_rounded_about_once(gpu_ready, rows, out_features, in_features):
     # Rows with one nonzero value: 2^-24 of the product left out, 2^-24 in the

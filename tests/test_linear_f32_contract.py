@@ -58,6 +58,12 @@ def test_workspace_arguments():
     assert size(8192, 4096, 1024) == split_bytes(4096, 1024)
     assert size(0, 64, 64) == size(-1, 64, 64) == size(1 << 31, 64, 64) == size(64, 64, 1 << 22) == 0
 
+    # Few tiles of long K: sums of 2 to 32 workgroups a tile, 4096 bytes to 32 x 32 results.
+    for m, n, k in ((16, 2048, 8192), (1, 4, 1024), (128, 2048, 8192), (64, 1024, 4096)):
+        need = size(m, n, k)
+        tiles32, tiles64 = -(-m // 32) * -(-n // 32), -(-m // 64) * -(-n // 64)
+        assert any(need % t == 0 and 2 <= need // t <= 32 for t in (tiles32 * 4096, tiles64 * 16384))
+
     # One tile more than a launch takes workgroups goes to the persistent grid,
     # however little work a tile has (the rule alone: nothing is launched).
     last = (2 ** 32 - 1) // 512 - 8
@@ -79,6 +85,9 @@ def test_workspace_arguments():
         (dict(ws=(1 << 30) + 16), _native.TTK_EINVAL, "overlaps an input"),
         (dict(b=(4 << 30) + 32), _native.TTK_EINVAL, "overlaps an input"),
         (dict(y=(4 << 30) + 32), _native.TTK_EINVAL, "y overlaps"),
+        (dict(M=16, N=2048, K=8192, ws=None, bytes=1 << 24), _native.TTK_EINVAL, "NULL"),
+        (dict(M=16, N=2048, K=8192, bytes=size(16, 2048, 8192) - 1), _native.TTK_EINVAL, "must hold"),
+        (dict(M=16, N=2048, K=8192, ws=(3 << 30) + 16), _native.TTK_EINVAL, "y overlaps"),
         (dict(M=0), _native.TTK_OK, ""),
     ):
         assert call(**over) == status

@@ -377,6 +377,46 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
   fl_vm_wait<0>();
 }
 
+// Tile o of the small form: bands of group_m rows of tiles.
+template <int TB>
+__device__ __forceinline__ void small_tile(const LinearF32Params& p, int o, int& m0, int& n0) {
+  const int span = p.group_m * p.tiles_n;
+  const int first = o / span * p.group_m;
+  const int gs = min(p.group_m, p.tiles_m - first);
+  const int rem = o % span;
+  m0 = (first + rem % gs) * (32 * TB);
+  n0 = rem / gs * (32 * TB);
+}
+
+// Stores chunk c of the tile at (m0, n0) from its sums: bias, activation, and
+// the fp32 operands again where three terms did not do.
+template <int TB, bool GELU, bool BIAS>
+__device__ __forceinline__ void small_result(const LinearF32Params& p, int m0, int n0, int c, int lane, f32x4 v) {
+  const int i = c / (4 * TB), j = (c >> 2) % TB, g = c & 3;
+  const int m = m0 + 32 * j + (lane & 31), f = n0 + 32 * i + 8 * g + 4 * (lane >> 5);
+  bool redo = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) redo |= redo_x3(v[e]);
+  if (m >= p.M || f >= p.N) return;
+  if (__builtin_expect(redo, 0)) {
+    const float* xr = p.x + static_cast<int64_t>(m) * p.ldx;
+#pragma unroll 1
+    for (int e = 0; e < 4; ++e) {
+      const float* wr = p.w + static_cast<int64_t>(f + e) * p.ldw;
+      float a = 0.0f;
+#pragma unroll 1
+      for (int k = 0; k < p.K; ++k) a = __builtin_fmaf(wr[k], xr[k], a);
+      v[e] = a;
+    }
+  }
+  if constexpr (BIAS) v += *reinterpret_cast<const f32x4*>(p.bias + f);
+  if constexpr (GELU) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = gelu_exact(v[e]);
+  }
+  *reinterpret_cast<f32x4*>(p.y + static_cast<int64_t>(m) * p.ldy + f) = v;
+}
+
 // Small products: one workgroup of NW wavefronts per TB*32 x TB*32 tile, the
 // wavefronts splitting K; X and W are both split in registers, so that no terms
 // of W have to be made first (a launch of 2.4 us for 256 x 256 weights, 7.5 us
@@ -396,8 +436,14 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
 // and the MFMAs one after the other (2600 cycles a k-step and SIMD in 64 x 64
 // tiles, 1536 of them MFMA): the next k-step's splits between this one's MFMAs
 // gained 5 - 13 % from K = 2048 up in few tiles and lost 5 - 20 % elsewhere.
-// The library's fp32 GEMM is faster where few tiles meet a long K (64 x 1024 x
-// 4096 11 us, 64 x 1024 x 1024 6.0 against 7.7), at three times the error.
+// Few tiles of long K left most CUs idle and one CU reading up to 1 MB of W:
+// there p.splits workgroups share a tile's K, each writing its sums to the
+// workspace, and linear_f32_join_kernel adds them in order (a launch of its own,
+// 2 us in a graph: the kernel boundary makes the sums visible, and nothing has
+// to be zeroed before).  In a graph, weights cold in the caches: 16 x 2048 x
+// 8192 53 -> 22 us (the library's fp32 GEMM 23), 64 x 2048 x 8192 55 -> 28 (42),
+// 16 x 1024 x 4096 27 -> 11 (12), 64 x 1024 x 4096 29 -> 14 (12), 16 x 768 x
+// 3072 22 -> 9.3 (11), 16 x 2048 x 2048 16 -> 10.5 (12).
 template <int TB, int NW, bool GELU, bool BIAS>
 __global__ __launch_bounds__(64 * NW, 2) void linear_f32_small_kernel(LinearF32Params p) {
   constexpr int R = TB == 1 ? 4 : 2;           // ring depth
@@ -413,16 +459,16 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_f32_small_kernel(LinearF32P
   // Workgroups are dealt round-robin to the 8 XCDs: each gets a contiguous run
   // of tiles, in bands of group_m rows of tiles, and keeps their operands in
   // its L2 (up to 10 % from two rounds of tiles on).
-  const int o = static_cast<int>(blockIdx.x & 7) * p.per_xcd + static_cast<int>(blockIdx.x >> 3);
+  const int unit = static_cast<int>(blockIdx.x >> 3);
+  const int o = static_cast<int>(blockIdx.x & 7) * p.per_xcd + unit / p.splits;
   if (o >= p.tiles) return;
-  const int span = p.group_m * p.tiles_n;
-  const int first = o / span * p.group_m;
-  const int gs = min(p.group_m, p.tiles_m - first);
-  const int rem = o % span;
-  const int m0 = (first + rem % gs) * (32 * TB);
-  const int n0 = rem / gs * (32 * TB);
+  const int part = unit % p.splits;  // of the tile's K
+  int m0, n0;
+  small_tile<TB>(p, o, m0, n0);
   const int KQ = p.K / 16;
-  const int q0 = KQ * wave / NW, q1 = KQ * (wave + 1) / NW;
+  const int share = part * NW + wave, shares = p.splits * NW;
+  const int q0 = static_cast<int>(static_cast<int64_t>(KQ) * share / shares);
+  const int q1 = static_cast<int>(static_cast<int64_t>(KQ) * (share + 1) / shares);
 
   // Copy c fills rows 16 c .. + 15; rows past the last repeat it.
   const unsigned chunk = static_cast<unsigned>((lane & 3) ^ ((lane >> 4) & 3)) * 16u;
@@ -509,38 +555,39 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_f32_small_kernel(LinearF32P
   __syncthreads();
 #pragma unroll
   for (int c = wave; c < TB * TB * 4; c += NW) {
-    const int i = c / (4 * TB), j = (c >> 2) % TB, g = c & 3;
-    const int m = m0 + 32 * j + r32, f = n0 + 32 * i + 8 * g + 4 * h;
-    const f32x4* part = reinterpret_cast<const f32x4*>(smem) + c * 64 + lane;
-    f32x4 v = part[0];
+    const f32x4* sum = reinterpret_cast<const f32x4*>(smem) + c * 64 + lane;
+    f32x4 v = sum[0];
 #pragma unroll
-    for (int s = 1; s < NW; ++s) v += part[s * (kRing / 16)];
-    bool redo = false;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) redo |= redo_x3(v[e]);
-    if (m >= p.M || f >= p.N) continue;
-    if (__builtin_expect(redo, 0)) {
-      const float* xr = p.x + static_cast<int64_t>(m) * p.ldx;
-#pragma unroll 1
-      for (int e = 0; e < 4; ++e) {
-        const float* wr = p.w + static_cast<int64_t>(f + e) * p.ldw;
-        float a = 0.0f;
-#pragma unroll 1
-        for (int k = 0; k < p.K; ++k) a = __builtin_fmaf(wr[k], xr[k], a);
-        v[e] = a;
-      }
+    for (int s = 1; s < NW; ++s) v += sum[s * (kRing / 16)];
+    if (p.splits > 1) {
+      static_cast<f32x4*>(p.part)[((static_cast<int64_t>(part) * p.tiles + o) * (TB * TB * 4) + c) * 64 + lane] = v;
+    } else {
+      small_result<TB, GELU, BIAS>(p, m0, n0, c, lane, v);
     }
-    if constexpr (BIAS) v += *reinterpret_cast<const f32x4*>(p.bias + f);
-    if constexpr (GELU) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = gelu_exact(v[e]);
-    }
-    *reinterpret_cast<f32x4*>(p.y + static_cast<int64_t>(m) * p.ldy + f) = v;
   }
 }
 
+// The results of tiles whose K several workgroups share: their sums, added in
+// order.  One wavefront per chunk of 64 x 4 results.
+template <int TB, bool GELU, bool BIAS>
+__global__ __launch_bounds__(kFlThreads) void linear_f32_join_kernel(LinearF32Params p) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int o = static_cast<int>(blockIdx.x) / (TB * TB);
+  const int c = static_cast<int>(blockIdx.x) % (TB * TB) * 4 + wave;
+  int m0, n0;
+  small_tile<TB>(p, o, m0, n0);
+  const f32x4* sum = static_cast<const f32x4*>(p.part) + (static_cast<int64_t>(o) * (TB * TB * 4) + c) * 64 + lane;
+  const int64_t step = static_cast<int64_t>(p.tiles) * (TB * TB * 4) * 64;
+  f32x4 v = sum[0];
+#pragma unroll 4
+  for (int s = 1; s < p.splits; ++s) v += sum[s * step];
+  small_result<TB, GELU, BIAS>(p, m0, n0, c, lane, v);
+}
+
 template <int TB, int NW>
-hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
+hipError_t launch_small(LinearF32Params& p, const LinearF32Plan& plan, void* workspace, bool gelu,
+                        hipStream_t stream) {
   p.tiles_n = (p.N - 1) / (32 * TB) + 1;
   p.tiles_m = (p.M - 1) / (32 * TB) + 1;
   p.tiles = p.tiles_m * p.tiles_n;
@@ -548,15 +595,19 @@ hipError_t launch_small(LinearF32Params& p, bool gelu, hipStream_t stream) {
   // A band is as square as an XCD's share allows.
   p.group_m = 1;
   while (2 * p.group_m <= p.tiles_m && 4 * p.group_m * p.group_m <= p.per_xcd) p.group_m *= 2;
-  const dim3 grid(8 * static_cast<unsigned>(p.per_xcd)), blk(64 * NW);
-  if (gelu) {
-    if (p.bias) linear_f32_small_kernel<TB, NW, true, true><<<grid, blk, 0, stream>>>(p);
-    else linear_f32_small_kernel<TB, NW, true, false><<<grid, blk, 0, stream>>>(p);
-  } else {
-    if (p.bias) linear_f32_small_kernel<TB, NW, false, true><<<grid, blk, 0, stream>>>(p);
-    else linear_f32_small_kernel<TB, NW, false, false><<<grid, blk, 0, stream>>>(p);
-  }
-  return hipGetLastError();
+  p.splits = plan.splits;
+  p.part = workspace;
+  auto launch = [&](auto gelu_tag, auto bias_tag) {
+    constexpr bool G = decltype(gelu_tag)::value, B = decltype(bias_tag)::value;
+    const dim3 grid(8 * static_cast<unsigned>(p.per_xcd) * static_cast<unsigned>(p.splits));
+    linear_f32_small_kernel<TB, NW, G, B><<<grid, dim3(64 * NW), 0, stream>>>(p);
+    if (p.splits > 1) {
+      linear_f32_join_kernel<TB, G, B><<<dim3(static_cast<unsigned>(p.tiles) * TB * TB), dim3(kFlThreads), 0, stream>>>(p);
+    }
+    return hipGetLastError();
+  };
+  if (gelu) return p.bias ? launch(std::true_type{}, std::true_type{}) : launch(std::true_type{}, std::false_type{});
+  return p.bias ? launch(std::false_type{}, std::true_type{}) : launch(std::false_type{}, std::false_type{});
 }
 
 int fl_cu_count() {
@@ -626,8 +677,9 @@ bool four_wavefronts(int64_t M, int64_t N, int64_t K) { return K <= 64 || tile_c
 
 }  // namespace
 
-LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready) {
-  if (ldw >= int64_t{1} << 22) return LinearF32Form::kTiles128;
+LinearF32Plan plan_linear_f32(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready) {
+  const LinearF32Plan tiled = {LinearF32Form::kTiles128, 1, terms_ready ? 0 : (N + 31) / 32 * 32 * K * 6};
+  if (ldw >= int64_t{1} << 22) return tiled;
   // The form with the least expected time (us), from the measured (256 CUs)
   // times of the three over products from 1 x 256 x 256 to 8192 x 4096 x 1024:
   // a launch's fixed cost and the chain of k-steps in one round of tiles, which
@@ -636,30 +688,52 @@ LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool
   // are there.  E.g. 256 x 256 x 256: 4.3 us for 32 x 32 tiles, 7.0 for 64 x
   // 64, 15.2 for 128 x 128; 512 x 1024 x 1024: 14.4, 15.7, 46; 1024 x 1024 x
   // 1024: 25.6, 18.5, 45; 4096 x 1024 x 1024: 88, 65, 54.
-  const double cus = fl_cu_count();
+  const int64_t cu_count = fl_cu_count();
+  const double cus = static_cast<double>(cu_count);
   const double m = static_cast<double>(M), n = static_cast<double>(N), k = static_cast<double>(K);
   const double n32 = tile_count(m, n, 32.0), n64 = tile_count(m, n, 64.0), n128 = tile_count(m, n, 128.0);
   const double r64 = std::ceil(n64 / cus), r128 = std::min(std::ceil(n128 / cus), 1.12 * n128 / cus);
-  const double t32 = n32 > cus ? 2.4 + std::ceil(n32 / (2.0 * cus)) * (1.6 + k / 100.0)
-                                : 3.0 + k / 250.0 + n32 / cus * (0.3 + k / 700.0);
-  const double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 78.0) : 4.5 + k / 113.0 + n64 / cus * (0.9 + k / 230.0);
+  auto one32 = [&](double tiles, double depth) { return 3.0 + depth / 250.0 + tiles / cus * (0.3 + depth / 700.0); };
+  auto one64 = [&](double tiles, double depth) { return 4.5 + depth / 113.0 + tiles / cus * (0.9 + depth / 230.0); };
+  double t32 = n32 > cus ? 2.4 + std::ceil(n32 / (2.0 * cus)) * (1.6 + k / 100.0) : one32(n32, k);
+  double t64 = r64 > 1.0 ? 2.5 + r64 * (3.2 + k / 78.0) : one64(n64, k);
   double t128 = 5.0 + k / kFlBK * (n128 > cus ? 1.37 * r128 : 0.85 + 0.52 * n128 / cus);
   if (!terms_ready) t128 += 3.0 + n * k / 0.6e6;
+  int s32 = 1, s64 = 1;
+  if (!terms_ready) {
+    // Several workgroups to a tile, where tiles leave CUs idle: at least two
+    // k-steps a wavefront, a CU each on the tile's XCD, and the launch that
+    // joins their sums.  (Among 2 .. 32 workgroups to a tile and both tile
+    // sizes, the choice came within 5 % of the best one over 16 .. 512 rows of
+    // the projections of d = 256 .. 2048, a few at 10 %.)
+    for (int s = 2; s * 256 <= K; ++s) {
+      const double join = 2.5 + s * m * n / 0.5e6;
+      auto fits = [&](double tiles) { return s * ((static_cast<int64_t>(tiles) + 7) / 8) <= cu_count / 8; };
+      if (!fits(n64)) break;
+      if (const double t = one64(s * n64, k / s) + join; t < t64) t64 = t, s64 = s;
+      if (!fits(n32)) continue;
+      if (const double t = one32(s * n32, k / s) + join; t < t32) t32 = t, s32 = s;
+    }
+  }
   // The small forms have a workgroup per tile: within HIP's limit of 2^32 - 1
   // work-items (the tiled form's grid is persistent).
   constexpr double kMaxTiles = 4294967295.0 / 512.0 - 8.0;
   const bool fits32 = n32 <= kMaxTiles, fits64 = n64 <= kMaxTiles;
-  if (fits32 && (t32 <= t64 || !fits64) && t32 <= t128) return LinearF32Form::kTiles32;
-  return fits64 && t64 <= t128 ? LinearF32Form::kTiles64 : LinearF32Form::kTiles128;
+  auto small = [](LinearF32Form form, int splits, double tiles, int64_t tile_bytes) {
+    return LinearF32Plan{form, splits, splits == 1 ? 0 : splits * static_cast<int64_t>(tiles) * tile_bytes};
+  };
+  if (fits32 && (t32 <= t64 || !fits64) && t32 <= t128) return small(LinearF32Form::kTiles32, s32, n32, 4096);
+  return fits64 && t64 <= t128 ? small(LinearF32Form::kTiles64, s64, n64, 16384) : tiled;
 }
 
-hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream) {
-  switch (form) {
+hipError_t launch_linear_f32(LinearF32Params& p, const LinearF32Plan& plan, void* workspace, bool gelu,
+                             hipStream_t stream) {
+  switch (plan.form) {
     case LinearF32Form::kTiles32:
-      if (four_wavefronts(p.M, p.N, p.K)) return launch_small<1, 4>(p, gelu, stream);
-      return launch_small<1, 8>(p, gelu, stream);
-    case LinearF32Form::kTiles64: return launch_small<2, 8>(p, gelu, stream);
-    case LinearF32Form::kTiles128: return launch_tiled(p, gelu, stream);
+      if (four_wavefronts(p.M, p.N, p.K)) return launch_small<1, 4>(p, plan, workspace, gelu, stream);
+      return launch_small<1, 8>(p, plan, workspace, gelu, stream);
+    case LinearF32Form::kTiles64: return launch_small<2, 8>(p, plan, workspace, gelu, stream);
+    case LinearF32Form::kTiles128: p.wp = workspace; return launch_tiled(p, gelu, stream);
   }
   return hipErrorInvalidValue;
 }

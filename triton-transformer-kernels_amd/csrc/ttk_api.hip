@@ -454,9 +454,8 @@ extern "C" int64_t ttk_linear_f32_split_bytes(int64_t N, int64_t K) {
 }
 
 extern "C" int64_t ttk_linear_f32_workspace_size(int64_t M, int64_t N, int64_t K) {
-  const int64_t bytes = ttk_linear_f32_split_bytes(N, K);
-  if (M <= 0 || M >= (int64_t{1} << 31) || bytes == 0) return 0;
-  return ttk::linear_f32_form(M, N, K, K, false) == ttk::LinearF32Form::kTiles128 ? bytes : 0;
+  if (M <= 0 || M >= (int64_t{1} << 31) || ttk_linear_f32_split_bytes(N, K) == 0) return 0;
+  return ttk::plan_linear_f32(M, N, K, K, false).bytes;
 }
 
 namespace {
@@ -478,15 +477,10 @@ ttk_status check_linear_f32_weight(const char* what, const void* w, int64_t N, i
   return TTK_OK;
 }
 
-// The buffer of W's terms: made by the call (`writable`) or given.
-ttk_status check_linear_f32_terms(const char* what, const void* terms, const void* w, int64_t N, int64_t K,
-                                  int64_t ldw, bool writable) {
-  if (!terms) return fail(TTK_EINVAL, "%s: the buffer of W's terms must not be NULL", what);
-  if (!aligned16(terms)) return fail(TTK_EUNSUPPORTED, "%s: the buffer of W's terms must be 16-byte aligned", what);
-  const uint64_t wbytes = (static_cast<uint64_t>(N - 1) * ldw + K) * 4;
-  if (writable && overlaps(terms, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K)), w, wbytes)) {
-    return fail(TTK_EINVAL, "%s: the buffer of W's terms overlaps w", what);
-  }
+// A buffer of W's terms, or the workspace of a call.
+ttk_status check_linear_f32_buffer(const char* what, const char* name, const void* buffer) {
+  if (!buffer) return fail(TTK_EINVAL, "%s: %s must not be NULL", what, name);
+  if (!aligned16(buffer)) return fail(TTK_EUNSUPPORTED, "%s: %s must be 16-byte aligned", what, name);
   return TTK_OK;
 }
 
@@ -498,9 +492,9 @@ ttk_status split_weight(const char* what, const void* w, void* terms, int64_t N,
   return TTK_OK;
 }
 
-// Y = act(X W^T + bias).  W's terms are in `terms` (make_terms: made there by
-// the call, in the form that reads them).
-ttk_status linear_f32(const void* x, const void* w, void* terms, bool make_terms, int64_t terms_bytes,
+// Y = act(X W^T + bias).  `buffer` holds W's terms (terms_ready) or is the
+// call's workspace.
+ttk_status linear_f32(const void* x, const void* w, void* buffer, bool terms_ready, int64_t buffer_bytes,
                       const void* bias, void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                       int64_t ldy, int activation, void* stream) {
   g_error[0] = '\0';
@@ -511,8 +505,8 @@ ttk_status linear_f32(const void* x, const void* w, void* terms, bool make_terms
   if (M == 0) return TTK_OK;
   ttk_status st = check_linear_f32_weight("fp32 linear", w, N, K, ldw);
   if (st != TTK_OK) return st;
-  if (!make_terms) {
-    st = check_linear_f32_terms("fp32 linear", terms, w, N, K, ldw, false);
+  if (terms_ready) {
+    st = check_linear_f32_buffer("fp32 linear", "the buffer of W's terms", buffer);
     if (st != TTK_OK) return st;
   }
   if (!x || !y) return fail(TTK_EINVAL, "fp32 linear: x and y must not be NULL");
@@ -524,43 +518,43 @@ ttk_status linear_f32(const void* x, const void* w, void* terms, bool make_terms
     return fail(TTK_EUNSUPPORTED, "fp32 linear: x, bias and y must be 16-byte aligned");
   }
   if (ldx % 4 != 0 || ldy % 4 != 0 || ldx < K || ldy < N || ldx >= (int64_t{1} << 22) ||
-      ldy >= (int64_t{1} << 22) || (make_terms && ldw >= (int64_t{1} << 22))) {
+      ldy >= (int64_t{1} << 22) || (!terms_ready && ldw >= (int64_t{1} << 22))) {
     return fail(TTK_EUNSUPPORTED,
                 "fp32 linear: ldx and ldy must be multiples of 4 below 2^22 with ldx >= K and ldy >= N "
                 "(ldx=%lld ldy=%lld)",
                 (long long)ldx, (long long)ldy);
   }
-  const ttk::LinearF32Form form = ttk::linear_f32_form(M, N, K, ldw, !make_terms);
-  const bool reads_terms = form == ttk::LinearF32Form::kTiles128;
-  const uint64_t tbytes = static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K));
+  const ttk::LinearF32Plan plan = ttk::plan_linear_f32(M, N, K, ldw, terms_ready);
+  const bool reads_terms = plan.form == ttk::LinearF32Form::kTiles128;
+  const uint64_t bbytes = static_cast<uint64_t>(terms_ready ? ttk_linear_f32_split_bytes(N, K) : plan.bytes);
   const uint64_t xbytes = (static_cast<uint64_t>(M - 1) * ldx + K) * 4;
   const uint64_t wbytes = (static_cast<uint64_t>(N - 1) * ldw + K) * 4;
   const uint64_t ybytes = (static_cast<uint64_t>(M - 1) * ldy + N) * 4;
-  if (make_terms && reads_terms) {
-    if (terms_bytes < static_cast<int64_t>(tbytes)) {
-      return fail(TTK_EINVAL, "fp32 linear: the workspace must hold %lld bytes (got %lld)", (long long)tbytes,
-                  (long long)terms_bytes);
+  if (!terms_ready && bbytes > 0) {
+    if (buffer_bytes < static_cast<int64_t>(bbytes)) {
+      return fail(TTK_EINVAL, "fp32 linear: the workspace must hold %lld bytes (got %lld)", (long long)bbytes,
+                  (long long)buffer_bytes);
     }
-    st = check_linear_f32_terms("fp32 linear", terms, w, N, K, ldw, true);
+    st = check_linear_f32_buffer("fp32 linear", "the workspace", buffer);
     if (st != TTK_OK) return st;
-    if (overlaps(terms, tbytes, x, xbytes) ||
-        (bias != nullptr && overlaps(terms, tbytes, bias, static_cast<uint64_t>(N) * 4))) {
+    if (overlaps(buffer, bbytes, w, wbytes)) return fail(TTK_EINVAL, "fp32 linear: the workspace overlaps w");
+    if (overlaps(buffer, bbytes, x, xbytes) ||
+        (bias != nullptr && overlaps(buffer, bbytes, bias, static_cast<uint64_t>(N) * 4))) {
       return fail(TTK_EINVAL, "fp32 linear: the workspace overlaps an input");
     }
   }
   if (overlaps(y, ybytes, x, xbytes) || overlaps(y, ybytes, w, wbytes) ||
-      ((reads_terms || !make_terms) && overlaps(y, ybytes, terms, tbytes)) ||
+      (bbytes > 0 && overlaps(y, ybytes, buffer, bbytes)) ||
       (bias != nullptr && overlaps(y, ybytes, bias, static_cast<uint64_t>(N) * 4))) {
     return fail(TTK_EINVAL, "fp32 linear: y overlaps an input");
   }
-  if (make_terms && reads_terms) {
-    st = split_weight("fp32 linear", w, terms, N, K, ldw, stream);
+  if (!terms_ready && reads_terms) {
+    st = split_weight("fp32 linear", w, buffer, N, K, ldw, stream);
     if (st != TTK_OK) return st;
   }
   ttk::LinearF32Params p{};
   p.x = static_cast<const float*>(x);
   p.w = static_cast<const float*>(w);
-  p.wp = reads_terms ? terms : nullptr;
   p.bias = static_cast<const float*>(bias);
   p.y = static_cast<float*>(y);
   p.ldx = ldx;
@@ -569,8 +563,8 @@ ttk_status linear_f32(const void* x, const void* w, void* terms, bool make_terms
   p.M = static_cast<int>(M);
   p.N = static_cast<int>(N);
   p.K = static_cast<int>(K);
-  const hipError_t err =
-      ttk::launch_linear_f32(p, form, activation == TTK_ACT_GELU, static_cast<hipStream_t>(stream));
+  const hipError_t err = ttk::launch_linear_f32(p, plan, buffer, activation == TTK_ACT_GELU,
+                                                static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(TTK_ELAUNCH, "fp32 linear: launch failed: %s", hipGetErrorString(err));
   return TTK_OK;
 }
@@ -581,21 +575,25 @@ extern "C" ttk_status ttk_linear_f32_split_weight(const void* w, void* w_split, 
                                                   int64_t ldw, void* stream) {
   g_error[0] = '\0';
   ttk_status st = check_linear_f32_weight("split weight", w, N, K, ldw);
-  if (st == TTK_OK) st = check_linear_f32_terms("split weight", w_split, w, N, K, ldw, true);
+  if (st == TTK_OK) st = check_linear_f32_buffer("split weight", "the buffer of W's terms", w_split);
+  if (st == TTK_OK && overlaps(w_split, static_cast<uint64_t>(ttk_linear_f32_split_bytes(N, K)), w,
+                               (static_cast<uint64_t>(N - 1) * ldw + K) * 4)) {
+    st = fail(TTK_EINVAL, "split weight: the buffer of W's terms overlaps w");
+  }
   return st == TTK_OK ? split_weight("split weight", w, w_split, N, K, ldw, stream) : st;
 }
 
 extern "C" ttk_status ttk_linear_f32_fwd(const void* x, const void* w, const void* w_split, const void* bias,
                                          void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                                          int64_t ldy, int activation, void* stream) {
-  return linear_f32(x, w, const_cast<void*>(w_split), false, 0, bias, y, M, N, K, ldx, ldw, ldy, activation, stream);
+  return linear_f32(x, w, const_cast<void*>(w_split), true, 0, bias, y, M, N, K, ldx, ldw, ldy, activation, stream);
 }
 
 extern "C" ttk_status ttk_linear_f32_fwd_ws(const void* x, const void* w, const void* bias, void* y, int64_t M,
                                             int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy,
                                             int activation, void* workspace, int64_t workspace_bytes,
                                             void* stream) {
-  return linear_f32(x, w, workspace, true, workspace_bytes, bias, y, M, N, K, ldx, ldw, ldy, activation, stream);
+  return linear_f32(x, w, workspace, false, workspace_bytes, bias, y, M, N, K, ldx, ldw, ldy, activation, stream);
 }
 
 namespace {

@@ -184,6 +184,8 @@ struct LinearF32Params {
   int tiles_m, tiles_n, tiles;
   int per_xcd;        // tiles dealt to each XCD (the last may get fewer)
   int group_m;        // token tiles per band of the tile order
+  int splits;         // workgroups that share a tile's K (1: none)
+  void* part;         // their sums, see linear_f32_small_kernel
 };
 
 // Host-side launchers (defined next to their kernels).  Return a HIP error.
@@ -213,12 +215,21 @@ hipError_t launch_linear(int dtype, int activation, LinearParams& p, hipStream_t
 // Kernel of an fp32 Linear launch (see linear_f32_fwd.hip): only the one with
 // 128 x 128 tiles reads W as terms (LinearF32Params::wp).
 enum class LinearF32Form { kTiles32, kTiles64, kTiles128 };
-// The fastest form; `terms_ready`: W's terms are there already.  Row strides of W
-// from 2^22 up take 128 x 128 tiles.
-LinearF32Form linear_f32_form(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready);
+struct LinearF32Plan {
+  LinearF32Form form;
+  int splits;  // workgroups that share a tile's K
+  // Workspace bytes: W's terms, unless they are there already, or the
+  // workgroups' sums.
+  int64_t bytes;
+};
+// The fastest plan; `terms_ready`: W's terms are there already, and there is no
+// workspace.  Row strides of W from 2^22 up take 128 x 128 tiles.
+LinearF32Plan plan_linear_f32(int64_t M, int64_t N, int64_t K, int64_t ldw, bool terms_ready);
 // fp32 Linear, optionally with the exact GELU; fills the tile fields of p and
-// sizes the grid.  K a multiple of 32, N of 4.
-hipError_t launch_linear_f32(LinearF32Params& p, LinearF32Form form, bool gelu, hipStream_t stream);
+// sizes the grid.  K a multiple of 32, N of 4.  `workspace` is p.wp of the
+// tiled form or takes plan.bytes of sums.
+hipError_t launch_linear_f32(LinearF32Params& p, const LinearF32Plan& plan, void* workspace, bool gelu,
+                             hipStream_t stream);
 // W [N, K] fp32 (row stride ldw, K a multiple of 16) as three bf16 terms in
 // MFMA fragment order: ceil(N / 32) * 32 * K * 6 bytes.
 hipError_t launch_split_weight(const float* w, void* wp, int N, int K, int64_t ldw, hipStream_t stream);
