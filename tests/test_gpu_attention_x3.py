@@ -49,6 +49,40 @@ def test_error_against_float64(gpu_ready, seq_len, head_dim, causal, masked):
     assert bool(((out.double() - exact).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("seq_len", [1, 16, 32, 33, 48, 64])
+@pytest.mark.parametrize("head_dim,batch", [(128, 87), (128, 175), (128, 261), (64, 175), (64, 515), (32, 343), (32, 515)])
+@pytest.mark.parametrize("causal", [False, True], ids=["noncausal", "causal"])
+@pytest.mark.parametrize("masked", [False, True], ids=["nomask", "masked"])
+def test_heads_that_share_a_workgroup(gpu_ready, seq_len, head_dim, batch, causal, masked):
+    # Up to 64 keys and more heads than workgroup slots (256, or 512 below head
+    # dim 128): two, three or four a workgroup, the last one with fewer.
+    # Non-finite operands of a head stay in it.
+    from transformer_opt.kernels import hip_attention
+
+    g = torch.Generator(device="cuda").manual_seed(seq_len * head_dim + batch)
+    packed = torch.randn(batch, seq_len, 3, 3, head_dim, device="cuda", generator=g)
+    q, k, v = packed.unbind(2)
+    mask = None
+    if masked:
+        mask = torch.rand(batch, seq_len, device="cuda", generator=g) < 0.7
+        mask[:, 0] = True
+        mask[3] = False
+    with torch.inference_mode():
+        clean = hip_attention(q, k, v, mask, causal=causal)
+        exact, spread = _exact(q, k, v, mask, causal, head_dim ** -0.5)
+    bound = (8 + 4 + seq_len / 32) * 2.0 ** -23 * spread + 1e-30  # as above
+    assert bool(((clean.double() - exact).abs() <= bound).all())
+    v[5, 0, 1, 3], k[9, 0, 2, 1], v[batch - 1, 0, 2, 0] = math.inf, math.nan, -math.inf
+    with torch.inference_mode():
+        out = hip_attention(q, k, v, mask, causal=causal)
+    out = out.clone()
+    assert not bool(out[5, :, 1, 3].isfinite().any()) and bool(out[9, :, 2].isnan().all())
+    assert not bool(out[batch - 1, :, 2, 0].isfinite().any())
+    for at in ((5, 1), (9, 2), (batch - 1, 2)):
+        out[at[0], :, at[1]] = clean[at[0], :, at[1]]
+    assert torch.equal(out, clean) or bool(((out.double() - exact).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("seq_len", [128, 1024])
 @pytest.mark.parametrize("head_dim", [32, 64, 128])
 def test_no_pull_towards_zero(gpu_ready, seq_len, head_dim):

@@ -2008,6 +2008,15 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 // [3, 777, 12, 128] 132 -> 82 us (67 with scan_keys).  Error against float64 at those shapes:
 // 0.65-0.8 of the fp32 MFMA kernel's.
 //
+// PACK: heads of up to 64 keys have rows for one or two wavefronts, and a
+// workgroup for each of them is a chain of load, split, store and barrier around
+// one or two tiles of work.  Up to four of them share a workgroup: their tiles
+// follow one another through the same pipeline, and each wavefront works on its
+// own head's.  [512, 16, 8, 128] non-causal 152 -> 76 us (102 on the fp32 MFMA
+// kernel), causal 162 -> 76 (155); [512, 33, 8, 128] 207 -> 161 (146), causal
+// 219 -> 154 (263); causal [512, 16, 8, 64] 52 -> 30 (52), [512, 64, 8, 64]
+// key-masked 85 -> 66 (101).
+//
 // A row with a non-finite operand in reach (or one that rounds to infinity)
 // comes out non-finite, and one of values too small for three terms below
 // 2^-80; its wavefront then computes its 32 rows again on the fp32 MFMA
@@ -2029,7 +2038,7 @@ struct X3Cfg {
 template <int D>
 constexpr int kX3Groups = D >= 128 ? 1 : 2;
 
-template <int D, bool CAUSAL, bool HAS_MASK>
+template <int D, bool CAUSAL, bool HAS_MASK, bool PACK = false>
 __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(AttnParams p) {
   using C = X3Cfg<D>;
   constexpr int BN = C::BN, G = C::G, NDB = C::NDB, CPR = C::CPR, CPT = C::CPT, KS = C::KS, KPL = C::KPL,
@@ -2045,10 +2054,18 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
   const int m = lane & 31;
   const int h = lane >> 5;
 
-  const Work w = work_item(p, CAUSAL);
+  const int S = p.S;
+  // PACK: a head takes tph wavefronts and tiles, tile t is tile t % tph of the
+  // workgroup's head t / tph, and a wavefront works on those of its own head
+  // from t_lo on.
+  const int tph = PACK ? (S > BN ? 2 : 1) : 1;
+  const int bh0 = PACK ? static_cast<int>(blockIdx.x) * p.pack : 0;
+  const int heads = PACK ? min(p.pack, p.BH - bh0) : 1;
+  const int slot = PACK ? wave / tph : 0;
+  const int t_lo = PACK ? min(slot, heads) * tph : 0;
+  const Work w = PACK ? Work{bh0 + min(slot, heads - 1), 0, 0, 1, 0, 1} : work_item(p, CAUSAL);
   const int b = w.bh / p.H;
   const int hh = w.bh - b * p.H;
-  const int S = p.S;
   const float* __restrict__ Q = static_cast<const float*>(p.q) + b * p.qb + hh * p.qh;
   const float* K = static_cast<const float*>(p.k) + b * p.kb + hh * p.kh;
   const float* V = static_cast<const float*>(p.v) + b * p.vb + hh * p.vh;
@@ -2056,6 +2073,8 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
   // Keys count from `off` (0 without a key mask), SK of them exist.
   int off = 0, SK = S;
 
+  const float* const kt = PACK ? static_cast<const float*>(p.k) : nullptr;
+  const float* const vt = PACK ? static_cast<const float*>(p.v) : nullptr;
   // Staging: chunk i of a thread is 4 values of row `srow + i * 256 / CPR`.
   constexpr int RPI = kThreads / CPR;  // rows per staging pass
   const int srow = tid / CPR;
@@ -2070,12 +2089,20 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
     koff[i] = (static_cast<unsigned>(srow + RPI * i) * static_cast<unsigned>(p.ks) + 4u * sc) * 4u;
     voff[i] = (static_cast<unsigned>(srow + RPI * i) * static_cast<unsigned>(p.vs) + 4u * sc) * 4u;
   }
-  auto tile_rsrc = [&](const float* base, int64_t rs, int t) __attribute__((always_inline)) {
+  // (PACK: `base` is the tensor's and has the strides of its batches and heads.)
+  auto tile_rsrc = [&](const float* base, int64_t rs, int64_t bs, int64_t hs, int t) __attribute__((always_inline)) {
+    if constexpr (PACK) {
+      const int th = min(t / tph, heads), bh = bh0 + th, tb = bh / p.H;
+      if (th < heads) base += tb * bs + (bh - tb * p.H) * hs;
+      t = th < heads ? t % tph : tph;
+    }
     const int rows = min(SK - t * BN, BN);
     const unsigned bytes = rows > 0 ? (static_cast<unsigned>(rows - 1) * static_cast<unsigned>(rs) + D) * 4u : 0u;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + (rows > 0 ? static_cast<int64_t>(t) * BN * rs : 0)),
                                              static_cast<short>(0), static_cast<int>(bytes), 0x00020000);
   };
+  auto k_rsrc = [&](int t) __attribute__((always_inline)) { return tile_rsrc(PACK ? kt : K, p.ks, p.kb, p.kh, t); };
+  auto v_rsrc = [&](int t) __attribute__((always_inline)) { return tile_rsrc(PACK ? vt : V, p.vs, p.vb, p.vh, t); };
   auto load4 = [](const __amdgpu_buffer_rsrc_t& r, unsigned off) __attribute__((always_inline)) -> f32x4 {
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
   };
@@ -2110,10 +2137,10 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
 
   for (int pass = 0; pass < w.npass; ++pass) {
     const int qb = pass == 0 ? w.q_first : w.q_second;
-    const int q0 = qb * kBM + wave * 32;
+    const int q0 = PACK ? (slot < heads ? (wave % tph) * 32 : 2 * BN) : qb * kBM + wave * 32;
     const int qrow = q0 + m;
     int kv_end = CAUSAL ? min(S, (qb + 1) * kBM) : S;
-    if constexpr (HAS_MASK) {
+    if constexpr (HAS_MASK && !PACK) {
       K -= static_cast<int64_t>(off) * p.ks;
       V -= static_cast<int64_t>(off) * p.vs;
       M -= static_cast<int64_t>(off) * p.ms;
@@ -2128,26 +2155,28 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       }
       SK = S - off;
     }
-    const int ntiles = (kv_end + BN - 1) / BN;
-    // Tiles with keys for this wavefront.
-    const int nlive = q0 >= S ? 0 : (CAUSAL ? min(ntiles, (max(-BN, q0 + 31 - off) + BN) / BN) : ntiles);
+    const int ntiles = PACK ? heads * tph : (kv_end + BN - 1) / BN;
+    // Tiles with keys for this wavefront: up to nlive, of PACK those from t_lo.
+    const int own = q0 >= S ? 0 : (CAUSAL ? q0 / BN + 1 : tph);
+    const int nlive = PACK ? t_lo + own : q0 >= S ? 0 : (CAUSAL ? min(ntiles, (max(-BN, q0 + 31 - off) + BN) / BN) : ntiles);
 
     bool rm = false;
     auto load_mask = [&](int t) __attribute__((always_inline)) {
       if constexpr (HAS_MASK) {
-        const int key = t * BN + m;
-        rm = h == 0 && key < SK && M[key * p.ms] != 0;
+        const uint8_t* mrow = PACK ? p.mask + (bh0 + t / tph) / p.H * p.mb : M;
+        const int key = (PACK ? t % tph : t) * BN + m;
+        rm = h == 0 && key < SK && mrow[key * p.ms] != 0;
       }
     };
     auto key_bits = [&](int t) __attribute__((always_inline)) -> uint64_t {
       if constexpr (HAS_MASK) return __builtin_amdgcn_ballot_w64(rm);
-      return range_bits(t * BN, SK);
+      return range_bits((PACK ? t % tph : t) * BN, SK);
     };
 
     // Prologue: K(0) into its buffer, K(1) and V(0) into registers.
     load_mask(0);
     {
-      const auto r0 = tile_rsrc(K, p.ks, 0);
+      const auto r0 = k_rsrc(0);
 #pragma unroll
       for (int i = 0; i < CPT; ++i) rk[i] = load4(r0, koff[i]);
     }
@@ -2167,7 +2196,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       split_pair(qf[g], 3, c[2], c[3]);
     }
     {
-      const auto k1 = tile_rsrc(K, p.ks, 1), v0 = tile_rsrc(V, p.vs, 0);
+      const auto k1 = k_rsrc(1), v0 = v_rsrc(0);
 #pragma unroll
       for (int i = 0; i < CPT; ++i) {
         split_pair(rk[i][0], rk[i][1], s_lo[0], s_lo[1], s_lo[2]);
@@ -2197,7 +2226,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
     St* kput = kdst + 3 * KPL;  // where K(t + 1) goes
     St* vput = vdst;            // where V(t) goes: V(t) lives in buffer t % 3
     int vb = 2;                 // buffer of V(t - 1)
-    __amdgpu_buffer_rsrc_t knext = tile_rsrc(K, p.ks, 2), vnext = tile_rsrc(V, p.vs, 1);
+    __amdgpu_buffer_rsrc_t knext = k_rsrc(2), vnext = v_rsrc(1);
     auto stage = [&](int c, int step) __attribute__((always_inline)) {
       const int i = c >> 1;
       f32x4& r = (c & 1) ? rv[i] : rk[i];
@@ -2238,7 +2267,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       kr[g & 1][1] = kread(buf, 1, g);
       k0f[g] = kread(buf, 0, g);
     };
-    k_frag(0, 0);
+    if constexpr (!PACK) k_frag(0, 0);
 
     // Iteration t: S(t) = K(t).Q^T with the staging of K(t + 1) and V(t) in its
     // shadow; the barrier that publishes them; then P(t - 1).V(t - 1) with the
@@ -2247,10 +2276,11 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
     // barrier too.
     for (int t = 0; t < ntiles; ++t) {
       const int kb = t & 1;
-      const int k0 = t * BN;
+      const int k0 = (PACK ? t % tph : t) * BN;
       const uint64_t kv = kvalid;
       if (HAS_MASK && t + 1 < ntiles) load_mask(t + 1);
-      const bool live = t < nlive;
+      const bool live = t < nlive && (!PACK || t >= t_lo);
+      if (PACK && t == t_lo) k_frag(kb, 0);
       f32x16 s[1];
       if (live) {
         // The small products of every k-step first, then the leading ones, in
@@ -2284,13 +2314,13 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
           stage(c, 1);
           stage(c, 2);
         }
-        if (t == nlive) {
+        if (t == nlive && (!PACK || nlive > t_lo)) {
           v_frag(vb, 0);
           v_frag(vb, 1);
         }
       }
-      knext = tile_rsrc(K, p.ks, t + 3);
-      vnext = tile_rsrc(V, p.vs, t + 2);
+      knext = k_rsrc(t + 3);
+      vnext = v_rsrc(t + 2);
       if (t + 1 < ntiles) kvalid = key_bits(t + 1);
       __syncthreads();
       if (live) {
@@ -2340,7 +2370,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
         l_run += ls;
 #pragma unroll
         for (int j = 0; j < 2; ++j) pk[j] = pn[j];
-      } else if (t == nlive && nlive > 0) {
+      } else if (t == nlive && nlive > t_lo) {
 #pragma unroll
         for (int n = 0; n < NPV; ++n) pv_mfma(vb, n);
       }
@@ -2348,7 +2378,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
       vb = vb == 2 ? 0 : vb + 1;
       vput = vb == 2 ? vdst : vput + 3 * VPL;
     }
-    if (nlive == ntiles) {
+    if (nlive == ntiles && (!PACK || nlive > t_lo)) {
       // V(ntiles - 1) became visible with the last iteration's barrier.
       v_frag(vb, 0);
       v_frag(vb, 1);
@@ -2398,7 +2428,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
 #pragma unroll
     for (int i = 0; i < NDB; ++i) acc[i] = f32x16{};
 #pragma unroll 1
-    for (int t = 0; t < nlive; ++t) {
+    for (int t = 0; t < (PACK ? own : nlive); ++t) {
       const int k0 = t * BN;
       const float* kp = K + static_cast<int64_t>(min(k0 + m, SK - 1)) * p.ks + h;
       const float* qp = Q + static_cast<int64_t>(min(qrow, S - 1)) * p.qs + h;
@@ -2546,6 +2576,16 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
   // One 64-key tile per head and rows for wavefronts 0-1 only: two heads per
   // workgroup (fp32 non-causal kernels, whose second K/V buffer is free).
   p.twin = (dtype == 0 && D < 32 && !CAUSAL && p.S <= 64) ? 1 : 0;
+  // fp32 heads of up to 64 keys, which have rows for one or two wavefronts of
+  // a workgroup: up to four or two of them together, once each of them has had
+  // a workgroup slot of its own.
+  p.pack = 1;
+  if constexpr (D >= 32) {
+    if (dtype == 0 && p.S <= 64) {
+      const int slots = p.cu_count * kX3Groups<D>;
+      p.pack = std::max(1, std::min(p.S > 32 ? 2 : 4, (p.BH + slots - 1) / slots));
+    }
+  }
   p.split = 0;
   if (dtype != 0 && CAUSAL && ws != nullptr) {
     const SplitPlan sp = plan_key_split(dtype, D, true, p.BH, p.S);
@@ -2649,7 +2689,12 @@ hipError_t launch_d(int dtype, AttnParams& p, void* ws, int64_t ws_bytes, hipStr
   switch (dtype) {
     case 0:
       if constexpr (D >= 32) {
-        attn_fwd_x3_kernel<D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p);
+        if (p.pack > 1) {
+          const dim3 packed(static_cast<unsigned>((p.BH + p.pack - 1) / p.pack));
+          attn_fwd_x3_kernel<D, CAUSAL, HAS_MASK, true><<<packed, blk, 0, stream>>>(p);
+        } else {
+          attn_fwd_x3_kernel<D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p);
+        }
       } else {
         attn_fwd_f32_kernel<D, CAUSAL, HAS_MASK><<<g, blk, 0, stream>>>(p);
       }

@@ -92,6 +92,7 @@ struct AttnParams {
   int units;         // workgroups per (batch, head)
   int cu_count;      // compute units of the device (wave-priority phase)
   int twin;          // fp32, S <= 64: two (batch, head) pairs per workgroup
+  int pack;          // fp32, head_dim 32 and up, S <= 64: heads per workgroup
   int fold;          // causal, one resident round: heavy/light query-tile order
   // Key-split causal grid (16-bit): query tiles heavier than the average
   // workgroup slot are split into chunks of key tiles; unit u of a (batch,
