@@ -2409,15 +2409,7 @@ __global__ __launch_bounds__(kThreads, kX3Groups<D>) void attn_fwd_x3_kernel(Att
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
       for (int r = 0; r < 16; ++r) watch.see(acc[db][r]);
-    bool redo = watch.any();
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) != 0, 0)) {
-      redo = redo_x3(lt);
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) redo |= redo_x3(acc[db][r]);
-    }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo) == 0, 1)) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(watch.any()) == 0, 1)) {
       store(lt);
       continue;
     }

@@ -79,17 +79,19 @@ constexpr float kRedoBelow = 0x1p-80f;
 __device__ __forceinline__ bool redo_x3(float v) {
   return !(v * 0.0f == 0.0f) || (v != 0.0f && __builtin_fabsf(v) < kRedoBelow);
 }
-// A first look over many results, 1.5 VALU operations each: without `any()`
-// none is to be formed again.  Zeros, which are not but count here, are told
-// apart by redo_x3.
+// The same over many results, three VALU operations each and no lane mask (33
+// compares a lane kept as masks spilled up to 190 SGPRs of the attention
+// kernels).  Twice the magnitude's bits less one orders zero above all others.
 struct RedoWatch {
-  float bad = 0.0f;         // NaN once a value was not finite
-  float least = INFINITY;   // smallest magnitude
+  float bad = 0.0f;              // NaN once a value was not finite
+  unsigned least = 0xffffffffu;  // of the magnitudes
   __device__ __forceinline__ void see(float v) {
     bad = __builtin_fmaf(v, 0.0f, bad);
-    least = __builtin_fminf(least, __builtin_fabsf(v));
+    least = min(least, (__float_as_uint(v) << 1) - 1u);
   }
-  __device__ __forceinline__ bool any() const { return !(bad == 0.0f) || least < kRedoBelow; }
+  __device__ __forceinline__ bool any() const {
+    return !(bad == 0.0f) || least < (__builtin_bit_cast(unsigned, kRedoBelow) << 1) - 1u;
+  }
 };
 
 }  // namespace ttk

@@ -299,13 +299,7 @@ __global__ __launch_bounds__(kFlThreads, 2) void linear_f32_kernel(LinearF32Para
         put(i, g, v);
         __builtin_amdgcn_sched_barrier(0);
       }
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(watch.any()) == 0, 1)) return;
-    bool redo = false;
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) redo |= redo_x3(hi[i][e] + lo[i][e]);
-    if (__builtin_amdgcn_ballot_w64(redo) != 0) {
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(watch.any()) != 0, 0)) {
       fl_vm_wait<0>();
 #pragma unroll 1
       for (int i = 0; i < TN; ++i) {
