@@ -325,7 +325,14 @@ extern "C" ttk_status ttk_residual_layernorm_fwd(const void* x, const void* u, c
   // Widths that no equal group divides: at most one workgroup per row's worth
   // of rows, whichever kernel runs.
   const bool row_limited = path == ttk::LnPath::kThreePass && !(vectors && per_lane <= 16);
-  if (path == ttk::LnPath::kThreePass && units <= 256 * (vectors ? 16 : 32)) {
+  // Up to 1024 rows (four workgroups of the three-pass kernel a CU) of 65 to 512
+  // values in vectors or 1024 single ones stay with it: a launch of 3 - 6 us is
+  // a chain of latencies, and a row has 256 lanes there.  bf16 256 x 200 3.65 us
+  // against 4.96, fp32 1024 x 1001 single elements 6.8 against 7.6; at 2048 rows
+  // the ragged kernel is within 8 % either way, at 4096 19 - 38 % faster, and at
+  // any number of wider rows (16 x 1000 vectors 5.1 against 4.3).
+  const bool few = rows <= 1024 && N > 64 && N <= (vectors ? 512 : 1024);
+  if (path == ttk::LnPath::kThreePass && !few && units <= 256 * (vectors ? 16 : 32)) {
     // About four units per lane on up to 64 lanes, then up to 16, then the
     // workgroup (up to 16 vectors or 32 elements per lane).
     int lpr = 8;
