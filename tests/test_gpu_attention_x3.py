@@ -49,13 +49,14 @@ def test_error_against_float64(gpu_ready, seq_len, head_dim, causal, masked):
     assert bool(((out.double() - exact).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("seq_len", [1, 16, 32, 33, 48, 64])
-@pytest.mark.parametrize("head_dim,batch", [(128, 87), (128, 175), (128, 261), (64, 175), (64, 515), (32, 343), (32, 515)])
+@pytest.mark.parametrize("seq_len", [1, 32, 33, 64])
+@pytest.mark.parametrize("head_dim,batch", [(128, 87), (128, 261), (64, 515), (32, 175), (32, 343)])
 @pytest.mark.parametrize("causal", [False, True], ids=["noncausal", "causal"])
 @pytest.mark.parametrize("masked", [False, True], ids=["nomask", "masked"])
 def test_heads_that_share_a_workgroup(gpu_ready, seq_len, head_dim, batch, causal, masked):
     # Up to 64 keys and more heads than workgroup slots (256, or 512 below head
-    # dim 128): two, three or four a workgroup, the last one with fewer.
+    # dim 128): one (head dim 32 up to 768 heads) to four a workgroup, the last
+    # one with fewer.
     # Non-finite operands of a head stay in it.
     from transformer_opt.kernels import hip_attention
 

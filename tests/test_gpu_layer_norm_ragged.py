@@ -46,8 +46,8 @@ def test_ragged_widths(gpu_ready, width, dtype, rows, offset):
         assert bool(((got.double() - exact).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("width", [65, 68, 100, 500, 501, 512, 516, 520, 1001, 1023, 1024])
+@pytest.mark.parametrize("width", [65, 100, 512, 520, 1001, 1024])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["fp32", "bf16"])
-@pytest.mark.parametrize("rows,offset", [(1024, 0), (1025, 0), (1024, 1), (1025, 1)])
+@pytest.mark.parametrize("rows,offset", [(1024, 0), (1025, 0), (1025, 1)])
 def test_either_side_of_the_rule_on_rows(gpu_ready, width, dtype, rows, offset):
     test_ragged_widths(gpu_ready, width, dtype, rows, offset)

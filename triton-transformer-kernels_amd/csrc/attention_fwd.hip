@@ -326,13 +326,15 @@ constexpr int kSpanLds = 4;     // words of LDS scratch
 // tile (about half as much VALU work again as the softmax).  With the span, the
 // 16-bit kernel runs its pipelined body on the whole blocks and applies masks
 // only where one has an invalid key.  Measured with prefixes uniform in [S / 2,
-// S]: fp16 [6, 1000, 16, 64] 50 -> 36 us, bf16 causal [4, 2048, 16, 64] 67 ->
-// 49 us, bf16 [4, 2048, 16, 128] 168 -> 123 us, fp32 [3, 777, 12, 128] (lengths
-// 470, 543, 404) 82 -> 66 us.  The scan costs 0.5 - 1 us of a launch: nothing
+// S] (three draws): fp16 [6, 1000, 16, 64] 43 -> 29 - 34 us, bf16 causal [4, 2048,
+// 16, 64] 60 -> 49 - 51 us, bf16 [4, 2048, 16, 128] 159 -> 123 - 131 us; fp32 [8,
+// 1024, 16, 64] 196 us without and 179 with.  At S = 16384, half of it padding,
+// every workgroup reads 8192 dropped V rows, and bf16 causal [1, 16384, 16, 128]
+// still takes 811 us where it took 1147.  The scan costs 0.5 - 1 us of a launch: nothing
 // on up to 512 keys, where it gained nothing either (bf16 [2, 300, 4, 64] 9.6
 // -> 10.1 us with it), and 0 - 7 % where invalid keys are scattered over all
-// blocks (bf16 [2, 600, 8, 64] 14.6 -> 15.6 us, fp16 [6, 1000, 16, 64] 46 -> 47
-// us, bf16 [8, 1000, 16, 64] 61 -> 59 us).
+// blocks (bf16 [2, 600, 8, 64] 14.6 -> 15.6 us, bf16 [8, 1000, 16, 64] 56.7 ->
+// 58.0 us).
 //
 // The scan is one dependent load: every wavefront reads the whole row (64 keys
 // a lane, as bytes of a bool mask with unit stride), so nothing is exchanged.
@@ -1999,14 +2001,15 @@ __global__ __launch_bounds__(kThreads, (BNK == 32 ? (D <= 64 ? 4 : 3) : kMinWave
 // (see the 16-bit kernel), so the accumulators are rescaled rarely.
 //
 // It is bound by VALU issue and the power limit together: per wavefront and
-// 32-key tile at head_dim 64, 48 MFMAs against ~330 VALU instructions (144 of
-// softmax and 88 of P's split for 16 scores a lane, 88 of staging); measured
-// at [8, 1024, 16, 64] non-causal, the matrix pipe is busy 54 % of the cycles
-// at 2.0 GHz.  Against the fp32 MFMA kernel: causal [8, 1024, 16, 64] 157 ->
-// 113 us (152 TFLOP/s), [8, 4096, 16, 64] 2181 -> 1440 us (191), [8, 1024,
-// 16, 128] 376 -> 243 us, [8, 1024, 16, 32] 94 -> 69 us; non-causal key-masked
-// [3, 777, 12, 128] 132 -> 82 us (67 with scan_keys).  Error against float64 at those shapes:
-// 0.65-0.8 of the fp32 MFMA kernel's.
+// 32-key tile at head_dim 64, 48 MFMAs against ~350 VALU instructions (144 of
+// softmax and 88 of P's split for 16 scores a lane, 88 of staging, 16 that join
+// the two sums); at [8, 1024, 16, 64] causal 7.7 other VALU instructions are
+// issued per MFMA and the matrix pipe is busy 39 % of the cycles.  Against the
+// fp32 MFMA kernel: causal [8, 1024, 16, 64] 157 -> 117 us (147 TFLOP/s), [8,
+// 4096, 16, 64] 2191 -> 1495 us (184), [8, 1024, 16, 128] 377 -> 235 us, [8, 1024,
+// 16, 32] 85 -> 67 us; non-causal key-masked [3, 777, 12, 128] 132 -> 84 us (70 -
+// 82 with scan_keys, by the lengths).  Error against float64: 0.5 - 0.8 of the
+// fp32 MFMA kernel's.
 //
 // PACK: heads of up to 64 keys have rows for one or two wavefronts, and a
 // workgroup for each of them is a chain of load, split, store and barrier around

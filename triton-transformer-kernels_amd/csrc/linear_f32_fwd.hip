@@ -28,8 +28,8 @@
 //
 // For the tiled kernel W is split by a launch of its own (launch_split_weight),
 // in MFMA fragment order: 6 bytes a weight, one contiguous 1 KB copy per
-// fragment, no work on it in the main loop.  X is split in registers: 5.5 VALU operations per value, in the shadow
-// of the MFMAs.
+// fragment, no work on it in the main loop.  X is split in registers: 5.5 VALU
+// operations per value, in the shadow of the MFMAs.
 //
 // Tiled kernel (one workgroup = 4 wavefronts, two workgroups per CU; a 128 x
 // 128 tile): a wavefront owns 32 tokens x 128 features, as C^T = W . X^T with
@@ -40,10 +40,11 @@
 // operands are read half a k-step ahead and the barrier of a stage sits where
 // its last fragments have been read.  The grid is persistent and copies the
 // next tile's first stages during the current tile's last.
-// Measured, against the library's fp32 GEMM: 8192 x 4096 x 1024 479 -> 321 us
-// (214 TFLOP/s; matrix pipe busy 70 % at the 1.7 GHz the power limit leaves),
-// 8192 x 1024 x 4096 460 -> 313 us, 32768 x 1536 x 512 367 -> 275 us, and the
-// GELU, a pass of its own of 39 us on the first, costs 6 us in the epilogue.
+// Measured, against the library's fp32 GEMM and with the launch that makes W's
+// terms: 8192 x 4096 x 1024 485 -> 329 - 338 us (the kernel alone 214 TFLOP/s at
+// best; matrix pipe busy 70 % at the 1.7 GHz the power limit leaves), 8192 x 1024 x
+// 4096 460 -> 315 us, 32768 x 1536 x 512 368 -> 270 - 277 us, and the GELU, a pass
+// of its own of 39 us on the first, costs 6 us in the epilogue.
 // 256-token tiles with one workgroup per CU ran 3-6 % slower (no second
 // workgroup to cover the epilogue), 128 x 64 and 128 x 32 tiles 15-50 %.
 #include <algorithm>
